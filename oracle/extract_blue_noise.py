@@ -1,13 +1,16 @@
-"""Extract the 64x64 blue-noise threshold matrix from the reference's
-src/internal/blue_noise.zig (Pixman's generated matrix) into a C header for
-the oracle build.  Reads /root/reference; run by oracle/Makefile only where
-the reference is present."""
+"""Extract the 64x64 blue-noise threshold matrix (Pixman's generated matrix)
+into a C header for the oracle build: from the reference's
+src/internal/blue_noise.zig, or from the library's blue_noise_64x64.inc where
+the reference's source is absent."""
 import re
 import sys
 
 src, dst = sys.argv[1], sys.argv[2]
 text = open(src).read()
-body = text[text.index("= .{") + 4: text.rindex("};")]
+if "= .{" in text:
+    body = text[text.index("= .{") + 4: text.rindex("};")]
+else:
+    body = "\n".join(ln for ln in text.splitlines() if not ln.startswith("//"))
 vals = [int(v) for v in re.findall(r"\d+", body)]
 assert len(vals) == 4096, len(vals)
 with open(dst, "w") as f:
