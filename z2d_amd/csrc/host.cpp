@@ -39,8 +39,7 @@ hipError_t z2d_launch_rowprog(const JobView &J, const uint32_t *list, uint32_t n
                               hipStream_t st);
 hipError_t z2d_launch_binning(const JobView &J, hipStream_t st);
 hipError_t z2d_launch_render(const JobView &J, uint32_t tile_base, uint32_t tile_count,
-                             uint32_t *cursor, uint32_t *cursor_fast, uint32_t n_blocks,
-                             uint32_t n_fast_blocks, hipStream_t st);
+                             hipStream_t st);
 hipError_t z2d_launch_composite_quad(const z2d::QuadJob &job, uint64_t n_quads, hipStream_t st);
 hipError_t z2d_launch_flatten(const z2d_path_node *raw, const z2d::FlatJob *jobs, uint32_t n_jobs,
                               z2d::FNode *out, z2d::FlatResult *res, uint32_t *rel,
@@ -806,6 +805,7 @@ struct z2d_gpu_batch {
   // The counters of the last render, copied to pinned memory at its end
   // (read after the stream completes: no extra synchronizing copy).
   HostBuf ctr_host;
+  bool counted = false;  // the last render counted its work
   // isolate_failures: a draw whose curve exceeds the subdivision limit is
   // dropped (renders nothing) and reported in `failed` as (insertion index,
   // status) instead of failing the whole batch (the server's requests fail
@@ -1307,11 +1307,9 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   const size_t o_ohist = L.take(b->longest_first ? (ORDER_BUCKETS + 1) * sizeof(uint32_t) : 0);
   const size_t o_sentries = L.take(max_strip_entries * sizeof(uint32_t));
   const size_t o_sslow = L.take((size_t)n_tiles * spt * sizeof(uint32_t));
+  const size_t o_slist = L.take((size_t)n_tiles * spt * sizeof(uint32_t));
   const size_t o_fast = L.take((size_t)nd * sizeof(FastDraw));
-  const size_t o_counters = L.take(16 * sizeof(uint32_t));
-  // render cursors: the general renderer's, then the fast one's (one per
-  // launch: the single launch uses slot ns, per-surface launches slot s)
-  const size_t o_cursors = L.take(2 * ((size_t)ns + 1) * sizeof(uint32_t));
+  const size_t o_counters = L.take(COUNTER_WORDS * sizeof(uint32_t));
   const size_t o_rows = L.take(max_rows * sizeof(RowRec));
   const size_t o_sedges = L.take(scratch * sizeof(z2d_edge));
   const size_t o_sx = L.take(scratch * sizeof(int32_t));
@@ -1321,9 +1319,9 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   e = b->stage.ensure(input_bytes);
   if (e != hipSuccess) return fail(ctx, e, "batch staging");
   if (!b->ctr_host.p) {
-    e = b->ctr_host.ensure(16 * sizeof(uint32_t), true);
+    e = b->ctr_host.ensure(COUNTER_WORDS * sizeof(uint32_t), true);
     if (e != hipSuccess) return fail(ctx, e, "batch counters");
-    std::memset(b->ctr_host.p, 0, 16 * sizeof(uint32_t));
+    std::memset(b->ctr_host.p, 0, COUNTER_WORDS * sizeof(uint32_t));
   }
   uint8_t *H = b->stage.p;
   uint8_t *D = b->arena.p;
@@ -1446,10 +1444,10 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   J.strip_entries = reinterpret_cast<uint32_t *>(D + o_sentries);
   J.max_strip_entries = (uint32_t)max_strip_entries;
   J.strip_slow = reinterpret_cast<uint32_t *>(D + o_sslow);
+  J.slow_list = reinterpret_cast<uint32_t *>(D + o_slist);
   J.fast = reinterpret_cast<FastDraw *>(D + o_fast);
   J.counters = reinterpret_cast<uint32_t *>(D + o_counters);
   J.count_stats = b->count_stats;
-  J.cursors = reinterpret_cast<uint32_t *>(D + o_cursors);
   J.rows = reinterpret_cast<RowRec *>(D + o_rows);
   J.max_rows = (uint32_t)max_rows;
   J.tiles = reinterpret_cast<const TileRef *>(D + o_tiles);
@@ -1463,19 +1461,18 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   return Z2D_OK;
 }
 
-// The render pipeline of a prepared batch on its stream: counters and
-// cursors cleared by fill kernels (no memset nodes, so the sequence can be
+// The render pipeline of a prepared batch on its stream: counters cleared by
+// fill kernels (no memset nodes, so the sequence can be
 // captured into a graph), edge build, row programs, binning, tile render.
 // mark_render records ev[1] between the binning and the render.
 static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_render) {
-  z2d_gpu_ctx *ctx = b->ctx;
   JobView &J = b->view;
   const uint32_t ns = J.n_surfaces;
   const hipStream_t st = bstream(b);
-  // every per-render reset: counters, render cursors, the entries' edge
-  // counts and cursors, their column ranges (empty until the edge binning
-  // widens them) and the scans' look-back words; done by the flattening's
-  // per-node kernel when there is one, else in a launch of their own
+  // every per-render reset: counters, the entries' edge counts and cursors,
+  // their column ranges (empty until the edge binning widens them) and the
+  // scans' look-back words; done by the flattening's per-node kernel when
+  // there is one, else in a launch of their own
   FillSet F{};
   auto add = [&](uint32_t *p, uint64_t n, uint32_t v) {
     if (n == 0) return;
@@ -1484,8 +1481,8 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
     F.v[F.count] = v;
     F.count++;
   };
-  add(J.counters, 16, 0u);
-  add(J.cursors, 2 * ((uint64_t)ns + 1), 0u);
+  const uint32_t ctr_words = J.count_stats ? COUNTER_WORDS : 16;
+  add(J.counters, ctr_words, 0u);
   if (J.n_bands) {
     add(J.entry_ecnt, 2ull * J.max_entries + 1, 0u);
     add(reinterpret_cast<uint32_t *>(J.entry_xlo), J.max_entries, 0x7FFFFFFFu);
@@ -1506,29 +1503,19 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
                            b->d_scratch_x, b->d_rowprog_soff, st);
   if (e == hipSuccess) e = z2d_launch_binning(J, st);
   if (e == hipSuccess && mark_render) e = hipEventRecord(b->ev[1], st);
-  // persistent workers: up to 8 four-wave workgroups of the general renderer
-  // and 16 one-wave workgroups of the fast one per CU (a launch with more
-  // strips than workers drains a shared queue)
-  const uint32_t max_blocks = (uint32_t)ctx->n_cus * 8;
-  const uint32_t max_fast = (uint32_t)ctx->n_cus * 16;
-  uint32_t *cur_fast = J.cursors + (ns + 1);
   if (mode == 0) {
-    const uint32_t items = J.n_tiles * J.strips_per_tile;
-    if (e == hipSuccess)
-      e = z2d_launch_render(J, 0, J.n_tiles, J.cursors + ns, cur_fast + ns,
-                            std::min(J.n_tiles, max_blocks), std::min(items, max_fast), st);
+    if (e == hipSuccess) e = z2d_launch_render(J, 0, J.n_tiles, st);
   } else {
     for (uint32_t s = 0; s < ns && e == hipSuccess; s++) {
       const uint32_t t0 = b->surf_tile_off[s], tn = b->surf_tile_off[s + 1] - t0;
-      e = z2d_launch_render(J, t0, tn, J.cursors + s, cur_fast + s, std::min(tn, max_blocks),
-                            std::min(tn * J.strips_per_tile, max_fast), st);
+      e = z2d_launch_render(J, t0, tn, st);
     }
   }
   // the counters (work counts, bin-overflow flag) to pinned memory, read
   // once the stream has completed
   if (e == hipSuccess)
-    e = hipMemcpyAsync(b->ctr_host.p, J.counters, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                       st);
+    e = hipMemcpyAsync(b->ctr_host.p, J.counters, ctr_words * sizeof(uint32_t),
+                       hipMemcpyDeviceToHost, st);
   return e;
 }
 
@@ -1545,6 +1532,7 @@ static int32_t batch_render(z2d_gpu_batch *b, uint32_t mode) {
   const hipStream_t st = bstream(b);
   for (int i = 0; i < 3; i++)
     if (!b->ev[i]) HIP_OK(ctx, hipEventCreate(&b->ev[i]));
+  b->counted = b->view.count_stats != 0;
   if (!b->use_graph) {
     HIP_OK(ctx, hipEventRecord(b->ev[0], st));
     HIP_OK(ctx, batch_enqueue(b, mode, true));
@@ -1576,6 +1564,24 @@ static int32_t batch_render(z2d_gpu_batch *b, uint32_t mode) {
   HIP_OK(ctx, hipEventRecord(b->ev[2], st));
   b->render_timed = false;
   return Z2D_OK;
+}
+
+// The work counts of the last counted render: the sums of the counters'
+// copies in pinned memory (zero for a render that did not count).
+struct WorkCounts {
+  uint64_t pix = 0, edges = 0, entries = 0, unpacked = 0;
+};
+static WorkCounts batch_counts(const z2d_gpu_batch *b) {
+  WorkCounts w;
+  if (!b->ctr_host.p || !b->counted) return w;
+  const uint32_t *c = reinterpret_cast<const uint32_t *>(b->ctr_host.p) + 16;
+  for (uint32_t i = 0; i < STAT_SLOTS; i++, c += STAT_WORDS) {
+    w.pix += (uint64_t)c[STAT_PIX] | ((uint64_t)c[STAT_PIX + 1] << 32);
+    w.edges += c[STAT_EDGES];
+    w.entries += c[STAT_ENTRIES];
+    w.unpacked += c[STAT_UNPACKED];
+  }
+  return w;
 }
 
 static int32_t batch_wait(z2d_gpu_batch *b) {
@@ -2243,12 +2249,12 @@ int32_t z2d_gpu_batch_counters(z2d_gpu_batch *b, uint32_t enable, uint64_t out[8
     for (int i = 0; i < 8; i++) out[i] = 0;
     if (b->prepared && b->ctr_host.p) {
       HIP_OK(b->ctx, hipStreamSynchronize(bstream(b)));
-      const uint32_t *c = reinterpret_cast<const uint32_t *>(b->ctr_host.p);
-      out[0] = (uint64_t)c[4] | ((uint64_t)c[5] << 32);
-      out[1] = c[6];
-      out[2] = c[7];
-      out[3] = c[2];
-      out[4] = c[8];
+      const WorkCounts w = batch_counts(b);
+      out[0] = w.pix;
+      out[1] = w.edges;
+      out[2] = w.entries;
+      out[3] = reinterpret_cast<const uint32_t *>(b->ctr_host.p)[2];
+      out[4] = w.unpacked;
       out[5] = b->view.max_entry_edges;
     }
   }
@@ -2985,9 +2991,8 @@ struct z2d_gpu_server {
     uint64_t pix = 0;
     bool overflow = false;
     if (sl.batch.prepared && sl.batch.ctr_host.p) {
-      const uint32_t *c = reinterpret_cast<const uint32_t *>(sl.batch.ctr_host.p);
-      pix = (uint64_t)c[4] | ((uint64_t)c[5] << 32);
-      overflow = c[2] != 0;
+      pix = batch_counts(&sl.batch).pix;
+      overflow = reinterpret_cast<const uint32_t *>(sl.batch.ctr_host.p)[2] != 0;
     }
     std::vector<SrvCopy> copies;
     copies.reserve(sl.reqs.size());

@@ -13,14 +13,12 @@ namespace z2d {
 
 // Tile shape of the renderer: TILE_W pixels x band_h rows per band entry
 // (JobView::band_h, TILE_H unless tuned; a multiple of ROWS_PER_THREAD up to
-// MAX_BAND_H); workgroups of 256 lanes (4 wave64s) hold four independent
-// strip workers.
+// MAX_BAND_H).
 constexpr int TILE_W = 64;
 constexpr int TILE_H = 16;
 constexpr int MAX_BAND_H = 32;
-constexpr int RENDER_THREADS = 256;
-// Each wave renders one strip of ROWS_PER_THREAD rows of a tile on its own
-// (no workgroup barriers): lane = column, one register per strip row.
+// A one-wave workgroup renders one strip of ROWS_PER_THREAD rows of a tile:
+// lane = column, one register per strip row.
 constexpr int ROWS_PER_THREAD = 4;
 constexpr int MAX_STRIPS_PER_TILE = MAX_BAND_H / ROWS_PER_THREAD;
 constexpr int STRIP_SUBROWS = ROWS_PER_THREAD * 4;
@@ -32,6 +30,13 @@ constexpr uint32_t PACKED_EDGE_LIMIT = 32767;
 // Length classes of the longest-first strip order (lists longer than this
 // share the first class).
 constexpr uint32_t ORDER_BUCKETS = 1024;
+// Work counters (count_stats) are kept in STAT_SLOTS copies, one cache line
+// each, a workgroup adding to the copy its index selects: adds to one
+// address are served one after another (about 12 ns each across the XCDs).
+constexpr uint32_t STAT_SLOTS = 64;
+constexpr uint32_t STAT_WORDS = 16;
+enum : uint32_t { STAT_PIX = 0, STAT_EDGES = 2, STAT_ENTRIES = 3, STAT_UNPACKED = 4 };
+constexpr uint32_t COUNTER_WORDS = 16 + STAT_SLOTS * STAT_WORDS;
 // Edge slots of one draw per k_edge_bins work item.
 constexpr uint32_t EDGE_GROUP = 64;
 
@@ -256,15 +261,15 @@ struct JobView {
   uint32_t max_strip_entries;
   // per strip: nonzero when an entry of its list is not a DRAW_FAST draw
   // with a packed edge list (the general k_render takes it, k_render_fast
-  // the others)
+  // the others), and the strips k_render takes, counters[9] of them
   uint32_t *strip_slow;
+  uint32_t *slow_list;
   FastDraw *fast;            // per draw: k_render_fast's constants
-  // [2] binning overflow flag; [4..5] pixel-draws (u64); [6] edges;
-  // [7] tile-draw entries rasterized; [8] entries on the unpacked path;
-  // [9] strips for the general renderer
+  // [2] binning overflow flag; [9] strips for the general renderer; from 16
+  // on the STAT_SLOTS copies of the work counters: pixel-draws (u64), edges,
+  // tile-draw entries rasterized, entries on the unpacked path
   uint32_t *counters;
   uint32_t count_stats;  // nonzero: accumulate pixel-draw / edge counts
-  uint32_t *cursors;     // tile work cursors, one per render launch
   RowRec *rows;
   uint32_t max_rows;
   const TileRef *tiles;

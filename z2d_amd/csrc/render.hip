@@ -16,8 +16,8 @@
 //   k_strip_pass / scan
 //                 per strip (TILE_W x ROWS_PER_THREAD pixels), the band
 //                 entries whose composite region meets it, in draw order
-//   k_render      persistent strip workers, one wave per strip at a time: the
-//                 strip stays in registers while each draw of its list is
+//   k_render      strip workers, one wave per strip: the strip stays in
+//                 registers while each draw of its list is
 //                 rasterized (exact f64 intercepts accumulated as winding
 //                 deltas in LDS, wave prefix scans for per-sample winding) and
 //                 composited in draw order; HBM sees one read and one write
@@ -421,6 +421,11 @@ __device__ void write_fast_draw(FastDraw &F, const DevDraw &D, const DevPaint &P
   }
 }
 
+// The copy of the work counters that workgroup (or draw) i adds to.
+__device__ __forceinline__ uint32_t *stat_slot(const JobView &J, uint32_t i) {
+  return J.counters + 16 + (i % STAT_SLOTS) * STAT_WORDS;
+}
+
 __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t d = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -476,7 +481,7 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
     }
   }
   D.edge_cnt = acc.n;
-  if (J.count_stats && acc.n) atomicAdd(&J.counters[6], acc.n);
+  if (J.count_stats && acc.n) atomicAdd(&stat_slot(J, d)[STAT_EDGES], acc.n);
   D.ext[0] = acc.top; D.ext[1] = acc.bottom; D.ext[2] = acc.left; D.ext[3] = acc.right;
 
   // Raster entry logic: visibility, draw window and composite region.
@@ -1472,13 +1477,17 @@ static void scan_u32(uint32_t *a, uint32_t n, uint64_t *stat, uint32_t *err, hip
 // k_strip_pass: per strip (ROWS_PER_THREAD rows of one tile), the entries of
 // its band list whose composite region meets the strip, in draw order.  One
 // wave per tile walks the band's entries; FILL=false counts per strip,
-// FILL=true writes after the scan.
+// FILL=true writes after the scan, and appends the strips that hold a
+// general-renderer entry to slow_list.  The list's length is one address and
+// adds to it are served one by one, so a workgroup of 16 tiles takes its
+// places with one add (one add per tile took 304 us for 134,000 tiles, a
+// fifth of them with such strips; this form 52 us).
 // ---------------------------------------------------------------------------
+constexpr uint32_t STRIP_PASS_TILES = 16;
+
 template <bool FILL>
-__global__ void k_strip_pass(JobView J) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (t >= J.n_tiles) return;
+__device__ void strip_pass_tile(const JobView &J, uint32_t t, uint32_t lane,
+                                uint32_t &slow_out) {
   const TileRef T = J.tiles[t];
   const uint32_t b = J.surf_band_off[T.surface] + T.ty;
   const uint32_t e0 = min(J.band_cnt[b], J.max_entries);
@@ -1523,17 +1532,31 @@ __global__ void k_strip_pass(JobView J) {
     for (int s = 0; s < MAX_STRIPS_PER_TILE; s++)
       if ((uint32_t)s < spt) J.strip_cnt[t * spt + s] = cnt[s];
   }
-  if (FILL && lane == 0) {
-    uint32_t n_slow = 0;
-#pragma unroll
-    for (int s = 0; s < MAX_STRIPS_PER_TILE; s++)
-      if ((uint32_t)s < spt) {
-        const bool sl = (slow_strips >> s) & 1u;
-        J.strip_slow[t * spt + s] = sl ? 1u : 0u;
-        n_slow += sl ? 1u : 0u;
-      }
-    if (n_slow) atomicAdd(&J.counters[9], n_slow);
+  if (FILL && lane < spt) J.strip_slow[t * spt + lane] = (slow_strips >> lane) & 1u;
+  slow_out = slow_strips;
+}
+
+template <bool FILL>
+__global__ void __launch_bounds__(64 * STRIP_PASS_TILES) k_strip_pass(JobView J) {
+  __shared__ uint32_t s_slow[STRIP_PASS_TILES], s_base;
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t t = blockIdx.x * STRIP_PASS_TILES + w;
+  uint32_t slow = 0;
+  if (t < J.n_tiles) strip_pass_tile<FILL>(J, t, lane, slow);
+  if (!FILL) return;
+  if (lane == 0) s_slow[w] = slow;
+  __syncthreads();
+  uint32_t before = 0, total = 0;
+  for (uint32_t i = 0; i < STRIP_PASS_TILES; i++) {
+    if (i == w) before = total;
+    total += (uint32_t)__popc(s_slow[i]);
   }
+  if (total == 0) return;  // uniform over the workgroup
+  if (threadIdx.x == 0) s_base = atomicAdd(&J.counters[9], total);
+  __syncthreads();
+  if (lane < J.strips_per_tile && ((slow >> lane) & 1u))
+    J.slow_list[s_base + before + (uint32_t)__popc(slow & ((1u << lane) - 1u))] =
+        t * J.strips_per_tile + lane;
 }
 
 // ---------------------------------------------------------------------------
@@ -1959,19 +1982,42 @@ __device__ __forceinline__ void coverage_msaa_rp(uint32_t (&acc)[FAST_ACC_ROWS][
   }
 }
 
-// Persistent strip workers: each wave takes (tile, strip) items from the
-// queue and renders every draw of the tile's band over its ROWS_PER_THREAD x
-// TILE_W pixels, which stay in registers from the first draw to the last.
-// ordered: take the strips in J.strip_order (a launch over all tiles).
-__global__ void __launch_bounds__(RENDER_THREADS, 3) k_render(JobView J, uint32_t tile_base,
-                                                           uint32_t tile_count,
-                                                           uint32_t *cursor, uint32_t ordered) {
-  __shared__ StripShared shw[RENDER_THREADS / 64];
+// A strip's work counts (stat_pix per lane, the others wave-uniform) added
+// to its workgroup's copy of the counters.
+__device__ __forceinline__ void strip_stats(const JobView &J, uint32_t stat_pix,
+                                            uint32_t stat_entries, uint32_t stat_unpacked,
+                                            uint32_t lane) {
+  const uint32_t pix = (uint32_t)wave_incl_scan((int32_t)stat_pix);  // < 2^32: 256 px x entries
+  if (lane != 63) return;
+  uint32_t *const c = stat_slot(J, blockIdx.x);
+  if (pix) atomicAdd(reinterpret_cast<unsigned long long *>(&c[STAT_PIX]), (unsigned long long)pix);
+  if (stat_entries) atomicAdd(&c[STAT_ENTRIES], stat_entries);
+  if (stat_unpacked) atomicAdd(&c[STAT_UNPACKED], stat_unpacked);
+}
+
+// The strip worker of the general renderer: one-wave workgroups, each of
+// which renders every draw of a strip's list over its ROWS_PER_THREAD x
+// TILE_W pixels; they stay in registers from the first draw to the last.
+// The hardware's dispatcher hands out the strips (a workgroup for each, or
+// for every fourth where there are many, see z2d_launch_render).  (Persistent waves took
+// them from a counter before; adds to one address are served one after
+// another, about 12 ns each, so the 537,000 strips of a batch of 1,024 uneven
+// surfaces took 6.5 ms in each renderer whatever was on them: 6.39 + 6.58 ms,
+// now 2.06 + 1.16; a page of text, 32,400 strips, 428 us, now 110.)
+//   STRIPS_SLOW     a launch over all tiles: item i is slow_list[i]
+//   STRIPS_ORDERED  a launch over all tiles in J.strip_order
+//   STRIPS_TILES    tiles [tile_base, tile_base + tile_count)
+// the last two pass by the strips of k_render_fast.
+enum : uint32_t { STRIPS_SLOW = 0, STRIPS_ORDERED = 1, STRIPS_TILES = 2 };
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+k_render(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t take) {
+  __shared__ StripShared sh;
   const uint32_t lane = threadIdx.x & 63;
-  StripShared &sh = shw[threadIdx.x >> 6];
   const uint32_t spt = J.strips_per_tile;
-  const uint32_t n_items = tile_count * spt;
-  if (load_uniform(&J.counters[9]) == 0) return;  // every strip is k_render_fast's
+  const uint32_t n_items =
+      take == STRIPS_SLOW ? load_uniform(&J.counters[9]) : tile_count * spt;
+  if (blockIdx.x >= n_items) return;
 
   // The accumulator starts at zero and every entry leaves it at zero.
   for (uint32_t i = lane; i < (uint32_t)(STRIP_SUBROWS * ACC_WORDS); i += 64)
@@ -1980,25 +2026,10 @@ __global__ void __launch_bounds__(RENDER_THREADS, 3) k_render(JobView J, uint32_
 
   uint32_t stat_pix = 0;  // work counters (count_stats), per lane
   uint32_t stat_entries = 0, stat_unpacked = 0;
-  for (;;) {
-    uint32_t item = 0;
-    if (lane == 0) item = atomicAdd(cursor, 1u);
-    item = __builtin_amdgcn_readfirstlane(item);
-    if (item >= n_items) {
-      if (J.count_stats) {
-        // one set of atomics per wave (per-entry atomics on one address
-        // serialize in L2)
-        unsigned long long wpix = stat_pix;
-        for (int off = 32; off > 0; off >>= 1) wpix += __shfl_xor(wpix, off, 64);
-        if (lane == 0) {
-          if (wpix) atomicAdd(reinterpret_cast<unsigned long long *>(&J.counters[4]), wpix);
-          if (stat_entries) atomicAdd(&J.counters[7], stat_entries);
-          if (stat_unpacked) atomicAdd(&J.counters[8], stat_unpacked);
-        }
-      }
-      break;
-    }
-    const uint32_t sidx = ordered ? load_uniform(&J.strip_order[item]) : tile_base * spt + item;
+  for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const uint32_t sidx = take == STRIPS_SLOW      ? load_uniform(&J.slow_list[item])
+                          : take == STRIPS_ORDERED ? load_uniform(&J.strip_order[item])
+                                                   : tile_base * spt + item;
     if (!load_uniform(&J.strip_slow[sidx])) continue;  // k_render_fast's strip
     const TileRef T = load_uniform(&J.tiles[sidx / spt]);
     const uint32_t strip = sidx % spt;
@@ -2352,6 +2383,7 @@ __global__ void __launch_bounds__(RENDER_THREADS, 3) k_render(JobView J, uint32_
       if (col_ok && py < H && pix[i] != orig[i]) store_raw(S, (int64_t)py * W + px, pix[i]);
     }
   }
+  if (J.count_stats) strip_stats(J, stat_pix, stat_entries, stat_unpacked, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2481,48 +2513,38 @@ __device__ __forceinline__ int32_t rfl(int32_t v) {
   return (int32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
-// At most 128 VGPRs (four waves per SIMD; LDS allows fourteen per CU).
+// At most 128 VGPRs (four waves per SIMD, the sixteen workgroups that the LDS
+// admits on a CU).  Strips are handed out as in k_render (take is never
+// STRIPS_SLOW here).
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-k_render_fast(JobView J, uint32_t tile_base,
-                                                     uint32_t tile_count, uint32_t *cursor,
-                                                     uint32_t ordered) {
+k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first,
+              uint32_t take) {
   __shared__ FastShared sh;
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t spt = J.strips_per_tile;
-  const uint32_t n_items = tile_count * spt;
-  for (uint32_t i = lane; i < (uint32_t)(FAST_ACC_ROWS * FAST_ACC_COLS); i += 64)
-    (&sh.acc[0][0])[i] = 0u;
-  if (lane <= (uint32_t)STRIP_SUBROWS) sh.ldiff[lane] = 0;
-  wave_lds_sync();
+  const uint32_t item = first + blockIdx.x;
+  if (item >= tile_count * spt) return;
+  const uint32_t sidx =
+      take == STRIPS_ORDERED ? load_uniform(&J.strip_order[item]) : tile_base * spt + item;
+  if (load_uniform(&J.strip_slow[sidx])) return;  // k_render's strip
 
   uint32_t stat_pix = 0, stat_entries = 0;  // work counters (count_stats)
-  for (;;) {
-    uint32_t item = 0;
-    if (lane == 0) item = atomicAdd(cursor, 1u);
-    item = __builtin_amdgcn_readfirstlane(item);
-    if (item >= n_items) {
-      if (J.count_stats) {
-        unsigned long long wpix = stat_pix;
-        for (int off = 32; off > 0; off >>= 1) wpix += __shfl_xor(wpix, off, 64);
-        if (lane == 0) {
-          if (wpix) atomicAdd(reinterpret_cast<unsigned long long *>(&J.counters[4]), wpix);
-          if (stat_entries) atomicAdd(&J.counters[7], stat_entries);
-        }
-      }
-      break;
-    }
-    const uint32_t sidx = ordered ? load_uniform(&J.strip_order[item]) : tile_base * spt + item;
-    if (load_uniform(&J.strip_slow[sidx])) continue;  // k_render's strip
+  {
     const TileRef T = load_uniform(&J.tiles[sidx / spt]);
     const uint32_t strip = sidx % spt;
     const DevSurface S = load_uniform(&J.surfaces[T.surface]);
     const int32_t W = S.w, H = S.h;
     const int32_t tx0 = (int32_t)T.tx * TILE_W;
     const int32_t ty0 = (int32_t)T.ty * (int32_t)J.band_h + (int32_t)strip * ROWS_PER_THREAD;
-    if (ty0 >= H) continue;
+    if (ty0 >= H) return;
     const uint32_t e0 = min(load_uniform(&J.strip_cnt[sidx]), J.max_strip_entries);
     const uint32_t e1 = min(load_uniform(&J.strip_cnt[sidx + 1]), J.max_strip_entries);
-    if (e0 == e1 && !S.clip) continue;
+    if (e0 == e1 && !S.clip) return;
+    // the winding deltas start at zero and every entry leaves them at zero
+    for (uint32_t i = lane; i < (uint32_t)(FAST_ACC_ROWS * FAST_ACC_COLS / 4); i += 64)
+      reinterpret_cast<uint4 *>(&sh.acc[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (lane <= (uint32_t)STRIP_SUBROWS) sh.ldiff[lane] = 0;
+    wave_lds_sync();
     const int32_t px = tx0 + (int32_t)lane;
     const bool col_ok = px < W;
     uint32_t pix[ROWS_PER_THREAD];
@@ -2748,6 +2770,7 @@ k_render_fast(JobView J, uint32_t tile_base,
       if (col_ok && py < H && ((dirty >> i) & 1u)) store_raw(S, (int64_t)py * W + px, pix[i]);
     }
   }
+  if (J.count_stats) strip_stats(J, stat_pix, stat_entries, 0u, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -3107,11 +3130,12 @@ hipError_t z2d_launch_binning(const JobView &J, hipStream_t st) {
   scan_u32(J.slot_cnt, J.n_slots, J.scan_tmp + J.scan_words, J.counters + 2, st);
   hipLaunchKernelGGL(k_band_pass<true>, grid, dim3(256), 0, st, J);
   if (J.n_tiles) {
-    dim3 tgrid((J.n_tiles + 3) / 4);
-    hipLaunchKernelGGL(k_strip_pass<false>, tgrid, dim3(256), 0, st, J);
+    const dim3 tgrid((J.n_tiles + STRIP_PASS_TILES - 1) / STRIP_PASS_TILES);
+    const dim3 tblock(64 * STRIP_PASS_TILES);
+    hipLaunchKernelGGL(k_strip_pass<false>, tgrid, tblock, 0, st, J);
     scan_u32(J.strip_cnt, J.n_tiles * J.strips_per_tile, J.scan_tmp + 2 * J.scan_words,
              J.counters + 2, st);
-    hipLaunchKernelGGL(k_strip_pass<true>, tgrid, dim3(256), 0, st, J);
+    hipLaunchKernelGGL(k_strip_pass<true>, tgrid, tblock, 0, st, J);
     if (J.strip_order) {
       const uint32_t ns = J.n_tiles * J.strips_per_tile;
       const dim3 og((ns + 255) / 256);
@@ -3166,18 +3190,23 @@ hipError_t z2d_launch_flatten(const z2d_path_node *raw, const FlatJob *jobs, uin
 }
 
 // The tile render of tiles [tile_base, tile_base + tile_count): k_render_fast
-// (one-wave workgroups) over the strips of fast draws, then k_render
-// (four-wave workgroups) over the others; each takes strips from its own
-// cursor and leaves the other's.
+// over the strips of fast draws, a workgroup per strip, then k_render over
+// the others.  How many those are is known on the device only: beyond 8,192
+// strips k_render gets a workgroup for every fourth, which costs a render
+// without any of them 3 us instead of 9 (32,400 strips) and leaves 8 waves a
+// SIMD to hand out where all are.
 hipError_t z2d_launch_render(const JobView &J, uint32_t tile_base, uint32_t tile_count,
-                             uint32_t *cursor, uint32_t *cursor_fast, uint32_t n_blocks,
-                             uint32_t n_fast_blocks, hipStream_t st) {
+                             hipStream_t st) {
   if (tile_count == 0) return hipSuccess;
-  const uint32_t ordered = (J.strip_order && tile_base == 0 && tile_count == J.n_tiles) ? 1u : 0u;
-  hipLaunchKernelGGL(k_render_fast, dim3(n_fast_blocks), dim3(64), 0, st, J, tile_base,
-                     tile_count, cursor_fast, ordered);
-  hipLaunchKernelGGL(k_render, dim3(n_blocks), dim3(RENDER_THREADS), 0, st, J, tile_base,
-                     tile_count, cursor, ordered);
+  const bool all = tile_base == 0 && tile_count == J.n_tiles;
+  const uint32_t take = all && J.strip_order ? STRIPS_ORDERED : all ? STRIPS_SLOW : STRIPS_TILES;
+  // a launch has fewer than 2^32 lanes
+  const uint32_t n = tile_count * J.strips_per_tile, most = 1u << 25;
+  for (uint32_t i = 0; i < n; i += most)
+    hipLaunchKernelGGL(k_render_fast, dim3(min(most, n - i)), dim3(64), 0, st, J, tile_base,
+                       tile_count, i, take == STRIPS_SLOW ? (uint32_t)STRIPS_TILES : take);
+  hipLaunchKernelGGL(k_render, dim3(min(most, n <= 8192 ? n : max(8192u, n / 4))), dim3(64), 0, st,
+                     J, tile_base, tile_count, take);
   return hipGetLastError();
 }
 
