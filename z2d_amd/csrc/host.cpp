@@ -40,7 +40,7 @@ hipError_t z2d_launch_rowprog(const JobView &J, const uint32_t *list, uint32_t n
 hipError_t z2d_launch_binning(const JobView &J, hipStream_t st);
 hipError_t z2d_launch_render(const JobView &J, uint32_t tile_base, uint32_t tile_count,
                              hipStream_t st);
-hipError_t z2d_launch_composite_quad(const z2d::QuadJob &job, uint64_t n_quads, hipStream_t st);
+hipError_t z2d_launch_composite_quad(const z2d::QuadJob &job, hipStream_t st);
 hipError_t z2d_launch_flatten(const z2d_path_node *raw, const z2d::FlatJob *jobs, uint32_t n_jobs,
                               z2d::FNode *out, z2d::FlatResult *res, uint32_t *rel,
                               const uint2 *curves, uint32_t n_curves, z2d::FlatTask *tasks,
@@ -1709,11 +1709,12 @@ static int32_t surface_release(z2d_gpu_ctx *ctx, SurfRef &r, bool copy_back) {
 // ---------------------------------------------------------------------------
 // compositor
 // ---------------------------------------------------------------------------
-// A source of the quad compositor: a pixel, or a surface read at the
-// destination's pixel index (same width, at least as tall, aligned for the
-// vector loads) in a 4-byte format or alpha8.
+// A source of the quad compositor: a pixel, or a surface in a 4-byte format or
+// alpha8 whose pixels all lie on it (the general compositor reads a pixel
+// past a surface's end as transparent).
 static bool quad_src(const DevCompParam &p, const CompJob &job, QuadSrc &o) {
   o.data = nullptr;
+  o.pitch = 0;
   o.fmt = 0;
   o.px = I4{0, 0, 0, 0};
   if (p.kind == Z2D_PARAM_PIXEL) {
@@ -1721,30 +1722,35 @@ static bool quad_src(const DevCompParam &p, const CompJob &job, QuadSrc &o) {
     o.px = p.px;
     return true;
   }
-  if (p.kind != Z2D_PARAM_SURFACE || p.base != 0 || p.surf.w != job.dst.w ||
-      p.surf.h < job.dst.h)
+  if (p.kind != Z2D_PARAM_SURFACE || p.base < 0 ||
+      p.base + (int64_t)(job.height - 1) * p.surf.w + job.width > (int64_t)p.surf.w * p.surf.h)
     return false;
-  const uintptr_t a = reinterpret_cast<uintptr_t>(p.surf.data);
-  if (fbits(p.surf.fmt) == 32 && (a & 15) == 0)
+  const bool word = fbits(p.surf.fmt) == 32;
+  if (word && (reinterpret_cast<uintptr_t>(p.surf.data) & 3) == 0)
     o.kind = QUAD_SURF32;
-  else if (p.surf.fmt == Z2D_FORMAT_ALPHA8 && (a & 3) == 0)
+  else if (p.surf.fmt == Z2D_FORMAT_ALPHA8)
     o.kind = QUAD_ALPHA8;
   else
     return false;
-  o.data = p.surf.data;
+  o.data = p.surf.data + p.base * (word ? 4 : 1);
+  o.pitch = (uint64_t)p.surf.w;
   o.fmt = p.surf.fmt;
   return true;
 }
 
-// The batches the quad compositor takes (on top of the streaming conditions):
-// one operator onto the destination with a surface or pixel source, or
-// {dst_in dst=src src=mask}, {op} (src and mask surfaces or pixels).
+// The batches the quad compositor takes: 4-byte formats, one operator onto
+// the destination with a surface or pixel source, or
+// {dst_in dst=src src=mask}, {op} (src and mask surfaces or pixels), over any
+// region.  A region of whole rows whose sources have the same width is one
+// row of all its pixels.
 static bool quad_job(const CompJob &job, QuadJob &q) {
-  if ((reinterpret_cast<uintptr_t>(job.dst.data) & 15) ||
-      (reinterpret_cast<uintptr_t>(job.out.data) & 15))
+  if (fbits(job.dst.fmt) != 32 || fbits(job.out.fmt) != 32 ||
+      (reinterpret_cast<uintptr_t>(job.dst.data) & 3) ||
+      (reinterpret_cast<uintptr_t>(job.out.data) & 3))
     return false;
-  q.dst = reinterpret_cast<const uint32_t *>(job.dst.data);
-  q.out = reinterpret_cast<uint32_t *>(job.out.data);
+  const size_t at = (size_t)job.y0 * (size_t)job.dst.w + (size_t)job.x0;
+  q.dst = reinterpret_cast<const uint32_t *>(job.dst.data) + at;
+  q.out = reinterpret_cast<uint32_t *>(job.out.data) + at;
   q.dst_fmt = job.dst.fmt;
   q.out_fmt = job.out.fmt;
   q.precision = job.precision;
@@ -1754,18 +1760,27 @@ static bool quad_job(const CompJob &job, QuadJob &q) {
     q.op = o.op;
     q.masked = 0;
     q.mask = q.src;
-    return true;
-  }
-  if (job.n_ops == 2) {
+  } else if (job.n_ops == 2) {
     const DevCompOp &m = job.ops[0], &o = job.ops[1];
     if (m.op != Z2D_OP_DST_IN || o.dst.kind != Z2D_PARAM_NONE || o.src.kind != Z2D_PARAM_NONE)
       return false;
     if (!quad_src(m.dst, job, q.src) || !quad_src(m.src, job, q.mask)) return false;
     q.op = o.op;
     q.masked = 1;
-    return true;
+  } else {
+    return false;
   }
-  return false;
+  const uint64_t w = (uint64_t)job.dst.w;
+  auto follows = [&](const QuadSrc &s) { return s.kind == QUAD_PIXEL || s.pitch == w; };
+  if (job.width == job.dst.w && follows(q.src) && follows(q.mask)) {
+    q.row_px = w * (uint64_t)job.height;
+    q.rows = 1;
+  } else {
+    q.row_px = (uint64_t)job.width;
+    q.rows = (uint32_t)job.height;
+  }
+  q.pitch = (uint32_t)w;
+  return true;
 }
 
 // noalloc: the variant that allocates no device or pinned memory: every
@@ -1911,15 +1926,20 @@ static int32_t composite_impl(z2d_gpu_ctx *ctx, z2d_surface_desc *dst_d, int32_t
       if (rc) break;
     }
   }
+  QuadJob qj;
+  const bool quad = rc == Z2D_OK && quad_job(job, qj);
   if (rc == Z2D_OK) {
+    hipError_t e = hipSuccess;
+    // the job on the device with its paints: one upload, before the timed
+    // launch (the quad compositor takes its job as a kernel argument)
     Layout L;
     const size_t o_job = L.take(sizeof(CompJob));
     const PaintTable::Offsets o_pt = pt.take(L);
     const size_t o_bn = L.take(sizeof(kBlueNoise));
     std::vector<uint8_t> host_stage;  // noalloc: pageable staging
-    hipError_t e = hipSuccess;
     uint8_t *H = nullptr, *D = nullptr;
-    if (noalloc) {
+    if (quad) {
+    } else if (noalloc) {
       if (L.off > kCompScratchBytes) {
         ctx->err = "composite_noalloc: the job needs " + std::to_string(L.off) +
                    " bytes of device scratch, more than its " +
@@ -1937,7 +1957,7 @@ static int32_t composite_impl(z2d_gpu_ctx *ctx, z2d_surface_desc *dst_d, int32_t
       H = ctx->comp_stage.p;
       D = ctx->comp_arena.p;
     }
-    if (rc == Z2D_OK) {
+    if (rc == Z2D_OK && !quad) {
       pt.write(H, D, o_pt);
       const DevPaint *dp = reinterpret_cast<const DevPaint *>(D + o_pt.paints);
       for (uint64_t k = 0; k < n_ops; k++) {
@@ -1951,32 +1971,28 @@ static int32_t composite_impl(z2d_gpu_ctx *ctx, z2d_surface_desc *dst_d, int32_t
       if (e == hipSuccess)
         e = z2d_launch_grad_setup(reinterpret_cast<DevGradient *>(D + o_pt.grads),
                                   (uint32_t)pt.grads.size(), ctx->stream);
-      if (e == hipSuccess) {
-        // Streaming path: whole 4-byte-format surfaces, aligned rows, every
-        // surface source covering the destination at the origin.
-        bool stream = fbits(job.dst.fmt) == 32 && fbits(job.out.fmt) == 32 && job.x0 == 0 &&
-                      job.y0 == 0 && job.width == job.dst.w && job.height == job.dst.h &&
-                      (job.dst.w % 4) == 0;
-        for (uint64_t k = 0; k < n_ops && stream; k++)
-          for (int side = 0; side < 2; side++) {
-            const DevCompParam &q = side == 0 ? job.ops[k].dst : job.ops[k].src;
-            if (q.kind == Z2D_PARAM_SURFACE && (q.base != 0 || q.surf.w != job.dst.w))
-              stream = false;
-          }
-        if (!noalloc) {
-          if (!ctx->ev[0]) e = hipEventCreate(&ctx->ev[0]);
-          if (e == hipSuccess && !ctx->ev[1]) e = hipEventCreate(&ctx->ev[1]);
-          if (e == hipSuccess) e = hipEventRecord(ctx->ev[0], ctx->stream);
+    }
+    if (rc == Z2D_OK) {
+      // Streaming path: whole 4-byte-format surfaces, aligned rows, every
+      // surface source covering the destination at the origin.
+      bool stream = fbits(job.dst.fmt) == 32 && fbits(job.out.fmt) == 32 && job.x0 == 0 &&
+                    job.y0 == 0 && job.width == job.dst.w && job.height == job.dst.h &&
+                    (job.dst.w % 4) == 0;
+      for (uint64_t k = 0; k < n_ops && stream; k++)
+        for (int side = 0; side < 2; side++) {
+          const DevCompParam &q = side == 0 ? job.ops[k].dst : job.ops[k].src;
+          if (q.kind == Z2D_PARAM_SURFACE && (q.base != 0 || q.surf.w != job.dst.w))
+            stream = false;
         }
-        QuadJob qj;
-        if (e != hipSuccess) {
-        } else if (stream && quad_job(job, qj))
-          e = z2d_launch_composite_quad(qj, (uint64_t)job.width * (uint64_t)job.height / 4,
-                                        ctx->stream);
-        else
-          e = z2d_launch_composite(reinterpret_cast<const CompJob *>(D + o_job), job, stream,
-                                   ctx->stream);
+      if (!noalloc) {
+        if (e == hipSuccess && !ctx->ev[0]) e = hipEventCreate(&ctx->ev[0]);
+        if (e == hipSuccess && !ctx->ev[1]) e = hipEventCreate(&ctx->ev[1]);
+        if (e == hipSuccess) e = hipEventRecord(ctx->ev[0], ctx->stream);
       }
+      if (e == hipSuccess)
+        e = quad ? z2d_launch_composite_quad(qj, ctx->stream)
+                 : z2d_launch_composite(reinterpret_cast<const CompJob *>(D + o_job), job, stream,
+                                        ctx->stream);
       if (e == hipSuccess && !noalloc) e = hipEventRecord(ctx->ev[1], ctx->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
       float ms = 0.0f;

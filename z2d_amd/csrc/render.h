@@ -302,21 +302,27 @@ struct CompJob {
 };
 
 // One source of the quad compositor: a 4-byte-format surface, an alpha8
-// surface or a constant pixel, read at the destination's own pixel index.
+// surface or a constant pixel.  Pixel (row, i) of the region is read at
+// data + (row * pitch + i) pixels.
 struct QuadSrc {
-  const uint8_t *data;  // surface kinds
+  const uint8_t *data;  // surface kinds: the region's first pixel
+  uint64_t pitch;       // pixels from a row to the next
   uint32_t kind;        // QUAD_PIXEL / QUAD_SURF32 / QUAD_ALPHA8
   uint32_t fmt;         // surface format (QUAD_SURF32)
   I4 px;                // QUAD_PIXEL
 };
 enum : uint32_t { QUAD_PIXEL = 0, QUAD_SURF32 = 1, QUAD_ALPHA8 = 2 };
 
-// Whole-surface SurfaceCompositor batches of one operator, or of
+// SurfaceCompositor batches of one operator, or of
 // {dst_in dst=src src=mask}, {op}: out = op(dst, src) per pixel, four pixels
-// per lane.
+// per lane.  A batch over whole surfaces of one width is one row of all
+// their pixels.
 struct QuadJob {
-  const uint32_t *dst;
+  const uint32_t *dst;  // the region's first pixel
   uint32_t *out;
+  uint64_t row_px;      // pixels of a row of the region
+  uint32_t rows;
+  uint32_t pitch;       // of dst and out
   uint32_t dst_fmt, out_fmt;
   uint32_t op;       // the operator applied to the destination
   uint32_t masked;   // nonzero: src = dst_in(src, mask) first
