@@ -73,34 +73,59 @@ Z2D_PX __forceinline__ uint32_t composite_src_over(uint32_t raw, uint32_t fmt, I
 }
 
 // The same two steps on RGBA8 words (red in the low byte), two channels at
-// a time in the 16-bit halves of a word: each product of a channel and an
-// 8-bit factor is below 2^16 (a packed 16-bit multiply), floor(x / 255) is
-// (x + (x >> 8) + 1) >> 8 for every x <= 65025, and no sum carries into the
-// other half, so every channel is the value the per-channel form computes.
+// a time in the 16-bit halves of a word, with packed 16-bit arithmetic.  For
+// x = a * b <= 255 * 255, floor(x / 255) is (y + (y >> 8)) >> 8 with
+// y = x + 1, and ceil(x / 255) the same with y = x + 255 (floor((x + 254) /
+// 255)); y + (y >> 8) stays below 2^16 in both, so each is a multiply-add, a
+// shift, an add and a shift, the last shared by what is added next.
 typedef unsigned short z_u16x2 __attribute__((ext_vector_type(2)));
-Z2D_PX __forceinline__ uint32_t mul_x2(uint32_t x, uint32_t m) {
-  const z_u16x2 a = __builtin_bit_cast(z_u16x2, x);
-  const z_u16x2 b = {(unsigned short)m, (unsigned short)m};
-  return __builtin_bit_cast(uint32_t, a * b);
+Z2D_PX __forceinline__ z_u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(z_u16x2, v); }
+Z2D_PX __forceinline__ uint32_t as_u32(z_u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+// 256 * (a * m + c - 1 divided by 255, rounded down) per half, plus a low
+// byte below 256 (a, m <= 255; c 1 or 255)
+Z2D_PX __forceinline__ z_u16x2 div255_hi(z_u16x2 a, z_u16x2 m, z_u16x2 c) {
+  const z_u16x2 y = a * m + c;
+  return y + (y >> (unsigned short)8);
 }
-Z2D_PX __forceinline__ uint32_t div255_x2(uint32_t x) {
-  return ((x + ((x >> 8) & 0x00FF00FFu) + 0x00010001u) >> 8) & 0x00FF00FFu;
+
+// A pixel in the strip worker's registers: red and blue, green and alpha, one
+// channel in the low byte of each 16-bit half.
+struct Px2 {
+  uint32_t rb, ga;
+};
+Z2D_PX __forceinline__ Px2 px2_rgba8(uint32_t raw) {
+  return Px2{raw & 0x00FF00FFu, (raw >> 8) & 0x00FF00FFu};
 }
-// mask_coverage on an RGBA8 word
+Z2D_PX __forceinline__ uint32_t px2_to_rgba8(Px2 p) { return p.rb | (p.ga << 8); }
+Z2D_PX __forceinline__ Px2 px2_unpack(uint32_t raw, uint32_t fmt) {
+  const I4 v = unpack(raw, fmt);
+  return Px2{v.r | (v.b << 16), v.g | (v.a << 16)};
+}
+Z2D_PX __forceinline__ uint32_t px2_pack(Px2 p, uint32_t fmt) {
+  return pack(I4{p.rb & 0xFFFFu, p.ga & 0xFFFFu, p.rb >> 16, p.ga >> 16}, fmt);
+}
+// src_over of the RGBA8 word s: per channel s + floor(d * (255 - sa) / 255),
+// truncated to a byte; alpha s + d - floor(s * d / 255), which is
+// s + ceil(d * (255 - s) / 255).  The sum of 256 times the quotient and 256
+// times the source holds the truncated byte in its high byte.
+Z2D_PX __forceinline__ Px2 px2_src_over(Px2 d, uint32_t s) {
+  const uint32_t na = 0x00FF00FFu - (s >> 24) * 0x00010001u;
+  const uint32_t s_rb = (s << 8) & 0xFF00FF00u, s_ga = s & 0xFF00FF00u;
+  const z_u16x2 rb = div255_hi(as_u16x2(d.rb), as_u16x2(na), as_u16x2(0x00010001u)) + as_u16x2(s_rb);
+  const z_u16x2 ga = div255_hi(as_u16x2(d.ga), as_u16x2(na), as_u16x2(0x00FF0001u)) + as_u16x2(s_ga);
+  return Px2{as_u32(rb >> (unsigned short)8), as_u32(ga >> (unsigned short)8)};
+}
+// mask_coverage on an RGBA8 word.  Full coverage (k = 16) leaves the word as
+// it is and none gives 0, whose src_over leaves the destination as it is.
 Z2D_PX __forceinline__ uint32_t mask_coverage_rgba8(uint32_t s, int k) {
-  const uint32_t a = (uint32_t)clampi(k * 16 - 1, 0, 255);
-  return div255_x2(mul_x2(s & 0x00FF00FFu, a)) | (div255_x2(mul_x2((s >> 8) & 0x00FF00FFu, a)) << 8);
+  const uint32_t a = (uint32_t)clampi(k * 16 - 1, 0, 255) * 0x00010001u;
+  const z_u16x2 rb = div255_hi(as_u16x2(s & 0x00FF00FFu), as_u16x2(a), as_u16x2(0x00010001u));
+  const z_u16x2 ga = div255_hi(as_u16x2((s >> 8) & 0x00FF00FFu), as_u16x2(a), as_u16x2(0x00010001u));
+  return ((as_u32(rb) >> 8) & 0x00FF00FFu) | (as_u32(ga) & 0xFF00FF00u);
 }
 // composite_src_over on an RGBA8 surface word d and RGBA8 source s
 Z2D_PX __forceinline__ uint32_t src_over_rgba8(uint32_t d, uint32_t s) {
-  const uint32_t sa = s >> 24, na = 255u - sa;
-  const uint32_t q_rb = div255_x2(mul_x2(d & 0x00FF00FFu, na));
-  const uint32_t q_ga = div255_x2(mul_x2((d >> 8) & 0x00FF00FFu, na));
-  const uint32_t o_rb = ((s & 0x00FF00FFu) + q_rb) & 0x00FF00FFu;
-  const uint32_t o_g = (((s >> 8) & 0xFFu) + (q_ga & 0xFFu)) & 0xFFu;
-  const uint32_t da = d >> 24;
-  const uint32_t o_a = (sa + da - imul8(sa, da)) & 0xFFu;
-  return o_rb | (o_g << 8) | (o_a << 24);
+  return px2_to_rgba8(px2_src_over(px2_rgba8(d), s));
 }
 
 }  // namespace z2d

@@ -2547,16 +2547,27 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
     wave_lds_sync();
     const int32_t px = tx0 + (int32_t)lane;
     const bool col_ok = px < W;
-    uint32_t pix[ROWS_PER_THREAD];
-    uint32_t dirty = 0;  // rows whose pixel a draw composited on or the clip changed
-    uint32_t vrows = 0;  // rows whose pixel of this lane's column is on the surface
+    // the strip's pixels, from here to the store below as channel pairs
+    Px2 pix[ROWS_PER_THREAD];
+    uint32_t dirty = 0;  // byte i nonzero: a draw composited on row i
+    const bool rgba8 = S.fmt == Z2D_FORMAT_RGBA;  // uniform: no format switch per row
+    if (rgba8) {
 #pragma unroll
-    for (int i = 0; i < ROWS_PER_THREAD; i++) {
-      const int32_t py = ty0 + i;
-      const bool on = col_ok && py < H;
-      pix[i] = on ? load_raw(S, (int64_t)py * W + px) : 0u;
-      vrows |= (on ? 1u : 0u) << i;
+      for (int i = 0; i < ROWS_PER_THREAD; i++) {
+        const int32_t py = ty0 + i;
+        pix[i] = px2_rgba8((col_ok && py < H)
+                               ? reinterpret_cast<const uint32_t *>(S.data)[(int64_t)py * W + px]
+                               : 0u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < ROWS_PER_THREAD; i++) {
+        const int32_t py = ty0 + i;
+        pix[i] = px2_unpack((col_ok && py < H) ? load_raw(S, (int64_t)py * W + px) : 0u, S.fmt);
+      }
     }
+    // packed alpha surfaces hold fewer bits than a lane between draws
+    const int a_bits = S.fmt >= Z2D_FORMAT_ALPHA4 ? fmt_bits(S.fmt) : 8;
     const int32_t ys_base = ty0 * 4, xs_base = tx0 * 4;
     constexpr int32_t COLS = TILE_W * 4, SR = ROWS_PER_THREAD * 4;
 
@@ -2581,17 +2592,21 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
         wave_lds_sync();
         if (lane < FAST_DRAW_CHUNKS) reinterpret_cast<uint4 *>(&sh.blk)[lane] = nb;
         wave_lds_sync();
+        // its region, rule and paint kind straight from the lanes holding them
+        const int32_t rx0 = __builtin_amdgcn_readlane(nb.x, 0),
+                      rx1 = __builtin_amdgcn_readlane(nb.y, 0),
+                      ry0 = __builtin_amdgcn_readlane(nb.z, 0),
+                      ry1 = __builtin_amdgcn_readlane(nb.w, 0);
+        const bool eo = __builtin_amdgcn_readlane(nb.y, 1) == Z2D_FILL_EVEN_ODD;
+        const uint32_t pf = __builtin_amdgcn_readlane(nb.z, 1);
         if (j + 1 < nc) {
           const uint32_t dn = __builtin_amdgcn_readlane(g_draw, j + 1);
           if (lane < FAST_DRAW_CHUNKS) nb = reinterpret_cast<const uint4 *>(J.fast + dn)[lane];
         }
         const FastDraw &B = sh.blk;
-        const int32_t rx0 = rfl(B.rx0), rx1 = rfl(B.rx1), ry0 = rfl(B.ry0), ry1 = rfl(B.ry1);
         // uniform: the draw's composite region misses this strip
         if (rx1 <= tx0 || rx0 >= tx0 + TILE_W) continue;
         if (ry1 <= ty0 || ry0 >= ty0 + ROWS_PER_THREAD) continue;
-        const uint32_t pf = rfl(B.paint), bflags = rfl(B.flags);
-        const bool eo = rfl(B.rule) == Z2D_FILL_EVEN_ODD;
         const uint32_t ne = __builtin_amdgcn_readlane(g_cnt, j);
         const REdge *edges = J.entry_edges + __builtin_amdgcn_readlane(g_off, j);
         if (J.count_stats) stat_entries++;
@@ -2694,80 +2709,86 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
         }
         wave_lds_sync();
 
-        // ---- composite: src_over of the masked paint
-        // covered pixels inside the composite region: rows [r_lo, r_hi) of
-        // the strip lie in [ry0, ry1) (uniform; the region meets the strip)
+        // ---- composite: src_over of the masked paint.  A draw's region lies
+        // on the surface; outside it (columns [rx0, rx1), rows [r_lo, r_hi)
+        // of the strip) the coverage is taken as 0, whose source is 0 and
+        // leaves the pixel as it is, so every row is composited without a
+        // branch.
         const int32_t r_lo = max(ry0, ty0) - ty0, r_hi = min(ry1, ty0 + ROWS_PER_THREAD) - ty0;
-        const uint32_t rmask = (1u << r_hi) - (1u << r_lo);
-        uint32_t kbits = 0;
-#pragma unroll
-        for (int i = 0; i < ROWS_PER_THREAD; i++) kbits |= (kk[i] > 0 ? 1u : 0u) << i;
-        const uint32_t need = (px >= rx0 && px < rx1) ? (vrows & rmask & kbits) : 0u;
-        if (__ballot(need != 0) == 0) continue;  // nothing covered in this strip (uniform)
-        const uint32_t praw = rfl(B.px);
-        const I4 p_px{praw & 0xFFu, (praw >> 8) & 0xFFu, (praw >> 16) & 0xFFu, praw >> 24};
-        const bool solid = pf == FAST_PAINT_SOLID;
-        if (!solid) {
-          const int32_t np = __popc(need);
-          const int32_t incl_p = wave_incl_scan(np);
-          const uint32_t tot_p = (uint32_t)__builtin_amdgcn_readlane(incl_p, 63);
-          uint32_t o = (uint32_t)(incl_p - np);
-#pragma unroll
-          for (int i = 0; i < ROWS_PER_THREAD; i++)
-            if ((need >> i) & 1u) sh.u.c.plist[o++] = (uint8_t)((i << 6) | lane);
-          wave_lds_sync();
-          if (pf == FAST_PAINT_LINEAR)
-            fast_gradient<FAST_PAINT_LINEAR>(B, sh, tot_p, lane, tx0, ty0);
-          else if (pf == FAST_PAINT_RADIAL)
-            fast_gradient<FAST_PAINT_RADIAL>(B, sh, tot_p, lane, tx0, ty0);
-          else
-            fast_gradient<FAST_PAINT_CONIC>(B, sh, tot_p, lane, tx0, ty0);
-          wave_lds_sync();
-        }
-        const bool fast_full = (bflags & DRAW_FAST_SRC) != 0;
-        const uint32_t full_raw = fast_full ? pack(p_px, S.fmt) : 0u;
-        const bool rgba8 = S.fmt == Z2D_FORMAT_RGBA;  // uniform
-        // the pixels composited on are stored (a composite that leaves a
-        // pixel as it was stores the same value)
-        stat_pix += (uint32_t)__popc(need);
-        dirty |= need;
+        const bool in_col = px >= rx0 && px < rx1;
+        uint32_t cov = 0;  // row i's coverage in byte i
 #pragma unroll
         for (int i = 0; i < ROWS_PER_THREAD; i++) {
-          if (!((need >> i) & 1u)) continue;
-          const int k = kk[i];
-          if (fast_full && k >= 16) {
-            pix[i] = full_raw;
-          } else {
-            uint32_t pv = solid ? B.srctab[k] : sh.u.c.ppaint[i][lane];
-            if (rgba8) {
-              if (!solid && k < 16) pv = mask_coverage_rgba8(pv, k);
-              pix[i] = src_over_rgba8(pix[i], pv);
-            } else {
-              I4 src{pv & 0xFFu, (pv >> 8) & 0xFFu, (pv >> 16) & 0xFFu, pv >> 24};
-              if (!solid && k < 16) src = mask_coverage(src, k);
-              pix[i] = composite_src_over(pix[i], S.fmt, src);
-            }
+          if (!(in_col && i >= r_lo && i < r_hi)) kk[i] = 0;
+          cov |= (uint32_t)kk[i] << (8 * i);
+        }
+        if (__ballot(cov != 0) == 0) continue;  // nothing covered in this strip (uniform)
+        dirty |= cov;
+        const bool solid = pf == FAST_PAINT_SOLID;
+        if (!solid || J.count_stats) {
+          uint32_t need = 0;
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++) need |= (kk[i] > 0 ? 1u : 0u) << i;
+          stat_pix += (uint32_t)__popc(need);
+          if (!solid) {
+            const int32_t np = __popc(need);
+            const int32_t incl_p = wave_incl_scan(np);
+            const uint32_t tot_p = (uint32_t)__builtin_amdgcn_readlane(incl_p, 63);
+            uint32_t o = (uint32_t)(incl_p - np);
+#pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++)
+              if ((need >> i) & 1u) sh.u.c.plist[o++] = (uint8_t)((i << 6) | lane);
+            wave_lds_sync();
+            if (pf == FAST_PAINT_LINEAR)
+              fast_gradient<FAST_PAINT_LINEAR>(B, sh, tot_p, lane, tx0, ty0);
+            else if (pf == FAST_PAINT_RADIAL)
+              fast_gradient<FAST_PAINT_RADIAL>(B, sh, tot_p, lane, tx0, ty0);
+            else
+              fast_gradient<FAST_PAINT_CONIC>(B, sh, tot_p, lane, tx0, ty0);
+            wave_lds_sync();
           }
+        }
+        if (solid) {
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++)
+            pix[i] = px2_src_over(pix[i], B.srctab[kk[i]]);
+        } else {
+          // (a pixel without coverage reads a stale sample, masked to 0)
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++)
+            pix[i] = px2_src_over(pix[i], mask_coverage_rgba8(sh.u.c.ppaint[i][lane], kk[i]));
+        }
+        if (a_bits < 8) {  // uniform
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++)
+            pix[i].ga = alpha_up8(alpha_down(pix[i].ga >> 16, a_bits), a_bits) << 16;
         }
       }
     }
 
-    if (S.clip) {
-      // Clip stage: Surface.composite(dst, mask, .dst_in) after the draws.
+    if (rgba8 && !S.clip) {
+#pragma unroll
+      for (int i = 0; i < ROWS_PER_THREAD; i++) {
+        const int32_t py = ty0 + i;
+        if (col_ok && py < H && ((dirty >> (8 * i)) & 0xFFu))
+          reinterpret_cast<uint32_t *>(S.data)[(int64_t)py * W + px] = px2_to_rgba8(pix[i]);
+      }
+    } else {
 #pragma unroll
       for (int i = 0; i < ROWS_PER_THREAD; i++) {
         const int32_t py = ty0 + i;
         if (!col_ok || py >= H) continue;
-        const I4 m{0, 0, 0, S.clip[(int64_t)py * W + px]};
-        const uint32_t before = pix[i];
-        pix[i] = pack(op_int(Z2D_OP_DST_IN, unpack(pix[i], S.fmt), m), S.fmt);
-        dirty |= (pix[i] != before ? 1u : 0u) << i;
+        uint32_t raw = px2_pack(pix[i], S.fmt);
+        bool changed = ((dirty >> (8 * i)) & 0xFFu) != 0;
+        if (S.clip) {
+          // Clip stage: Surface.composite(dst, mask, .dst_in) after the draws.
+          const I4 m{0, 0, 0, S.clip[(int64_t)py * W + px]};
+          const uint32_t before = raw;
+          raw = pack(op_int(Z2D_OP_DST_IN, unpack(raw, S.fmt), m), S.fmt);
+          changed |= raw != before;
+        }
+        if (changed) store_raw(S, (int64_t)py * W + px, raw);
       }
-    }
-#pragma unroll
-    for (int i = 0; i < ROWS_PER_THREAD; i++) {
-      const int32_t py = ty0 + i;
-      if (col_ok && py < H && ((dirty >> i) & 1u)) store_raw(S, (int64_t)py * W + px, pix[i]);
     }
   }
   if (J.count_stats) strip_stats(J, stat_pix, stat_entries, 0u, lane);
