@@ -1931,20 +1931,47 @@ __device__ __forceinline__ void coverage_msaa(uint32_t (&acc)[STRIP_SUBROWS][ACC
   }
 }
 
-// Row-paired winding deltas (the fast strip worker's layout): word [p][c]
-// holds sample column c of sample rows 2p (low half) and 2p + 1 (high half)
-// as lo + hi * 65536 in 32-bit arithmetic (the LDS atomics carry between the
-// halves).  Every winding and partial sum of a draw whose band entry has at
-// most PACKED_EDGE_LIMIT edges lies in [-32767, 32767], so the 32-bit sums
-// are exact, and U = W + 0x8000 for a sum W = lo + hi * 65536 holds hi in its
-// high half (mod 2^16) and lo + 0x8000 in its low half with no borrow:
-// lo is odd iff bit 0 of U is set, hi iff bit 16; U ^ 0x8000 holds lo and hi
-// as 16-bit halves, each zero iff that winding is.
-constexpr int FAST_ACC_ROWS = STRIP_SUBROWS / 2, FAST_ACC_COLS = TILE_W * 4;
+// Inclusive exclusive-or scan over the lanes of a wave (the steps of
+// wave_incl_scan with an xor).  Every lane of the wave must be active.
+__device__ __forceinline__ uint32_t wave_xor_scan(uint32_t x) {
+  asm("s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+      "s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_xor_b32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
+      : "+v"(x));
+  return x;
+}
 
-// coverage_msaa over the row-paired deltas: per pair of sample rows one
-// 16-byte read of the lane's four columns, one wave scan, and per column an
-// add and a packed test of both rows, counted by popcount.
+// The fast strip worker's crossings, FAST_ACC_ROWS words per sample column of
+// the strip.  A sample is inside by the parity of the crossings at columns up
+// to its own (even-odd) or by their winding (non-zero), so what a column has
+// to hold depends on the rule:
+//   WIND_EO    one bit per sample row (16 of them) in row 0, crossings
+//              flipping their bit: exact for any number of edges
+//   WIND_NZ    four sample rows (a pixel row) per word, row b as w_b * 256^b
+//              summed in 32-bit arithmetic.  The sums are taken modulo 2^32,
+//              where they stay exact whatever carries between the bytes, so
+//              a word decodes if the four windings at its column lie in
+//              [-127, 127]: adding 0x80808080 then leaves each byte
+//              w_b + 128.
+//   WIND_NZ16  two sample rows per word as lo + hi * 65536, windings in
+//              [-32767, 32767]: half a strip (8 sample rows) at a time, for
+//              the entries whose windings may not fit a byte
+// Words of the earlier layout, two rows to a word for both rules, took 8 reads
+// and wave scans per entry; these take 1 (even-odd) and 4, and the block's
+// LDS goes from 10.0 KB to 5.9 KB.
+constexpr int FAST_ACC_ROWS = ROWS_PER_THREAD, FAST_ACC_COLS = TILE_W * 4;
+enum WindMode { WIND_EO = 0, WIND_NZ = 1, WIND_NZ16 = 2 };
+typedef uint32_t FastAcc[FAST_ACC_ROWS][FAST_ACC_COLS];
+
 // 1 in each 16-bit half of v that is nonzero, 0 in each that is zero (a
 // packed unsigned min with 1; written out because the compiler otherwise
 // expands the packed min into per-half compares).
@@ -1954,11 +1981,50 @@ __device__ __forceinline__ uint32_t pk_nonzero_u16(uint32_t v) {
   return r;
 }
 
-template <bool EO>
-__device__ __forceinline__ void coverage_msaa_rp(uint32_t (&acc)[FAST_ACC_ROWS][FAST_ACC_COLS],
-                                                 uint32_t lane, int *kk) {
+// Covered samples per pixel of the lane's column (kk, a strip's rows; rows
+// row0 and row0 + 1 for WIND_NZ16), by prefix sums of the crossings up to
+// each sample column (lane-local over the pixel's 4 columns, a wave scan
+// across lanes).  Reads and clears the words.  left (WIND_EO): the sample
+// rows with an odd number of crossings left of the strip.
+__device__ __forceinline__ void coverage_eo(FastAcc &acc, uint32_t lane, uint32_t left, int *kk) {
+  uint4 *slot = reinterpret_cast<uint4 *>(&acc[0][lane * 4]);
+  const uint4 p = *slot;
+  *slot = make_uint4(0u, 0u, 0u, 0u);
+  const uint32_t tot = p.x ^ p.y ^ p.z ^ p.w;
+  const uint32_t u0 = wave_xor_scan(tot) ^ tot ^ left ^ p.x;
+  const uint32_t u1 = u0 ^ p.y, u2 = u1 ^ p.z, u3 = u2 ^ p.w;
+  // two columns to a word: the 4 sample rows of pixel row i are bits 4i.. of
+  // each half
+  const uint32_t v0 = u0 | (u1 << 16), v1 = u2 | (u3 << 16);
 #pragma unroll
   for (int i = 0; i < ROWS_PER_THREAD; i++) {
+    const uint32_t m = 0x000F000Fu << (4 * i);
+    kk[i] = __popc(v0 & m) + __popc(v1 & m);
+  }
+}
+__device__ __forceinline__ void coverage_nz(FastAcc &acc, uint32_t lane, int *kk) {
+#pragma unroll
+  for (int i = 0; i < ROWS_PER_THREAD; i++) {
+    uint4 *slot = reinterpret_cast<uint4 *>(&acc[i][lane * 4]);
+    const uint4 p = *slot;
+    *slot = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t tot = p.x + p.y + p.z + p.w;
+    uint32_t u = (uint32_t)wave_incl_scan((int32_t)tot) - tot + 0x80808080u;
+    const uint32_t col[4] = {p.x, p.y, p.z, p.w};
+    uint32_t k = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      u += col[j];
+      // a byte's mean with 255, rounded down, is below 128 for 0 alone
+      const uint32_t nz = __builtin_amdgcn_lerp(u ^ 0x80808080u, 0xFFFFFFFFu, 0u);
+      k += (uint32_t)__popc(nz & 0x80808080u);
+    }
+    kk[i] = (int)k;
+  }
+}
+__device__ __forceinline__ void coverage_nz16(FastAcc &acc, uint32_t lane, int *kk) {
+#pragma unroll
+  for (int i = 0; i < ROWS_PER_THREAD / 2; i++) {
     uint32_t k = 0;
 #pragma unroll
     for (int pr = 0; pr < 2; pr++) {
@@ -1966,16 +2032,12 @@ __device__ __forceinline__ void coverage_msaa_rp(uint32_t (&acc)[FAST_ACC_ROWS][
       const uint4 p = *slot;
       *slot = make_uint4(0u, 0u, 0u, 0u);
       const uint32_t tot = p.x + p.y + p.z + p.w;
-      const uint32_t exc = (uint32_t)wave_incl_scan((int32_t)tot) - tot;
+      uint32_t u = (uint32_t)wave_incl_scan((int32_t)tot) - tot + 0x8000u;
       const uint32_t col[4] = {p.x, p.y, p.z, p.w};
-      uint32_t u = exc + 0x8000u;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         u += col[j];
-        if (EO)
-          k += (uint32_t)__popc(u & 0x00010001u);
-        else
-          k += (uint32_t)__popc(pk_nonzero_u16(u ^ 0x8000u));
+        k += (uint32_t)__popc(pk_nonzero_u16(u ^ 0x8000u));
       }
     }
     kk[i] = (int)k;
@@ -2399,13 +2461,11 @@ k_render(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t take) {
 // -> gradient no longer stalls every entry.
 // ---------------------------------------------------------------------------
 struct FastShared {
-  // winding deltas, row-paired (coverage_msaa_rp; zero between entries)
-  uint32_t acc[FAST_ACC_ROWS][FAST_ACC_COLS];
+  FastAcc acc;  // the entry's crossings (WindMode; zero between entries)
   union {
     struct {                             // coverage (phase A)
-      // owning lane of each work item (0x80: delta -1); the owner's edge
-      // terms are read from its registers (ds_bpermute), not staged here,
-      // which keeps the block within 10 KiB: 16 workgroups per CU
+      // owning lane of the work items, at an owner's first item (its edge's
+      // terms are read from its registers by ds_bpermute)
       uint8_t own[64 * STRIP_SUBROWS];
     } a;
     struct {                             // composite
@@ -2414,10 +2474,142 @@ struct FastShared {
     } c;
   } u;
   FastDraw blk;  // the current entry's draw constants
-  // winding of the edges wholly left of the strip, as a difference array
-  // over its sample rows (zero between entries)
+  // non-zero rule: winding of the edges wholly left of the strip, as a
+  // difference array over its sample rows (zero between entries)
   int32_t ldiff[STRIP_SUBROWS + 1];
 };
+
+// Phase A: the crossings of a draw's band edges with SR sample rows from ys0
+// on, added to acc.  An edge wholly right of the strip does nothing, one
+// wholly left of it counts in every sample row it is active on (its bits of
+// `left` for even-odd, per lane, to be combined over the wave; two entries of
+// a row difference array for non-zero); the other edges' (edge, sample row)
+// items are compacted by a wave scan and spread over the lanes.
+// inner: nonzero in some lane if a crossing lies past column 0; n_cross: the
+// edges with items.
+template <int MODE, int SR>
+__device__ __forceinline__ void fast_edges(const REdge *edges, uint32_t ne, FastShared &sh,
+                                           uint32_t lane, int32_t ys0, int32_t xs_base,
+                                           uint32_t &inner, uint32_t &left, uint32_t &n_cross) {
+  constexpr int32_t COLS = TILE_W * 4;
+  inner = 0;
+  left = 0;
+  n_cross = 0;
+  for (uint32_t c0 = 0; c0 < ne; c0 += 64) {
+    const uint32_t k = c0 + lane;
+    int32_t n_sr = 0, lo = 0;
+    REdge ed{0.0, 0.0, 0.0, 0, 0};
+    if (k < ne) {
+      ed = edges[k];
+      const int32_t a = max(ed.ylo, ys0), b = min(ed.yhi2 >> 1, ys0 + SR - 1);
+      if (a <= b) {
+        n_sr = b - a + 1;
+        lo = a - ys0;
+        // the crossings are monotone in the row, so their extremes are at
+        // the first and last active rows
+        const double xa = redge_x(ed.top, ed.x_start, ed.x_inc, a);
+        const double xb = redge_x(ed.top, ed.x_start, ed.x_inc, b);
+        const double xr = (double)(xs_base + COLS) + 1.0, xl = (double)xs_base - 1.0;
+        if (xa > xr && xb > xr) {
+          n_sr = 0;
+        } else if (xa < xl && xb < xl) {  // (rounded below the first sample column)
+          if (MODE == WIND_EO) {
+            left ^= ((1u << n_sr) - 1u) << lo;
+          } else {
+            const int32_t dv = (ed.yhi2 & 1) ? -1 : 1;
+            atomicAdd(&sh.ldiff[lo], dv);
+            atomicAdd(&sh.ldiff[lo + n_sr], -dv);
+            left = 1;
+          }
+          n_sr = 0;
+        }
+      }
+    }
+    const int32_t incl = wave_incl_scan(n_sr);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
+    if (total == 0) continue;  // uniform
+    if (MODE == WIND_NZ) n_cross += (uint32_t)__popcll(__ballot(n_sr > 0));
+    const uint32_t my_off = (uint32_t)(incl - n_sr);
+    // an owner's first item, first row and direction
+    const uint32_t info = ((ed.yhi2 & 1) ? 0x80000000u : 0u) | ((uint32_t)lo << 16) | my_off;
+    // owners in lane order have items in order: each marks its first item,
+    // and an item's owner is the largest mark up to it
+    reinterpret_cast<uint4 *>(sh.u.a.own)[lane] = make_uint4(0u, 0u, 0u, 0u);
+    wave_lds_sync();
+    if (n_sr > 0) sh.u.a.own[my_off] = (uint8_t)lane;
+    wave_lds_sync();
+    uint32_t before = 0;  // the owner of the last item of the round before
+    // every lane takes part in each round's scan and register reads (the
+    // owner of an item may be a lane with no item of its own this round)
+    for (uint32_t it0 = 0; it0 < total; it0 += 64) {
+      const uint32_t it = it0 + lane;
+      const uint32_t lj = max(
+          (uint32_t)wave_max_scan((int32_t)sh.u.a.own[it & (64u * STRIP_SUBROWS - 1u)]), before);
+      before = (uint32_t)__builtin_amdgcn_readlane((int32_t)lj, 63);
+      const uint32_t q = lane_read_u32(info, lj);
+      const double etop = lane_read_f64(ed.top, lj), exs = lane_read_f64(ed.x_start, lj),
+                   exi = lane_read_f64(ed.x_inc, lj);
+      if (it >= total) continue;
+      const uint32_t sr = ((q >> 16) & 0x7FFFu) + (it - (q & 0xFFFFu));
+      const int32_t x = round_i32(redge_x(etop, exs, exi, ys0 + (int32_t)sr));
+      const int32_t xr = x - xs_base;
+      if (xr >= COLS) continue;
+      const int32_t col = xr < 0 ? 0 : xr;
+      inner |= (uint32_t)col;
+      if (MODE == WIND_EO) {
+        atomicXor(&sh.acc[0][col], 1u << sr);
+      } else {
+        const uint32_t dv = (q >> 31) ? 0xFFFFFFFFu : 1u;
+        if (MODE == WIND_NZ)
+          atomicAdd(&sh.acc[sr >> 2][col], dv << (8u * (sr & 3u)));
+        else
+          atomicAdd(&sh.acc[sr >> 1][col], dv << (16u * (sr & 1u)));
+      }
+    }
+    wave_lds_sync();
+  }
+}
+
+// The non-zero rule's left edges: each sample row's winding from the
+// difference array (cleared), in lane `row`, 0 in the others.
+__device__ __forceinline__ int32_t left_windings(FastShared &sh, uint32_t lane) {
+  wave_lds_sync();
+  int32_t dl = 0;
+  if (lane <= (uint32_t)STRIP_SUBROWS) {
+    dl = lane < (uint32_t)STRIP_SUBROWS ? sh.ldiff[lane] : 0;
+    sh.ldiff[lane] = 0;
+  }
+  const int32_t wl = wave_incl_scan(dl);
+  return lane < (uint32_t)STRIP_SUBROWS ? wl : 0;
+}
+
+// The non-zero rule's coverage of a strip whose windings may not fit a byte:
+// its two halves one after the other, two sample rows to a word.
+__device__ __forceinline__ void coverage_halves(const REdge *edges, uint32_t ne, FastShared &sh,
+                                             uint32_t lane, int32_t ys_base, int32_t xs_base,
+                                             int *kk) {
+#pragma unroll 1
+  for (int h = 0; h < 2; h++) {
+    uint32_t inner, left, n_cross;
+    fast_edges<WIND_NZ16, STRIP_SUBROWS / 2>(edges, ne, sh, lane,
+                                             ys_base + h * (STRIP_SUBROWS / 2), xs_base, inner,
+                                             left, n_cross);
+    const int32_t wl = left_windings(sh, lane);
+    if (wl != 0 && lane < (uint32_t)STRIP_SUBROWS / 2)
+      atomicAdd(&sh.acc[lane >> 1][0], (uint32_t)wl << (16u * (lane & 1u)));
+    wave_lds_sync();
+    int k2[ROWS_PER_THREAD / 2];
+    coverage_nz16(sh.acc, lane, k2);
+    if (h == 0) {
+      kk[0] = k2[0];
+      kk[1] = k2[1];
+    } else {
+      kk[2] = k2[0];
+      kk[3] = k2[1];
+    }
+    wave_lds_sync();
+  }
+}
 
 // Gradient.getOffset (src/gradient.zig:349-375, :605-652, :731-742) on a
 // fast draw's block: the arithmetic of linear_offset / radial_offset /
@@ -2569,7 +2761,6 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
     // packed alpha surfaces hold fewer bits than a lane between draws
     const int a_bits = S.fmt >= Z2D_FORMAT_ALPHA4 ? fmt_bits(S.fmt) : 8;
     const int32_t ys_base = ty0 * 4, xs_base = tx0 * 4;
-    constexpr int32_t COLS = TILE_W * 4, SR = ROWS_PER_THREAD * 4;
 
     for (uint32_t c = e0; c < e1; c += 64) {
       // this chunk's entries, one per lane
@@ -2611,101 +2802,47 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
         const REdge *edges = J.entry_edges + __builtin_amdgcn_readlane(g_off, j);
         if (J.count_stats) stat_entries++;
 
-        // ---- phase A: winding deltas of the band edges (as k_render; an
-        // edge wholly left of the strip adds its direction at column 0 of
-        // each of its rows through two entries of a row difference array)
-        uint32_t inner = 0;
-        bool any_left = false;
-        for (uint32_t c0 = 0; c0 < ne; c0 += 64) {
-          const uint32_t k = c0 + lane;
-          int32_t n_sr = 0, lo = 0;
-          REdge ed{0.0, 0.0, 0.0, 0, 0};
-          if (k < ne) {
-            ed = edges[k];
-            const int32_t a = max(ed.ylo, ys_base), b = min(ed.yhi2 >> 1, ys_base + SR - 1);
-            if (a <= b) {
-              n_sr = b - a + 1;
-              lo = a - ys_base;
-              const double xa = redge_x(ed.top, ed.x_start, ed.x_inc, a);
-              const double xb = redge_x(ed.top, ed.x_start, ed.x_inc, b);
-              if (fmin(xa, xb) > (double)(xs_base + COLS) + 1.0) {
-                n_sr = 0;  // every crossing right of the strip: none here
-              } else if (fmax(xa, xb) < (double)xs_base - 1.0) {
-                // every crossing left of the strip (rounded below its first
-                // sample column): column 0 of rows [lo, lo + n_sr)
-                const int32_t dv = (!eo && (ed.yhi2 & 1)) ? -1 : 1;
-                atomicAdd(&sh.ldiff[lo], dv);
-                atomicAdd(&sh.ldiff[lo + n_sr], -dv);
-                any_left = true;
-                n_sr = 0;
-              }
-            }
-          }
-          const int32_t incl = wave_incl_scan(n_sr);
-          const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
-          if (total == 0) continue;  // uniform
-          const uint32_t my_off = (uint32_t)(incl - n_sr);
-          const uint32_t lo_off = ((uint32_t)lo << 16) | my_off;
-          const uint8_t tag = (uint8_t)(lane | ((!eo && (ed.yhi2 & 1)) ? 0x80u : 0u));
-          for (int t = 0; t < n_sr; t++) sh.u.a.own[my_off + (uint32_t)t] = tag;
-          wave_lds_sync();
-          // every lane takes part in each round's register reads (the owner
-          // of an item may be a lane with no item of its own this round)
-          for (uint32_t it0 = 0; it0 < total; it0 += 64) {
-            const uint32_t it = it0 + lane;
-            const bool live = it < total;
-            const uint32_t v = live ? (uint32_t)sh.u.a.own[it] : 0u;
-            const uint32_t lj = v & 63u;
-            const uint32_t q = lane_read_u32(lo_off, lj);
-            const double etop = lane_read_f64(ed.top, lj), exs = lane_read_f64(ed.x_start, lj),
-                         exi = lane_read_f64(ed.x_inc, lj);
-            if (!live) continue;
-            const int sr = (int)(q >> 16) + (int)(it - (q & 0xFFFFu));
-            const int32_t x = round_i32(redge_x(etop, exs, exi, ys_base + sr));
-            const int32_t xr = x - xs_base;
-            if (xr >= COLS) continue;
-            const int32_t col = xr < 0 ? 0 : xr;
-            inner |= (uint32_t)col;
-            const uint32_t dv = (v & 0x80u) ? 0xFFFFFFFFu : 1u;
-            atomicAdd(&sh.acc[sr >> 1][col], (sr & 1) ? (dv << 16) : dv);
-          }
-          wave_lds_sync();
-        }
-
-        if (__ballot(any_left)) {
-          // the left edges' winding per row: prefix of the difference array
-          wave_lds_sync();
-          int32_t dl = 0;
-          if (lane <= (uint32_t)SR) {
-            dl = lane < (uint32_t)SR ? sh.ldiff[lane] : 0;
-            sh.ldiff[lane] = 0;
-          }
-          const int32_t wl = wave_incl_scan(dl);
-          if (lane < (uint32_t)SR && wl != 0)
-            atomicAdd(&sh.acc[lane >> 1][0], (lane & 1) ? ((uint32_t)wl << 16) : (uint32_t)wl);
-          wave_lds_sync();
-        }
-
-        // ---- phase B: covered samples per pixel
+        // ---- phases A and B: covered samples per pixel
         int kk[ROWS_PER_THREAD];
-        if (__ballot(inner != 0) == 0) {
-          // every delta at column 0: uniform winding across each sample row
-          // (lane = sample row; the even lane clears the pair's word)
-          uint32_t w0 = 0;
-          if (lane < (uint32_t)SR) w0 = sh.acc[lane >> 1][0];
-          wave_lds_sync();
-          if (lane < (uint32_t)SR && !(lane & 1)) sh.acc[lane >> 1][0] = 0u;
-          int32_t wl, wh;
-          unpack_pair(w0, wl, wh);
-          const int32_t w_row = (lane & 1) ? wh : wl;
-          const uint64_t in_rows = __ballot(lane < (uint32_t)SR && wind_in(w_row, eo));
-#pragma unroll
-          for (int i = 0; i < ROWS_PER_THREAD; i++)
-            kk[i] = 4 * __popcll((in_rows >> (4 * i)) & 0xFull);
-        } else if (eo) {
-          coverage_msaa_rp<true>(sh.acc, lane, kk);
+        uint32_t inner, left, n_cross;
+        if (eo) {
+          fast_edges<WIND_EO, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, inner, left,
+                                             n_cross);
+          if (__ballot(left != 0))  // parity of the left edges over the wave
+            left = (uint32_t)__builtin_amdgcn_readlane((int32_t)wave_xor_scan(left), 63);
+          coverage_eo(sh.acc, lane, left, kk);
         } else {
-          coverage_msaa_rp<false>(sh.acc, lane, kk);
+          fast_edges<WIND_NZ, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, inner, left,
+                                             n_cross);
+          int32_t wl = 0;
+          if (__ballot(left != 0)) {
+            wl = left_windings(sh, lane);
+            if (wl != 0) atomicAdd(&sh.acc[lane >> 2][0], (uint32_t)wl << (8u * (lane & 3u)));
+          }
+          wave_lds_sync();
+          // |winding| <= half the edges (contours return to their start), and
+          // <= that at the strip's left plus the edges crossing it
+          if (ne > 254u && n_cross + (uint32_t)wave_max_i32(abs(wl)) > 127u) {
+#pragma unroll
+            for (int i = 0; i < FAST_ACC_ROWS; i++)
+              *reinterpret_cast<uint4 *>(&sh.acc[i][lane * 4]) = make_uint4(0u, 0u, 0u, 0u);
+            wave_lds_sync();
+            coverage_halves(edges, ne, sh, lane, ys_base, xs_base, kk);
+          } else if (__ballot(inner != 0) == 0) {
+            // every crossing at column 0: uniform winding across each sample
+            // row (lane = sample row; every fourth lane clears the word)
+            uint32_t w0 = 0;
+            if (lane < (uint32_t)STRIP_SUBROWS) w0 = sh.acc[lane >> 2][0];
+            wave_lds_sync();
+            if (lane < (uint32_t)STRIP_SUBROWS && !(lane & 3u)) sh.acc[lane >> 2][0] = 0u;
+            const bool in = (((w0 + 0x80808080u) >> (8u * (lane & 3u))) & 0xFFu) != 0x80u;
+            const uint64_t in_rows = __ballot(lane < (uint32_t)STRIP_SUBROWS && in);
+#pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++)
+              kk[i] = 4 * __popcll((in_rows >> (4 * i)) & 0xFull);
+          } else {
+            coverage_nz(sh.acc, lane, kk);
+          }
         }
         wave_lds_sync();
 
