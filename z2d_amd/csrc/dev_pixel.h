@@ -636,6 +636,32 @@ Z2D_PX __forceinline__ void user_to_device(const double *m, double &x, double &y
   x = ox + m[4];
   y = oy + m[5];
 }
+// A double constant, with LOCAL made where it is used, in scalar (KONST_S) or
+// vector (KONST_V) registers.  The compiler lifts constants out of the fast
+// strip worker's loops, where an atan2's three dozen took vector registers
+// for the whole kernel (20 of 119).
+#if defined(__HIP_DEVICE_COMPILE__)
+template <uint64_t BITS>
+__device__ __forceinline__ double konst_s() {
+  uint32_t lo, hi;
+  asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"((uint32_t)BITS));
+  asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((uint32_t)(BITS >> 32)));
+  return __hiloint2double((int)hi, (int)lo);
+}
+template <uint64_t BITS>
+__device__ __forceinline__ double konst_v() {
+  uint32_t lo, hi;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(lo) : "i"((uint32_t)BITS));
+  asm volatile("v_mov_b32 %0, %1" : "=v"(hi) : "i"((uint32_t)(BITS >> 32)));
+  return __hiloint2double((int)hi, (int)lo);
+}
+#define KONST_S(c) (LOCAL ? konst_s<__builtin_bit_cast(uint64_t, (double)(c))>() : (c))
+#define KONST_V(c) (LOCAL ? konst_v<__builtin_bit_cast(uint64_t, (double)(c))>() : (c))
+#else
+#define KONST_S(c) (c)
+#define KONST_V(c) (c)
+#endif
+
 // std.math.atan / std.math.atan2 for f64 as Zig's standard library computes
 // them (lib/std/math/atan.zig, atan2.zig, the reference's third-party
 // dependency): the published fdlibm algorithm (Sun Microsystems
@@ -644,17 +670,18 @@ Z2D_PX __forceinline__ void user_to_device(const double *m, double &x, double &y
 // chains and adds atan of the range's centre in two parts; atan2 handles
 // signs, zeros and infinities and takes atan(|y/x|).  A few live doubles,
 // so a conic gradient's sampler stays small.
+template <bool LOCAL>
 Z2D_PX __forceinline__ double zatan(double x) {
-  const double atanhi0 = 4.63647609000806093515e-01, atanhi1 = 7.85398163397448278999e-01,
-               atanhi2 = 9.82793723247329054082e-01, atanhi3 = 1.57079632679489655800e+00;
-  const double atanlo0 = 2.26987774529616870924e-17, atanlo1 = 3.06161699786838301793e-17,
-               atanlo2 = 1.39033110312309984516e-17, atanlo3 = 6.12323399573676603587e-17;
+  constexpr double atanhi0 = 4.63647609000806093515e-01, atanhi1 = 7.85398163397448278999e-01,
+                   atanhi2 = 9.82793723247329054082e-01, atanhi3 = 1.57079632679489655800e+00;
+  constexpr double atanlo0 = 2.26987774529616870924e-17, atanlo1 = 3.06161699786838301793e-17,
+                   atanlo2 = 1.39033110312309984516e-17, atanlo3 = 6.12323399573676603587e-17;
   uint32_t ix = dhi(x);
   const uint32_t sign = ix >> 31;
   ix &= 0x7FFFFFFFu;
   if (ix >= 0x44100000u) {  // |x| >= 2^66
     if (z_isnan(x)) return x;
-    const double z = atanhi3 + 0x1.0p-120;
+    const double z = KONST_V(atanhi3) + 0x1.0p-120;
     return sign ? -z : z;
   }
   int id;
@@ -682,52 +709,60 @@ Z2D_PX __forceinline__ double zatan(double x) {
   const double z = x * x;
   const double w = z * z;
   const double s1 =
-      z * (3.33333333333329318027e-01 +
-           w * (1.42857142725034663711e-01 +
-                w * (9.09088713343650656196e-02 +
-                     w * (6.66107313738753120669e-02 +
-                          w * (4.97687799461593236017e-02 + w * 1.62858201153657823623e-02)))));
+      z * (KONST_S(3.33333333333329318027e-01) +
+           w * (KONST_S(1.42857142725034663711e-01) +
+                w * (KONST_S(9.09088713343650656196e-02) +
+                     w * (KONST_S(6.66107313738753120669e-02) +
+                          w * (KONST_S(4.97687799461593236017e-02) +
+                               w * KONST_S(1.62858201153657823623e-02))))));
   const double s2 =
-      w * (-1.99999999998764832476e-01 +
-           w * (-1.11111104054623557880e-01 +
-                w * (-7.69187620504482999495e-02 +
-                     w * (-5.83357013379057348645e-02 + w * -3.65315727442169155270e-02))));
+      w * (KONST_S(-1.99999999998764832476e-01) +
+           w * (KONST_S(-1.11111104054623557880e-01) +
+                w * (KONST_S(-7.69187620504482999495e-02) +
+                     w * (KONST_S(-5.83357013379057348645e-02) +
+                          w * KONST_S(-3.65315727442169155270e-02)))));
   if (id < 0) return x - x * (s1 + s2);
-  const double hi = id == 0 ? atanhi0 : id == 1 ? atanhi1 : id == 2 ? atanhi2 : atanhi3;
-  const double lo = id == 0 ? atanlo0 : id == 1 ? atanlo1 : id == 2 ? atanlo2 : atanlo3;
+  double hi = KONST_V(atanhi3), lo = KONST_V(atanlo3);
+  if (id == 0) hi = KONST_V(atanhi0), lo = KONST_V(atanlo0);
+  if (id == 1) hi = KONST_V(atanhi1), lo = KONST_V(atanlo1);
+  if (id == 2) hi = KONST_V(atanhi2), lo = KONST_V(atanlo2);
   const double zz = hi - ((x * (s1 + s2) - lo) - x);
   return sign ? -zz : zz;
 }
+template <bool LOCAL = false>
 Z2D_PX __forceinline__ double zatan2(double y, double x) {
-  const double pi = 3.1415926535897931160E+00, pi_lo = 1.2246467991473531772E-16;
+  constexpr double pi = 3.1415926535897931160E+00, pi_lo = 1.2246467991473531772E-16;
   if (z_isnan(x) || z_isnan(y)) return x + y;
   uint32_t ix = dhi(x), iy = dhi(y);
   const uint32_t lx = dlo(x), ly = dlo(y);
-  if (((ix - 0x3FF00000u) | lx) == 0) return zatan(y);  // x = 1.0
+  if (((ix - 0x3FF00000u) | lx) == 0) return zatan<LOCAL>(y);  // x = 1.0
   const uint32_t m = ((iy >> 31) & 1u) | ((ix >> 30) & 2u);  // 2 sign(x) + sign(y)
   ix &= 0x7FFFFFFFu;
   iy &= 0x7FFFFFFFu;
   if ((iy | ly) == 0) {  // y = 0
     if (m < 2) return y;
-    return m == 2 ? pi : -pi;
+    return m == 2 ? KONST_V(pi) : KONST_V(-pi);
   }
-  if ((ix | lx) == 0) return (m & 1u) ? -pi / 2 : pi / 2;  // x = 0
+  if ((ix | lx) == 0) return (m & 1u) ? KONST_V(-pi / 2) : KONST_V(pi / 2);  // x = 0
   if (ix == 0x7FF00000u) {  // x infinite
     if (iy == 0x7FF00000u)
-      return m == 0 ? pi / 4 : m == 1 ? -pi / 4 : m == 2 ? 3 * pi / 4 : -3 * pi / 4;
-    return m == 0 ? 0.0 : m == 1 ? -0.0 : m == 2 ? pi : -pi;
+      return m == 0   ? KONST_V(pi / 4)
+             : m == 1 ? KONST_V(-pi / 4)
+             : m == 2 ? KONST_V(3 * pi / 4)
+                      : KONST_V(-3 * pi / 4);
+    return m == 0 ? 0.0 : m == 1 ? -0.0 : m == 2 ? KONST_V(pi) : KONST_V(-pi);
   }
   if (ix + (64u << 20) < iy || iy == 0x7FF00000u)  // |y/x| > 2^64
-    return (m & 1u) ? -pi / 2 : pi / 2;
+    return (m & 1u) ? KONST_V(-pi / 2) : KONST_V(pi / 2);
   double z;
   if ((m & 2u) && iy + (64u << 20) < ix)  // |y/x| < 2^-64, x < 0
     z = 0.0;
   else
-    z = zatan(fabs(y / x));
+    z = zatan<LOCAL>(fabs(y / x));
   if (m == 0) return z;
   if (m == 1) return -z;
-  if (m == 2) return pi - (z - pi_lo);
-  return (z - pi_lo) - pi;
+  if (m == 2) return KONST_S(pi) - (z - KONST_S(pi_lo));
+  return (z - KONST_S(pi_lo)) - KONST_S(pi);
 }
 
 Z2D_PX __forceinline__ double dclamp01(double v) { return fmax(0.0, fmin(v, 1.0)); }
@@ -843,21 +878,25 @@ Z2D_PX __forceinline__ void stops_find8(const float *st, uint32_t n_stops, float
   const int n = (int)n_stops;
   transparent = offset < 0.0f || n == 0;
   const float o = fminz(offset, 1.0f);
-  const float4 a = *reinterpret_cast<const float4 *>(st);
-  const float4 b = *reinterpret_cast<const float4 *>(st + 4);
   // The offset is never NaN (fminf) and the stops are finite or +inf, so
   // each difference st[k] - o is +0 exactly when st[k] == o (x - x), has its
   // sign bit set exactly when st[k] < o (a difference of distinct floats is
   // never +0, and a flushed one keeps its sign), and is +inf for padding:
   // the stops below the offset are the differences' sign bits, and a tie is
-  // a zero smallest magnitude.
-  const float d[8] = {a.x - o, a.y - o, a.z - o, a.w - o, b.x - o, b.y - o, b.z - o, b.w - o};
+  // a zero smallest magnitude.  The second four are looked at only where
+  // there are that many (n_stops is wave-uniform).
   uint32_t nb = 0;
+  float dmin = __builtin_inff();
+  auto four = [&](const float *q) {
+    const float4 a = *reinterpret_cast<const float4 *>(q);
+    const float d[4] = {a.x - o, a.y - o, a.z - o, a.w - o};
 #pragma unroll
-  for (int k = 0; k < 8; k++) nb += __builtin_bit_cast(uint32_t, d[k]) >> 31;
+    for (int k = 0; k < 4; k++) nb += __builtin_bit_cast(uint32_t, d[k]) >> 31;
+    dmin = fminf(dmin, fminf(fminf(fabsf(d[0]), fabsf(d[1])), fminf(fabsf(d[2]), fabsf(d[3]))));
+  };
+  four(st);
+  if (n > 4) four(st + 4);
   const int below = (int)nb;
-  const float dmin = fminf(fminf(fminf(fabsf(d[0]), fabsf(d[1])), fminf(fabsf(d[2]), fabsf(d[3]))),
-                           fminf(fminf(fabsf(d[4]), fabsf(d[5])), fminf(fabsf(d[6]), fabsf(d[7]))));
   const bool tie = dmin == 0.0f;
   if (transparent) {
     i0 = i1 = 0;
