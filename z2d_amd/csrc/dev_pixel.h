@@ -404,22 +404,44 @@ Z2D_PX inline I4 op_int(uint32_t op, I4 d, I4 s) {
 // ---------------------------------------------------------------------------
 // float operators
 // ---------------------------------------------------------------------------
-Z2D_PX __forceinline__ float dodge_ch(float s, float d, float sa, float da) {
+// Quotients by one divisor: its reciprocal, correctly rounded, once, then per
+// numerator a product and one correction by the exact remainder, which gives
+// the correctly rounded quotient (Markstein's theorem; three instructions
+// where a division takes ten).  A zero divisor keeps the product with the
+// infinite reciprocal, which is the division's infinity or NaN; divisors so
+// small or large that the reciprocal or the remainder could leave the normal
+// range (no 8-bit lane gives one) are divided by.
+struct Divisor {
+  float b, y;
+  bool plain;
+};
+Z2D_PX __forceinline__ Divisor divisor(float b) {
+  const float m = fabsf(b);
+  return Divisor{b, 1.0f / b, !(m == 0.0f || (m >= 0x1p-60f && m <= 0x1p60f))};
+}
+Z2D_PX __forceinline__ float div_by(float a, const Divisor &d) {
+  if (d.plain) return a / d.b;
+  const float q = a * d.y;
+  const float r = __builtin_fmaf(__builtin_fmaf(-d.b, q, a), d.y, q);
+  return d.b == 0.0f ? q : r;
+}
+
+// m: d / da
+Z2D_PX __forceinline__ float dodge_ch(float s, float d, float sa, float da, float m) {
   if (s == sa && d == 0.0f) return s * (1.0f - da);
   if (s == sa) return sa * da + s * (1.0f - da) + d * (1.0f - sa);
-  return sa * da * fminz(1.0f, d / da * sa / (sa - s)) + s * (1.0f - da) + d * (1.0f - sa);
+  return sa * da * fminz(1.0f, m * sa / (sa - s)) + s * (1.0f - da) + d * (1.0f - sa);
 }
 // The reference's p0 receives (sca, dca, sa): its first branch tests
 // sca == 0 && dca == sa.
-Z2D_PX __forceinline__ float burn_ch(float s, float d, float sa, float da) {
+Z2D_PX __forceinline__ float burn_ch(float s, float d, float sa, float da, float m) {
   if (s == 0.0f && d == sa) return sa * da + d * (1.0f - sa);
   if (s == 0.0f) return d * (1.0f - sa);
-  return sa * da * (1.0f - fminz(1.0f, (1.0f - d / da) * sa / s)) + s * (1.0f - da) +
+  return sa * da * (1.0f - fminz(1.0f, (1.0f - m) * sa / s)) + s * (1.0f - da) +
          d * (1.0f - sa);
 }
-Z2D_PX __forceinline__ float soft_ch(float s, float d, float sa, float da) {
+Z2D_PX __forceinline__ float soft_ch(float s, float d, float sa, float da, float m) {
   if (da == 0.0f) return s;
-  float m = d / da;
   if (2.0f * s <= sa)
     return d * (sa + (2.0f * s - sa) * (1.0f - m)) + s * (1.0f - da) + d * (1.0f - sa);
   if (4.0f * d <= da)
@@ -436,30 +458,34 @@ Z2D_PX __forceinline__ float mn3(F3 c) { return fminz(fminz(c.r, c.g), c.b); }
 Z2D_PX __forceinline__ float lum3(F3 c) { return c.r * 0.3f + c.g * 0.59f + c.b * 0.11f; }
 // clipColor with the reference's vector semantics: the x>a branch wins over
 // the n<0 branch and both read the unclipped channel.
-Z2D_PX __forceinline__ float clip1(float c, float l, float n, float x, float a) {
-  float r = c;
+Z2D_PX __forceinline__ F3 clip3(F3 c, float a) {
+  const float l = lum3(c), n = mn3(c), x = mx3(c);
+  F3 r = c;
   if (n < 0.0f) {
-    float t = l - n;
-    r = t == 0.0f ? 0.0f : l + ((c - l) * l) / t;
+    const float t = l - n;
+    const Divisor d = divisor(t);
+    r = t == 0.0f ? F3{0.0f, 0.0f, 0.0f}
+                  : F3{l + div_by((c.r - l) * l, d), l + div_by((c.g - l) * l, d),
+                       l + div_by((c.b - l) * l, d)};
   }
   if (x > a) {
-    float t = x - l;
-    r = t == 0.0f ? 0.0f : l + ((c - l) * (a - l)) / t;
+    const float t = x - l, al = a - l;
+    const Divisor d = divisor(t);
+    r = t == 0.0f ? F3{0.0f, 0.0f, 0.0f}
+                  : F3{l + div_by((c.r - l) * al, d), l + div_by((c.g - l) * al, d),
+                       l + div_by((c.b - l) * al, d)};
   }
   return r;
-}
-Z2D_PX __forceinline__ F3 clip3(F3 c, float a) {
-  float l = lum3(c), n = mn3(c), x = mx3(c);
-  return F3{clip1(c.r, l, n, x, a), clip1(c.g, l, n, x, a), clip1(c.b, l, n, x, a)};
 }
 Z2D_PX __forceinline__ F3 setlum3(F3 c, float l) {
   float d = l - lum3(c);
   return F3{c.r + d, c.g + d, c.b + d};
 }
 Z2D_PX __forceinline__ F3 setsat3(F3 c, float s) {
-  float n = mn3(c), x = mx3(c), d = x - n;
-  return F3{d == 0.0f ? 0.0f : (c.r - n) * s / d, d == 0.0f ? 0.0f : (c.g - n) * s / d,
-            d == 0.0f ? 0.0f : (c.b - n) * s / d};
+  const float n = mn3(c), x = mx3(c), d = x - n;
+  if (d == 0.0f) return F3{0.0f, 0.0f, 0.0f};
+  const Divisor q = divisor(d);
+  return F3{div_by((c.r - n) * s, q), div_by((c.g - n) * s, q), div_by((c.b - n) * s, q)};
 }
 Z2D_PX __forceinline__ F4 ns_out(F3 c, F4 d, F4 s) {
   return F4{s.r * (1.0f - d.a) + d.r * (1.0f - s.a) + c.r,
@@ -516,12 +542,18 @@ Z2D_PX inline F4 op_float(uint32_t op, F4 d, F4 s) {
       return F4{fmaxz(s.r * d.a, d.r * s.a) + s.r * (1.0f - d.a) + d.r * (1.0f - s.a),
                 fmaxz(s.g * d.a, d.g * s.a) + s.g * (1.0f - d.a) + d.g * (1.0f - s.a),
                 fmaxz(s.b * d.a, d.b * s.a) + s.b * (1.0f - d.a) + d.b * (1.0f - s.a), ua};
-    case Z2D_OP_COLOR_DODGE:
-      return F4{dodge_ch(s.r, d.r, s.a, d.a), dodge_ch(s.g, d.g, s.a, d.a),
-                dodge_ch(s.b, d.b, s.a, d.a), ua};
-    case Z2D_OP_COLOR_BURN:
-      return F4{burn_ch(s.r, d.r, s.a, d.a), burn_ch(s.g, d.g, s.a, d.a),
-                burn_ch(s.b, d.b, s.a, d.a), ua};
+    case Z2D_OP_COLOR_DODGE: {
+      const Divisor q = divisor(d.a);
+      return F4{dodge_ch(s.r, d.r, s.a, d.a, div_by(d.r, q)),
+                dodge_ch(s.g, d.g, s.a, d.a, div_by(d.g, q)),
+                dodge_ch(s.b, d.b, s.a, d.a, div_by(d.b, q)), ua};
+    }
+    case Z2D_OP_COLOR_BURN: {
+      const Divisor q = divisor(d.a);
+      return F4{burn_ch(s.r, d.r, s.a, d.a, div_by(d.r, q)),
+                burn_ch(s.g, d.g, s.a, d.a, div_by(d.g, q)),
+                burn_ch(s.b, d.b, s.a, d.a, div_by(d.b, q)), ua};
+    }
     case Z2D_OP_HARD_LIGHT: {
 #define Z2D_HL(sc, dc)                                                                    \
   ((2.0f * (sc) <= s.a) ? (2.0f * (sc) * (dc) + (sc) * (1.0f - d.a) + (dc) * (1.0f - s.a)) \
@@ -529,9 +561,12 @@ Z2D_PX inline F4 op_float(uint32_t op, F4 d, F4 s) {
       return F4{Z2D_HL(s.r, d.r), Z2D_HL(s.g, d.g), Z2D_HL(s.b, d.b), ua};
 #undef Z2D_HL
     }
-    case Z2D_OP_SOFT_LIGHT:
-      return F4{soft_ch(s.r, d.r, s.a, d.a), soft_ch(s.g, d.g, s.a, d.a),
-                soft_ch(s.b, d.b, s.a, d.a), ua};
+    case Z2D_OP_SOFT_LIGHT: {
+      const Divisor q = divisor(d.a);
+      return F4{soft_ch(s.r, d.r, s.a, d.a, div_by(d.r, q)),
+                soft_ch(s.g, d.g, s.a, d.a, div_by(d.g, q)),
+                soft_ch(s.b, d.b, s.a, d.a, div_by(d.b, q)), ua};
+    }
     case Z2D_OP_DIFFERENCE:
       return F4{s.r + d.r - 2.0f * fminz(s.r * d.a, d.r * s.a),
                 s.g + d.g - 2.0f * fminz(s.g * d.a, d.g * s.a),
@@ -577,8 +612,14 @@ __host__ __device__ __forceinline__ bool op_is_bounded(uint32_t op) {
            op == Z2D_OP_DST_ATOP);
 }
 
+// v / 255 in f32: the product with the rounded reciprocal corrected by the
+// remainder, equal to the division for every v below 65536.
+Z2D_PX __forceinline__ float div255f(uint32_t v) {
+  const float x = (float)v, q = x * (1.0f / 255.0f);
+  return __builtin_fmaf(__builtin_fmaf(-255.0f, q, x), 1.0f / 255.0f, q);
+}
 Z2D_PX __forceinline__ F4 decode_raw(I4 v) {
-  return F4{(float)v.r / 255.0f, (float)v.g / 255.0f, (float)v.b / 255.0f, (float)v.a / 255.0f};
+  return F4{div255f(v.r), div255f(v.g), div255f(v.b), div255f(v.a)};
 }
 Z2D_PX __forceinline__ I4 encode_raw(F4 v) {
   return I4{f2u8(255.0f * v.r), f2u8(255.0f * v.g), f2u8(255.0f * v.b), f2u8(255.0f * v.a)};
