@@ -41,6 +41,8 @@ hipError_t z2d_launch_binning(const JobView &J, hipStream_t st);
 hipError_t z2d_launch_render(const JobView &J, uint32_t tile_base, uint32_t tile_count,
                              hipStream_t st);
 hipError_t z2d_launch_composite_quad(const z2d::QuadJob &job, hipStream_t st);
+hipError_t z2d_launch_composite_paint(const z2d::PaintJob &job, uint32_t kind, bool dither,
+                                      hipStream_t st);
 hipError_t z2d_launch_flatten(const z2d_path_node *raw, const z2d::FlatJob *jobs, uint32_t n_jobs,
                               z2d::FNode *out, z2d::FlatResult *res, uint32_t *rel,
                               const uint2 *curves, uint32_t n_curves, z2d::FlatTask *tasks,
@@ -1783,6 +1785,44 @@ static bool quad_job(const CompJob &job, QuadJob &q) {
   return true;
 }
 
+// The batches the paint kernel takes: one operator in integer precision onto
+// a 4-byte destination from a gradient or dither (whose region is the whole
+// surface), its gradient interpolated in linear RGB with at most FAST_STOPS
+// stops.  kind: the gradient's type, or 3 for the dither of a color.
+static bool paint_job(const CompJob &job, const z2d_comp_op &op, PaintJob &p, uint32_t &kind,
+                      bool &dither) {
+  const DevCompOp &o = job.ops[0];
+  if (job.n_ops != 1 || job.precision != Z2D_PRECISION_INTEGER ||
+      o.dst.kind != Z2D_PARAM_NONE || fbits(job.dst.fmt) != 32 || fbits(job.out.fmt) != 32 ||
+      (reinterpret_cast<uintptr_t>(job.dst.data) & 3) ||
+      (reinterpret_cast<uintptr_t>(job.out.data) & 3) || job.x0 != 0 || job.y0 != 0 ||
+      job.width != job.dst.w || job.height != job.dst.h || job.dst.w > 0x40000000)
+    return false;
+  const z2d_gradient_desc *g = nullptr;
+  if (o.src.kind == Z2D_PARAM_GRADIENT) {
+    g = op.src.gradient;
+    dither = false;
+  } else if (o.src.kind == Z2D_PARAM_DITHER) {
+    if (op.src.dither.source == Z2D_DITHER_SRC_GRADIENT) g = op.src.dither.gradient;
+    dither = true;
+    if (op.src.dither.scale > 30 || op.src.dither.type > Z2D_DITHER_BLUE_NOISE) return false;
+  } else {
+    return false;
+  }
+  if (g && (g->method != Z2D_INTERP_LINEAR_RGB || g->n_stops > FAST_STOPS || g->type > 2))
+    return false;
+  if (!g && !(dither && op.src.dither.source != Z2D_DITHER_SRC_GRADIENT)) return false;
+  kind = g ? g->type : 3u;
+  p.dst = reinterpret_cast<const uint32_t *>(job.dst.data);
+  p.out = reinterpret_cast<uint32_t *>(job.out.data);
+  p.w = job.dst.w;
+  p.h = job.dst.h;
+  p.dst_fmt = job.dst.fmt;
+  p.out_fmt = job.out.fmt;
+  p.op = o.op;
+  return true;
+}
+
 // noalloc: the variant that allocates no device or pinned memory: every
 // surface must be a device descriptor, the job lives in the device's fixed
 // scratch (a job larger than it is refused) and is staged from pageable
@@ -1989,10 +2029,20 @@ static int32_t composite_impl(z2d_gpu_ctx *ctx, z2d_surface_desc *dst_d, int32_t
         if (e == hipSuccess && !ctx->ev[1]) e = hipEventCreate(&ctx->ev[1]);
         if (e == hipSuccess) e = hipEventRecord(ctx->ev[0], ctx->stream);
       }
-      if (e == hipSuccess)
-        e = quad ? z2d_launch_composite_quad(qj, ctx->stream)
-                 : z2d_launch_composite(reinterpret_cast<const CompJob *>(D + o_job), job, stream,
-                                        ctx->stream);
+      PaintJob pj;
+      uint32_t kind = 0;
+      bool dither = false;
+      if (e != hipSuccess) {
+      } else if (quad) {
+        e = z2d_launch_composite_quad(qj, ctx->stream);
+      } else if (paint_job(job, ops[0], pj, kind, dither)) {
+        pj.paint = job.ops[0].src.paint;
+        pj.blue_noise = job.blue_noise;
+        e = z2d_launch_composite_paint(pj, kind, dither, ctx->stream);
+      } else {
+        e = z2d_launch_composite(reinterpret_cast<const CompJob *>(D + o_job), job, stream,
+                                 ctx->stream);
+      }
       if (e == hipSuccess && !noalloc) e = hipEventRecord(ctx->ev[1], ctx->stream);
       if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
       float ms = 0.0f;

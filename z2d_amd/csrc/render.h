@@ -330,6 +330,18 @@ struct QuadJob {
   QuadSrc src, mask;
 };
 
+// SurfaceCompositor batches of one operator in integer precision that paint a
+// whole 4-byte surface with a gradient (linear RGB, at most FAST_STOPS stops)
+// or a dither of one or of a color.
+struct PaintJob {
+  const uint32_t *dst;
+  uint32_t *out;
+  int32_t w, h;
+  uint32_t dst_fmt, out_fmt, op;
+  const DevPaint *paint;
+  const uint16_t *blue_noise;
+};
+
 // Up to six word fills in one launch (the zeroing at the start of a render
 // pipeline): fill f writes v[f] to n[f] words at p[f].
 struct FillSet {
