@@ -109,9 +109,17 @@ Z2D_PX __forceinline__ double zmodd(double x, double y) {
 // v >= 0 (checked over all 2^32 floats with the sign copied onto the
 // addend), and for v < 0 it is at most 0 as roundf(v) is, so the clamp
 // gives 0 either way; the clamp takes NaN to 0.
+// The device's conversion truncates, takes NaN and everything below zero to 0
+// and saturates above, so there one integer minimum is left of the clamp.
 Z2D_PX __forceinline__ uint32_t f2u8(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v + 0x1.fffffep-2f));
+  return min(r, 65535u);
+#else
   const float r = truncf(v + 0x1.fffffep-2f);
   return (uint32_t)fminf(fmaxf(r, 0.0f), 65535.0f);
+#endif
 }
 
 // (int32_t)round(v) (half away from zero) as one add and the truncating

@@ -3071,22 +3071,28 @@ __global__ void __launch_bounds__(256) k_composite_stream(const CompJob *__restr
 // k_composite before, 142.7 us a pass then and 48.5 now (start and end of the
 // call included).
 // ---------------------------------------------------------------------------
+// A format's byte order as the selectors of a byte permute, to and from RGBA8
+// (0x0C selects a zero byte, 0x0D one of 255).
 struct Fmt32 {
-  uint32_t sr, sb, has_a;  // red and blue byte shifts; alpha byte present
+  uint32_t to, from;
 };
 __device__ __forceinline__ Fmt32 fmt32(uint32_t fmt) {
-  const bool bgr = fmt == Z2D_FORMAT_ARGB || fmt == Z2D_FORMAT_XRGB;
-  return Fmt32{bgr ? 16u : 0u, bgr ? 0u : 16u,
-               (fmt == Z2D_FORMAT_RGBA || fmt == Z2D_FORMAT_ARGB) ? 1u : 0u};
+  switch (fmt) {
+    case Z2D_FORMAT_ARGB: return Fmt32{0x03000102u, 0x03000102u};
+    case Z2D_FORMAT_XRGB: return Fmt32{0x0D000102u, 0x0C000102u};
+    case Z2D_FORMAT_RGB: return Fmt32{0x0D020100u, 0x0C020100u};
+    default: return Fmt32{0x03020100u, 0x03020100u};
+  }
 }
 // unpack / pack of the four 4-byte formats
 __device__ __forceinline__ I4 unpack32(uint32_t raw, Fmt32 f) {
-  return I4{(raw >> f.sr) & 0xFFu, (raw >> 8) & 0xFFu, (raw >> f.sb) & 0xFFu,
-            f.has_a ? raw >> 24 : 255u};
+  const uint32_t w = __builtin_amdgcn_perm(raw, raw, f.to);
+  return I4{w & 0xFFu, (w >> 8) & 0xFFu, (w >> 16) & 0xFFu, w >> 24};
 }
 __device__ __forceinline__ uint32_t pack32(I4 v, Fmt32 f) {
-  const uint32_t a = f.has_a ? (v.a & 0xFFu) << 24 : 0u;
-  return ((v.r & 0xFFu) << f.sr) | ((v.g & 0xFFu) << 8) | ((v.b & 0xFFu) << f.sb) | a;
+  const uint32_t w =
+      (v.r & 0xFFu) | ((v.g & 0xFFu) << 8) | ((v.b & 0xFFu) << 16) | ((v.a & 0xFFu) << 24);
+  return __builtin_amdgcn_perm(w, w, f.from);
 }
 // Four consecutive pixels (n of them in the last quad of a row, the others
 // read as 0): 16 and 4 bytes at any pixel's address, one load each.
@@ -3198,7 +3204,7 @@ __global__ void __launch_bounds__(256) k_composite_quad(QuadJob J) {
 // source kind is a template parameter, and the dither thresholds, which
 // repeat every 64 columns, are read once per row and lane.  A 3840x2160
 // surface, radial gradient under blue noise: 153 us a launch in the general
-// kernel before, 52 now; 177 and 78 us a call.
+// kernel before, 48 now; 164 and 73 us a call.
 // ---------------------------------------------------------------------------
 constexpr uint32_t PAINT_COLOR = 3;  // KIND: a gradient type, or a color's dither
 
