@@ -207,6 +207,10 @@ struct z2d_gpu_ctx {
   hipEvent_t png_ev[2] = {nullptr, nullptr};
   float last_png_ms = 0.0f;   // device time of the last PNG encode
   uint8_t *comp_scratch = nullptr;  // this device's fixed composite scratch
+  // the painter calls' batch of one draw: its buffers and events stay from
+  // call to call (allocating them took half of a small call)
+  struct z2d_gpu_batch *painter = nullptr;
+  std::mutex painter_mu;
 };
 
 struct z2d_gpu_surface {
@@ -804,6 +808,7 @@ struct z2d_gpu_batch {
   uint32_t longest_first = 0;  // strip queue order of the single-launch render
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   bool render_timed = false;  // the last render recorded ev[1] before the tile render
+  bool timed = true;          // renders record their device time
   // The counters of the last render, copied to pinned memory at its end
   // (read after the stream completes: no extra synchronizing copy).
   HostBuf ctr_host;
@@ -1533,13 +1538,13 @@ static int32_t batch_render(z2d_gpu_batch *b, uint32_t mode) {
   HIP_OK(ctx, hipSetDevice(ctx->device));
   const hipStream_t st = bstream(b);
   for (int i = 0; i < 3; i++)
-    if (!b->ev[i]) HIP_OK(ctx, hipEventCreate(&b->ev[i]));
+    if (b->timed && !b->ev[i]) HIP_OK(ctx, hipEventCreate(&b->ev[i]));
   b->counted = b->view.count_stats != 0;
   if (!b->use_graph) {
-    HIP_OK(ctx, hipEventRecord(b->ev[0], st));
-    HIP_OK(ctx, batch_enqueue(b, mode, true));
-    HIP_OK(ctx, hipEventRecord(b->ev[2], st));
-    b->render_timed = true;
+    if (b->timed) HIP_OK(ctx, hipEventRecord(b->ev[0], st));
+    HIP_OK(ctx, batch_enqueue(b, mode, b->timed));
+    if (b->timed) HIP_OK(ctx, hipEventRecord(b->ev[2], st));
+    b->render_timed = b->timed;
     return Z2D_OK;
   }
   // graph replay: captured once per prepared batch, launch mode and counter
@@ -2093,6 +2098,8 @@ void z2d_gpu_destroy(z2d_gpu_ctx *ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  z2d_gpu_batch_destroy(ctx->painter);
+  ctx->painter = nullptr;
   ctx->comp_arena.release();
   ctx->comp_stage.release();
   ctx->png_work.release();
@@ -2345,25 +2352,45 @@ void z2d_gpu_batch_destroy(z2d_gpu_batch *b) {
   delete b;
 }
 
-// One painter call on a descriptor through a single-draw batch.
+// One painter call on a descriptor through a single-draw batch.  The context
+// keeps one: every call ends with the stream drained, so its buffers are free
+// again when it returns (a call that finds it in use by another thread makes
+// its own).  Buffers beyond kPainterKeep bytes are given back.
+constexpr size_t kPainterKeep = (size_t)64 << 20;
+
 static int32_t single_draw(z2d_gpu_ctx *ctx, z2d_surface_desc *surface,
                            int32_t (*add)(z2d_gpu_batch *, z2d_gpu_surface *, const void *),
                            const void *arg) {
   SurfRef ref;
   int32_t rc = surface_from_desc(ctx, surface, ref);
   if (rc) return rc;
-  z2d_gpu_batch b;
+  std::unique_lock<std::mutex> lk(ctx->painter_mu, std::try_to_lock);
+  z2d_gpu_batch own;
+  if (lk.owns_lock() && !ctx->painter) ctx->painter = new (std::nothrow) z2d_gpu_batch();
+  z2d_gpu_batch &b = lk.owns_lock() && ctx->painter ? *ctx->painter : own;
   b.ctx = ctx;
+  // prepare's uploads may stay in flight: the staging buffers are not touched
+  // again before the wait below
+  b.async_prepare = true;
+  b.timed = false;
   rc = add(&b, ref.s, arg);
   if (rc == Z2D_OK && !b.draws.empty()) {
     rc = batch_prepare(&b);
     if (rc == Z2D_OK) rc = batch_render(&b, 0);
-    if (rc == Z2D_OK) rc = batch_wait(&b);
+    if (rc == Z2D_OK)
+      rc = batch_wait(&b);
+    else
+      (void)hipStreamSynchronize(ctx->stream);  // uploads of a failed prepare
   }
-  b.arena.release();
-  b.stage.release();
-  for (int i = 0; i < 3; i++)
-    if (b.ev[i]) (void)hipEventDestroy(b.ev[i]);
+  batch_clear(&b);
+  if (b.arena.cap + b.stage.cap + b.flat_buf.cap + b.flat_stage.cap > kPainterKeep) {
+    b.arena.release();
+    b.stage.release();
+    b.flat_buf.release();
+    b.flat_stage.release();
+    b.raw_nodes.shrink_to_fit();
+    b.in_edges.shrink_to_fit();
+  }
   int32_t rc2 = surface_release(ctx, ref, rc == Z2D_OK);
   return rc ? rc : rc2;
 }
