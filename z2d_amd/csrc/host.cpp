@@ -1256,7 +1256,9 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
     h.d.band_lo = h.band_lo;
     h.d.band_hi = h.band_hi;
     h.d.entry_base = (uint32_t)std::min<uint64_t>(max_entries, 0xFFFFFFFFull);
-    for (uint32_t k = 0; k < h.d.node_cnt; k += EDGE_GROUP) egroups.push_back(make_uint2(i, k));
+    egroups.push_back(make_uint2(i, 0));  // (a draw without nodes is set up too)
+    for (uint32_t k = EDGE_GROUP; k < h.d.node_cnt; k += EDGE_GROUP)
+      egroups.push_back(make_uint2(i, k));
     max_entries += h.band_hi - h.band_lo + 1;
     max_strip_entries += (uint64_t)(h.band_hi - h.band_lo + 1) * spt *
                          (h.tcol_hi - h.tcol_lo + 1);
@@ -1304,6 +1306,7 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   const uint32_t scan_words = (uint32_t)(scan_n / SCAN_BLOCK + 2);
   const size_t o_scantmp = L.take((size_t)3 * scan_words * sizeof(uint64_t));
   const size_t o_drows = L.take((size_t)nd * sizeof(int2));
+  const size_t o_dacc = L.take((size_t)nd * sizeof(DrawAcc));
   const size_t o_entries = L.take(max_entries * sizeof(BandEntry));
   const size_t o_blist = L.take(max_entries * sizeof(uint4));
   const size_t o_ecnt = L.take((2 * max_entries + 1) * sizeof(uint32_t));  // + cursors
@@ -1417,6 +1420,7 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   J.edges = reinterpret_cast<z2d_edge *>(D + o_edges);
   J.draws = reinterpret_cast<DevDraw *>(D + o_draws);
   J.draw_rows = reinterpret_cast<int2 *>(D + o_drows);
+  J.draw_acc = reinterpret_cast<DrawAcc *>(D + o_dacc);
   J.n_draws = nd;
   J.surfaces = reinterpret_cast<DevSurface *>(D + o_surfs);
   J.n_surfaces = ns;
@@ -1476,8 +1480,8 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
   JobView &J = b->view;
   const uint32_t ns = J.n_surfaces;
   const hipStream_t st = bstream(b);
-  // every per-render reset: counters, the entries' edge counts and cursors,
-  // their column ranges (empty until the edge binning widens them) and the
+  // every per-render reset: counters, what the draws' edges add up, the
+  // entries' edge counts and cursors, their column ranges (empty until the edge binning widens them) and the
   // scans' look-back words; done by the flattening's per-node kernel when
   // there is one, else in a launch of their own
   FillSet F{};
@@ -1490,6 +1494,7 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
   };
   const uint32_t ctr_words = J.count_stats ? COUNTER_WORDS : 16;
   add(J.counters, ctr_words, 0u);
+  add(reinterpret_cast<uint32_t *>(J.draw_acc), (uint64_t)J.n_draws * (sizeof(DrawAcc) / 4), 0u);
   if (J.n_bands) {
     add(J.entry_ecnt, 2ull * J.max_entries + 1, 0u);
     add(reinterpret_cast<uint32_t *>(J.entry_xlo), J.max_entries, 0x7FFFFFFFu);

@@ -37,14 +37,25 @@ constexpr uint32_t STAT_SLOTS = 64;
 constexpr uint32_t STAT_WORDS = 16;
 enum : uint32_t { STAT_PIX = 0, STAT_EDGES = 2, STAT_ENTRIES = 3, STAT_UNPACKED = 4 };
 constexpr uint32_t COUNTER_WORDS = 16 + STAT_SLOTS * STAT_WORDS;
-// Edge slots of one draw per k_edge_bins work item.
+// Edge slots of one draw per work item of k_edge_build and k_edge_bins.
 constexpr uint32_t EDGE_GROUP = 64;
 
-// Flattened path node (move_to / line_to / close_path only; curves are
-// flattened on the host by the reference's Spline algorithm first).
+// Flattened path node (move_to / line_to / close_path only).  A close_path
+// holds the point its contour returns to, and whether an edge leads there
+// (`closes`): at least two lines of the contour move and its last point is
+// not its first.
 struct FNode {
   double x, y;
-  uint32_t tag, pad;
+  uint32_t tag, closes;
+};
+
+// What the edges of a draw of several edge groups leave for its set-up,
+// gathered by k_edge_build (zero at the start of a render).
+struct DrawAcc {
+  // extents (top, bottom, left, right) as the largest keys (f64_key;
+  // complemented for top and left)
+  unsigned long long key[4];
+  unsigned long long done;  // groups done << 32 | edges built
 };
 
 // Bézier flattening on the device (k_flatten): one job per fill draw.
@@ -115,7 +126,7 @@ enum DrawMode : uint32_t { MODE_DIRECT = 0, MODE_MSAA = 1, MODE_SSAA = 2 };
 
 struct DevDraw {
   // inputs
-  uint32_t node_off, node_cnt;  // flattened nodes; edge slots use the same range
+  uint32_t node_off, node_cnt;  // flattened nodes; their edge slots use the same range
   uint32_t surface;
   uint32_t mode;       // DrawMode (alpha1 targets already forced to direct)
   uint32_t rule, op;
@@ -128,7 +139,7 @@ struct DevDraw {
   // the draw's entries: entry_base + (band - band_lo)
   uint32_t band_lo, band_hi, entry_base;
   // written by k_edge_build
-  uint32_t edge_cnt;
+  uint32_t edge_cnt;  // edge slots; a slot without an edge has y0 == y1 == 0
   uint32_t flags;
   double ext[4];  // top, bottom, left, right (scaled space)
   int32_t rx0, ry0, rx1, ry1;  // composite region [rx0,rx1) x [ry0,ry1)
@@ -209,8 +220,9 @@ struct TileRef {
 struct JobView {
   const FNode *nodes;
   const z2d_edge *in_edges;  // edges of polygon draws
-  z2d_edge *edges;  // edge slots, indexed like nodes
+  z2d_edge *edges;  // edge slots of flattened draws, indexed like nodes
   DevDraw *draws;
+  DrawAcc *draw_acc;
   int2 *draw_rows;  // per draw: composite rows [y0, y1), empty when not visible
   uint32_t n_draws;
   DevSurface *surfaces;
@@ -243,7 +255,8 @@ struct JobView {
   uint32_t *entry_cur;       // max_entries: fill cursors (follows entry_ecnt)
   int32_t *entry_xlo;        // max_entries: sample-column range of the entry's edges
   int32_t *entry_xhi;
-  const uint2 *egroups;      // edge-binning work: draw, first edge slot
+  // edge work: draw, first edge slot (at least one item per draw)
+  const uint2 *egroups;
   uint32_t n_egroups;
   REdge *entry_edges;        // the edges of each entry's list, capacity max_entry_edges
   uint32_t max_entry_edges;
@@ -342,12 +355,12 @@ struct PaintJob {
   const uint16_t *blue_noise;
 };
 
-// Up to six word fills in one launch (the zeroing at the start of a render
+// Up to eight word fills in one launch (the zeroing at the start of a render
 // pipeline): fill f writes v[f] to n[f] words at p[f].
 struct FillSet {
-  uint32_t *p[6];
-  uint64_t n[6];
-  uint32_t v[6];
+  uint32_t *p[8];
+  uint64_t n[8];
+  uint32_t v[8];
   uint32_t count;
 };
 

@@ -4,7 +4,8 @@
 //   k_edge_build  flattened nodes -> Polygon edges + extents + draw setup
 //                 (fill_plotter.plot, Polygon.addEdge/inBox and the raster
 //                 entry logic of src/internal/raster/{direct,multisample,
-//                 supersample}.zig)
+//                 supersample}.zig), and the edges counted per (draw, band)
+//                 entry
 //   k_rowprog     serial row emulation, only for draws whose coverage depends
 //                 on the reference's sort order (unbalanced contours) or whose
 //                 direct-mode unbounded clears depend on whole rows
@@ -202,6 +203,13 @@ __device__ __forceinline__ int32_t wave_max_scan(int32_t v) {
       : "+v"(v));
   return v;
 }
+// Orders this wave's LDS accesses before and after the call (lanes of one
+// wave exchanging data through LDS).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // A lane's value read by every lane (src wave-uniform).
 __device__ __forceinline__ uint32_t lane_u32(uint32_t v, uint32_t src) {
   return __builtin_amdgcn_readlane(v, src);
@@ -255,105 +263,14 @@ __device__ __forceinline__ double wave_fmax_f64(double v) {
   return fmax(fmax(lane_f64(v, 15), lane_f64(v, 31)), fmax(lane_f64(v, 47), lane_f64(v, 63)));
 }
 
-// fill_plotter.plot (src/internal/tess/fill_plotter.zig:21-97) with the
-// PointBuffer(1, 3) of src/internal/tess/point_buffer.zig, one lane per
-// node.  Only the buffer's first point, last point and fill count (capped
-// at 3) are ever read.  The last point before a node is the previous node's
-// point when that node is a move or a line (a line to an equal point leaves
-// it equal); the host sends draws with a line right after a close to the
-// serial form below.  A line emits when it moves; a close emits when it
-// starts a run of closes, at least two lines moved since the subpath's
-// move, and the last point is not the first.  Edge slots are a wave scan of
-// the emit flags; the extents are the running min/max, with the first edge
-// seeding them as in Polygon.addEdge (a NaN there sticks).
-__device__ void plot_parallel(const FNode *nodes, uint32_t n, double scale, z2d_edge *out,
-                              ExtAcc &acc) {
-  const uint32_t lane = threadIdx.x & 63;
-  const double inf = __builtin_huge_val();
-  double c_fx = 0.0, c_fy = 0.0, c_px = 0.0, c_py = 0.0;
-  uint32_t c_ptag = 0xFFFFFFFFu;
-  bool c_have = false;
-  int32_t c_cnt = 0;
-  uint32_t ebase = 0;
-  double m_top = inf, m_bot = -inf, m_left = inf, m_right = -inf;
-  double f_top = 0.0, f_bot = 0.0, f_left = 0.0, f_right = 0.0;
-  for (uint32_t base = 0; base < n; base += 64) {
-    const uint32_t k = base + lane;
-    FNode nd{0.0, 0.0, 0xFFFFFFFFu, 0u};
-    if (k < n) nd = nodes[k];
-    uint32_t tag = nd.tag;
-    if (tag == Z2D_NODE_MOVE_TO && k == n - 1) tag = 0xFFFFFFFFu;  // a final move is ignored
-    const double px = lane_prev_f64(nd.x, c_px), py = lane_prev_f64(nd.y, c_py);
-    const uint32_t ptag = lane_prev_u32(tag, c_ptag);
-    const int32_t head = wave_max_scan(tag == Z2D_NODE_MOVE_TO ? (int32_t)lane : -1);
-    const int32_t hsrc = head >= 0 ? head : 0;
-    const double hx = __shfl(nd.x, hsrc, 64), hy = __shfl(nd.y, hsrc, 64);
-    const double fx = head >= 0 ? hx : c_fx, fy = head >= 0 ? hy : c_fy;
-    const bool have = head >= 0 || c_have;
-    const bool line_moves = tag == Z2D_NODE_LINE_TO && have && !pt_eq(px, py, nd.x, nd.y);
-    const int32_t a = line_moves ? 1 : 0;
-    const int32_t ps = wave_incl_scan(a);
-    const int32_t ps_head = __shfl(ps, hsrc, 64);
-    const int32_t cnt_before = head >= 0 ? ps - a - ps_head : c_cnt + ps - a;
-    const bool close_emits = tag == Z2D_NODE_CLOSE_PATH && have &&
-                             ptag != Z2D_NODE_CLOSE_PATH && cnt_before >= 2 &&
-                             !pt_eq(px, py, fx, fy);
-    const double tx = line_moves ? nd.x : fx, ty = line_moves ? nd.y : fy;
-    // Polygon.addEdge (src/internal/tess/Polygon.zig:61-109)
-    const double ax = px * scale, ay = py * scale, bx = tx * scale, by = ty * scale;
-    const bool emit = (line_moves || close_emits) && (ay < by || ay > by);
-    const uint64_t m = __ballot(emit);
-    double top = 0.0, bot = 0.0, left = 0.0, right = 0.0;
-    if (emit) {
-      z2d_edge e;
-      e.y0 = ay;
-      e.y1 = by;
-      if (ay < by) {
-        e.x_start = ax;
-        e.x_inc = (bx - ax) / (by - ay);
-      } else {
-        e.x_start = bx;
-        e.x_inc = (ax - bx) / (ay - by);
-      }
-      top = e.y0 < e.y1 ? e.y0 : e.y1;
-      bot = e.y0 < e.y1 ? e.y1 : e.y0;
-      left = ax < bx ? ax : bx;
-      right = ax < bx ? bx : ax;
-      out[ebase + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = e;
-      m_top = fmin(m_top, top);
-      m_bot = fmax(m_bot, bot);
-      m_left = fmin(m_left, left);
-      m_right = fmax(m_right, right);
-    }
-    if (ebase == 0 && m != 0) {
-      const int fl = __ffsll((unsigned long long)m) - 1;
-      f_top = lane_f64(top, (uint32_t)fl);
-      f_bot = lane_f64(bot, (uint32_t)fl);
-      f_left = lane_f64(left, (uint32_t)fl);
-      f_right = lane_f64(right, (uint32_t)fl);
-    }
-    ebase += (uint32_t)__popcll(m);
-    c_px = lane_f64(nd.x, 63);
-    c_py = lane_f64(nd.y, 63);
-    c_ptag = lane_u32(tag, 63);
-    c_fx = lane_f64(fx, 63);
-    c_fy = lane_f64(fy, 63);
-    c_have = lane_u32(have ? 1u : 0u, 63) != 0;
-    c_cnt = (int32_t)lane_u32((uint32_t)(cnt_before + a), 63);
-  }
-  m_top = wave_fmin_f64(m_top);
-  m_bot = wave_fmax_f64(m_bot);
-  m_left = wave_fmin_f64(m_left);
-  m_right = wave_fmax_f64(m_right);
-  acc.n = ebase;
-  if (ebase) {
-    acc.top = f_top != f_top ? f_top : m_top;
-    acc.bottom = f_bot != f_bot ? f_bot : m_bot;
-    acc.left = f_left != f_left ? f_left : m_left;
-    acc.right = f_right != f_right ? f_right : m_right;
-  } else {
-    acc.top = acc.bottom = acc.left = acc.right = 0.0;
-  }
+// A double as an unsigned key in the same order (never 0 for a number), and
+// back.
+__device__ __forceinline__ unsigned long long f64_key(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  return (u >> 63) ? ~u : (u | (1ull << 63));
+}
+__device__ __forceinline__ double key_f64(unsigned long long k) {
+  return __longlong_as_double((long long)((k >> 63) ? (k & ~(1ull << 63)) : ~k));
 }
 
 // The fast renderer's paint class of a paint (FAST_PAINT_NONE: the general
@@ -429,65 +346,16 @@ __device__ __forceinline__ uint32_t *stat_slot(const JobView &J, uint32_t i) {
   return J.counters + 16 + (i % STAT_SLOTS) * STAT_WORDS;
 }
 
-__global__ void __launch_bounds__(256) k_edge_build(JobView J) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t d = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (d >= J.n_draws) return;
+// The set-up of draw d once its edges are built (one lane): the raster entry
+// logic, visibility, draw window and composite region, and the fast
+// renderer's block.
+__device__ void draw_setup(const JobView &J, uint32_t d, uint32_t flags, const ExtAcc &acc) {
   DevDraw &D = J.draws[d];
   const DevSurface S = J.surfaces[D.surface];
   const double scale = D.mode == MODE_DIRECT ? 1.0 : 4.0;
-  z2d_edge *out = J.edges + D.node_off;
-  uint32_t flags = D.flags & (DRAW_UNBALANCED | DRAW_ROWPROG | DRAW_SERIAL_PLOT);
-  ExtAcc acc{0, 0.0, 0.0, 0.0, 0.0};
-  if (D.input_edges) {
-    for (uint32_t k = lane; k < D.node_cnt; k += 64) out[k] = J.in_edges[D.in_edge_off + k];
-    acc.n = D.node_cnt;
-    acc.top = D.in_ext[0]; acc.bottom = D.in_ext[1];
-    acc.left = D.in_ext[2]; acc.right = D.in_ext[3];
-  } else if (!(flags & DRAW_SERIAL_PLOT)) {
-    plot_parallel(J.nodes + D.node_off, D.node_cnt, scale, out, acc);
-  }
-  // a solid paint's coverage table, for the fast renderer should the draw
-  // be one (lane k: entry k)
-  if (J.fast && lane <= 16 && J.paints[D.paint].kind == Z2D_PATTERN_OPAQUE)
-    J.fast[d].srctab[lane] = fast_srctab_entry(J.paints[D.paint], lane);
-  if (lane != 0) return;
   J.draw_rows[d] = make_int2(0, 0);  // not visible unless set below
-  if (!D.input_edges && (flags & DRAW_SERIAL_PLOT)) {
-    // The same state machine node by node (a line may follow a close).
-    double fx = 0.0, fy = 0.0, lx = 0.0, ly = 0.0;
-    int len = 0;
-    const FNode *nodes = J.nodes + D.node_off;
-    const uint32_t n = D.node_cnt;
-    for (uint32_t i = 0; i < n; i++) {
-      const FNode nd = nodes[i];
-      if (nd.tag == Z2D_NODE_MOVE_TO) {
-        if (i == n - 1) break;
-        fx = lx = nd.x;
-        fy = ly = nd.y;
-        len = 1;
-      } else if (nd.tag == Z2D_NODE_LINE_TO) {
-        if (len == 0) continue;  // InvalidState is rejected on the host
-        if (!pt_eq(lx, ly, nd.x, nd.y)) {
-          add_edge(out, acc, scale, lx, ly, nd.x, nd.y);
-          lx = nd.x;
-          ly = nd.y;
-          if (len < 3) len++;
-        }
-      } else if (nd.tag == Z2D_NODE_CLOSE_PATH) {
-        if (len >= 3 && !pt_eq(lx, ly, fx, fy)) {
-          add_edge(out, acc, scale, lx, ly, fx, fy);
-          lx = fx;
-          ly = fy;
-        }
-      }
-    }
-  }
-  D.edge_cnt = acc.n;
-  if (J.count_stats && acc.n) atomicAdd(&stat_slot(J, d)[STAT_EDGES], acc.n);
   D.ext[0] = acc.top; D.ext[1] = acc.bottom; D.ext[2] = acc.left; D.ext[3] = acc.right;
 
-  // Raster entry logic: visibility, draw window and composite region.
   const int32_t W = S.w, H = S.h;
   const bool bounded = op_is_bounded(D.op);
   if (!bounded) flags |= DRAW_UNBOUNDED;
@@ -571,6 +439,12 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
   }
 }
 
+// A draw's edge slots: built by k_edge_build, or the caller's edges where they
+// are.
+__device__ __forceinline__ const z2d_edge *draw_edges(const JobView &J, const DevDraw &D) {
+  return D.input_edges ? J.in_edges + D.in_edge_off : J.edges + D.node_off;
+}
+
 // ---------------------------------------------------------------------------
 // k_rowprog: the reference's serial scanline loop for one draw per thread
 // (WorkingEdgeSet rescan/inc/sort/filter, src/internal/tess/Polygon.zig:
@@ -588,8 +462,11 @@ __global__ void k_rowprog(JobView J, const uint32_t *draw_list, uint32_t n_list,
   const DevSurface S = J.surfaces[D.surface];
   z2d_edge *E = scratch_edges + scratch_off[i];
   int32_t *X = scratch_x + scratch_off[i];
-  const uint32_t n_all = D.edge_cnt;
-  for (uint32_t k = 0; k < n_all; k++) E[k] = J.edges[D.node_off + k];
+  uint32_t n_all = 0;
+  for (uint32_t k = 0; k < D.edge_cnt; k++) {
+    const z2d_edge e = draw_edges(J, D)[k];
+    if (D.input_edges || e.y0 != e.y1) E[n_all++] = e;  // (not a slot without an edge)
+  }
   RowRec *R = J.rows + D.row_off;
   const bool direct_unbounded = D.mode == MODE_DIRECT && (D.flags & DRAW_UNBOUNDED);
   const int32_t W = S.w;
@@ -811,8 +688,8 @@ struct DevFlattener {
     box[2] = fmin(box[2], p.y);
     box[3] = fmax(box[3], p.y);
   }
-  __device__ void emit(uint32_t tag, FPt p) {
-    if (EMIT) out[n] = FNode{p.x, p.y, tag, 0u};
+  __device__ void emit(uint32_t tag, FPt p, bool closes = false) {
+    if (EMIT) out[n] = FNode{p.x, p.y, tag, closes ? 1u : 0u};
     n++;
     // the (edge, band) bound over the emitted stream, as the host computes it
     if (tag == Z2D_NODE_MOVE_TO) {
@@ -885,8 +762,9 @@ __global__ void k_flatten_serial(const z2d_path_node *__restrict__ raw,
       f.track(c);
       f.curve(b, c, d, J.tol_sq);
     } else {  // close
-      f.emit(Z2D_NODE_CLOSE_PATH, FPt{0.0, 0.0});
-      if (f.len >= 3 && !fpeq(f.buf[f.len - 1], f.buf[0])) f.add(f.buf[0]);
+      const bool closes = f.len >= 3 && !fpeq(f.buf[f.len - 1], f.buf[0]);
+      f.emit(Z2D_NODE_CLOSE_PATH, f.len ? f.buf[0] : FPt{0.0, 0.0}, closes);
+      if (closes) f.add(f.buf[0]);
     }
   }
   if (f.len > 0 && !fpeq(f.buf[f.len - 1], f.buf[0])) balanced = false;
@@ -1017,8 +895,9 @@ __global__ void __launch_bounds__(256) k_flatten_wave(const z2d_path_node *__res
       box[2] = fmin(box[2], r.box[2]);
       box[3] = fmax(box[3], r.box[3]);
     } else if (EMIT && act && tag != Z2D_NODE_CURVE_TO) {
-      o[rl[i]] = FNode{tag == Z2D_NODE_CLOSE_PATH ? 0.0 : p.x,
-                       tag == Z2D_NODE_CLOSE_PATH ? 0.0 : p.y, tag, 0u};
+      // (a close of a draw kept here comes after two lines that move)
+      const bool close = tag == Z2D_NODE_CLOSE_PATH;
+      o[rl[i]] = FNode{close ? mv.x : p.x, close ? mv.y : p.y, tag, close ? 1u : 0u};
     }
     c_cur += (uint32_t)__popcll(cm);
     if (!EMIT) {
@@ -1632,19 +1511,231 @@ __device__ __forceinline__ double redge_x(double top, double x_start, double x_i
 }
 
 // ---------------------------------------------------------------------------
+// k_edge_build: the edges of a draw, 64 node slots per wave (slot k: the edge
+// that node k adds, if any), their extents, and their number per (draw, band)
+// entry.  fill_plotter.plot (src/internal/tess/fill_plotter.zig:21-97) with
+// the PointBuffer(1, 3) of src/internal/tess/point_buffer.zig asks of the
+// nodes before a line or close only its predecessor's point, and of a close
+// what the flattening left in it (FNode), so every slot is on its own; draws
+// in which a line follows a close go node by node in their first wave.
+// The wave that completes a draw sets it up (draw_setup).
+// Bound by latency: one wave per draw before, which took a chunk of 64 nodes
+// after the other (57 us for 101 draws of a page of text, 19 us for the 61
+// of a small frame, and 13.5 and 5.5 us more in a pass of its own for the
+// counting); 20 and 14 us now, of memory latency and of the last wave's set-up.
+// ---------------------------------------------------------------------------
+// The bands [lo, hi] of `rows` sample rows, among [rb_lo, rb_hi], that an edge
+// meets: top < b's last sample row + 0.5 and bot >= its first + 0.5 (the
+// active-edge test over the band; lo > hi: none).  Both hold over a range of
+// bands; floor estimates, wider by one, are corrected with the exact
+// comparisons.
+__device__ __forceinline__ void edge_bands(double top, double bot, int32_t rows, int32_t rb_lo,
+                                           int32_t rb_hi, int32_t &lo, int32_t &hi) {
+  const double flo = fmax(floor(top / (double)rows) - 1.0, (double)rb_lo);
+  const double fhi = fmin(floor(bot / (double)rows) + 1.0, (double)rb_hi);
+  lo = INT32_MAX;
+  hi = INT32_MIN;
+  if (!(flo <= fhi)) return;
+  int32_t l = (int32_t)flo, h = (int32_t)fhi;
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    if (!(top < (double)((l + 1) * rows - 1) + 0.5)) l++;
+    if (!(bot >= (double)(h * rows) + 0.5)) h--;
+  }
+  if (l > h) return;
+  lo = l;
+  hi = h;
+}
+// A wave's edges against the bands [ulo, uhi]: edge by edge, a lane per band,
+// where that is fewer steps (a rectangle's two edges down a whole surface)
+// than band by band, a lane per edge.
+__device__ __forceinline__ bool by_edge(uint64_t edges, int32_t ulo, int32_t uhi) {
+  const int32_t n = uhi - ulo + 1;
+  return (int32_t)__popcll(edges) * ((n + 63) >> 6) < n;
+}
+
+__global__ void __launch_bounds__(256) k_edge_build(JobView J) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t g = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (g >= J.n_egroups) return;
+  const uint2 it = J.egroups[g];  // draw, first slot
+  const uint32_t d = it.x;
+  DevDraw &D = J.draws[d];
+  uint32_t flags = D.flags & (DRAW_UNBALANCED | DRAW_ROWPROG | DRAW_SERIAL_PLOT);
+  const uint32_t n = D.node_cnt, input = D.input_edges;
+  const bool serial = !input && (flags & DRAW_SERIAL_PLOT);
+  if (serial && it.y != 0) return;
+  // groups that the set-up waits for (given edges come with their extents)
+  const uint32_t n_groups = serial || input || n == 0 ? 1u : (n + EDGE_GROUP - 1) / EDGE_GROUP;
+  const bool direct = D.mode == MODE_DIRECT;
+  const double scale = direct ? 1.0 : 4.0;
+  const int32_t band_rows = (int32_t)J.band_h * (direct ? 1 : 4);
+  z2d_edge *const out = J.edges + D.node_off;
+  DrawAcc &A = J.draw_acc[d];
+  // a solid paint's coverage table, for the fast renderer should the draw be
+  // one (lane k: entry k)
+  if (it.y == 0 && J.fast && lane <= 16 && J.paints[D.paint].kind == Z2D_PATTERN_OPAQUE)
+    J.fast[d].srctab[lane] = fast_srctab_entry(J.paints[D.paint], lane);
+
+  ExtAcc acc{0, 0.0, 0.0, 0.0, 0.0};
+  uint32_t first = it.y, end = min(it.y + EDGE_GROUP, n);  // the slots counted below
+  if (serial) {
+    // the plotter's state machine node by node (a line may follow a close)
+    if (lane == 0) {
+      double fx = 0.0, fy = 0.0, lx = 0.0, ly = 0.0;
+      int len = 0;
+      const FNode *nodes = J.nodes + D.node_off;
+      for (uint32_t i = 0; i < n; i++) {
+        const FNode nd = nodes[i];
+        if (nd.tag == Z2D_NODE_MOVE_TO) {
+          if (i == n - 1) break;
+          fx = lx = nd.x;
+          fy = ly = nd.y;
+          len = 1;
+        } else if (nd.tag == Z2D_NODE_LINE_TO) {
+          if (len == 0) continue;  // InvalidState is rejected on the host
+          if (!pt_eq(lx, ly, nd.x, nd.y)) {
+            add_edge(out, acc, scale, lx, ly, nd.x, nd.y);
+            lx = nd.x;
+            ly = nd.y;
+            if (len < 3) len++;
+          }
+        } else if (nd.tag == Z2D_NODE_CLOSE_PATH) {
+          if (len >= 3 && !pt_eq(lx, ly, fx, fy)) {
+            add_edge(out, acc, scale, lx, ly, fx, fy);
+            lx = fx;
+            ly = fy;
+          }
+        }
+      }
+    }
+    __threadfence_block();  // lane 0's edges, read below by the others
+    first = 0;
+    end = lane_u32(acc.n, 0);
+  }
+  for (uint32_t k0 = first; k0 < end; k0 += 64) {
+    const uint32_t k = k0 + lane;
+    const bool slot = k < end;
+    z2d_edge ed{0.0, 0.0, 0.0, 0.0};
+    bool emit = false;
+    if (serial) {
+      if (slot) ed = out[k];
+      emit = slot;
+    } else if (input) {
+      if (slot) ed = J.in_edges[D.in_edge_off + k];
+      emit = slot;
+    } else {
+      const FNode *nodes = J.nodes + D.node_off;
+      FNode nd{0.0, 0.0, 0xFFFFFFFFu, 0u}, pv{0.0, 0.0, 0xFFFFFFFFu, 0u};
+      if (slot) nd = nodes[k];
+      if (lane == 0 && k0 > 0) pv = nodes[k0 - 1];
+      const double px = lane_prev_f64(nd.x, pv.x), py = lane_prev_f64(nd.y, pv.y);
+      const uint32_t ptag = lane_prev_u32(nd.tag, pv.tag);
+      // (a line or close before the first move is rejected on the host)
+      const bool moves = !pt_eq(px, py, nd.x, nd.y);
+      const double ax = px * scale, ay = py * scale, bx = nd.x * scale, by = nd.y * scale;
+      emit = slot && k > 0 && moves && (ay < by || ay > by) &&
+             (nd.tag == Z2D_NODE_LINE_TO ||
+              (nd.tag == Z2D_NODE_CLOSE_PATH && nd.closes && ptag != Z2D_NODE_CLOSE_PATH));
+      double top = 0.0, bot = 0.0, left = 0.0, right = 0.0;
+      if (emit) {  // Polygon.addEdge (src/internal/tess/Polygon.zig:61-109)
+        ed.y0 = ay;
+        ed.y1 = by;
+        if (ay < by) {
+          ed.x_start = ax;
+          ed.x_inc = (bx - ax) / (by - ay);
+        } else {
+          ed.x_start = bx;
+          ed.x_inc = (ax - bx) / (ay - by);
+        }
+        top = ay < by ? ay : by;
+        bot = ay < by ? by : ay;
+        left = ax < bx ? ax : bx;
+        right = ax < bx ? bx : ax;
+      }
+      if (slot) out[k] = ed;
+      const uint64_t m = __ballot(emit);
+      if (m) {
+        const double inf = __builtin_huge_val();
+        acc.n = (uint32_t)__popcll(m);
+        acc.top = wave_fmin_f64(emit ? top : inf);
+        acc.bottom = wave_fmax_f64(emit ? bot : -inf);
+        acc.left = wave_fmin_f64(emit ? left : inf);
+        acc.right = wave_fmax_f64(emit ? right : -inf);
+        if (n_groups > 1 && lane < 4) {
+          const double v = lane == 0 ? acc.top : lane == 1 ? acc.bottom : lane == 2 ? acc.left : acc.right;
+          atomicMax(&A.key[lane], lane & 1u ? f64_key(v) : ~f64_key(v));
+        }
+      }
+    }
+    // the edges counted per band of the draw's entries
+    const double top = ed.y0 < ed.y1 ? ed.y0 : ed.y1, bot = ed.y0 < ed.y1 ? ed.y1 : ed.y0;
+    int32_t lo = INT32_MAX, hi = INT32_MIN;
+    if (emit) edge_bands(top, bot, band_rows, (int32_t)D.band_lo, (int32_t)D.band_hi, lo, hi);
+    const int32_t ulo = wave_min_i32(lo), uhi = wave_max_i32(hi);
+    const uint64_t em = __ballot(lo <= hi);
+    const bool transposed = by_edge(em, ulo, uhi);
+    for (int32_t w = ulo; w <= uhi; w += 64) {
+      const int32_t bj = w + (int32_t)lane;  // this lane's band
+      uint32_t cnt = 0;
+      if (transposed) {
+        for (uint64_t r = em; r; r &= r - 1) {
+          const uint32_t e = (uint32_t)__builtin_ctzll(r);
+          const int32_t l = (int32_t)lane_u32((uint32_t)lo, e), h = (int32_t)lane_u32((uint32_t)hi, e);
+          cnt += (l <= bj && bj <= h) ? 1u : 0u;
+        }
+      } else {
+        const int32_t wend = min(uhi, w + 63);
+        for (int32_t bnd = w; bnd <= wend; bnd++) {
+          const uint32_t c = (uint32_t)__popcll(__ballot(lo <= bnd && bnd <= hi));
+          if (bj == bnd) cnt = c;
+        }
+      }
+      if (cnt) atomicAdd(&J.entry_ecnt[D.entry_base + ((uint32_t)bj - D.band_lo)], cnt);
+    }
+  }
+  if (n_groups > 1) {
+    // the draw's last group sets it up: this wave's maxima have been made
+    // (waited for) when it counts itself done, and they and the reads below
+    // are atomics at device scope, so the last group reads every group's
+    // without a fence (whose write-back of the L2 took 36 ns a group)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    unsigned long long done = 0;
+    if (lane == 0) done = atomicAdd(&A.done, (1ull << 32) | acc.n) + ((1ull << 32) | acc.n);
+    if (lane != 0 || (uint32_t)(done >> 32) != n_groups) return;
+    acc.n = (uint32_t)done;
+    double v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const unsigned long long k =
+          __hip_atomic_load(&A.key[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      v[i] = key_f64(i & 1 ? k : ~k);
+    }
+    if (acc.n) acc = ExtAcc{acc.n, v[0], v[1], v[2], v[3]};
+  }
+  if (lane != 0 || (input && it.y != 0)) return;
+  if (input) acc = ExtAcc{n, D.in_ext[0], D.in_ext[1], D.in_ext[2], D.in_ext[3]};
+  D.edge_cnt = serial ? acc.n : n;
+  if (J.count_stats && acc.n) atomicAdd(&stat_slot(J, d)[STAT_EDGES], acc.n);
+  draw_setup(J, d, flags, acc);
+}
+
+// ---------------------------------------------------------------------------
 // k_edge_bins: per (draw, band) entry, copies of the draw's edges whose
 // y-range meets the band's sample rows (top < last mid && bottom >= first mid,
 // the active-edge test of src/internal/raster/multisample.zig and direct.zig
 // taken over the band); strips then walk only those edges.  One wave per
-// group of EDGE_GROUP edge slots of a draw: each chunk of 64 edges is tested
-// against the bands it can meet.  FILL=false counts per entry (atomics on
-// the zeroed entry_ecnt); FILL=true, after the scan, appends to the entry's
-// list through the entry_cur cursors (the order inside a list is free: the
-// winding deltas of the edges are summed).
+// group of EDGE_GROUP edge slots of a draw, after the scan of k_edge_build's
+// counts, appending to the entries' lists through the entry_cur cursors (the
+// order inside a list is free: the winding deltas of the edges are summed).
+// Bound by latency where few edges meet many bands: a band after the other
+// was 0.43 us each for a background rectangle's two edges, 58 us of the 61 us
+// that a 2160-row page took; with a lane per band instead (by_edge) it takes 20,
+// a small frame of 38 bands 9 instead of 17.
 // ---------------------------------------------------------------------------
-template <bool FILL>
-__global__ void k_edge_bins(JobView J) {
-  const uint32_t lane = threadIdx.x & 63;
+__global__ void __launch_bounds__(256) k_edge_bins(JobView J) {
+  __shared__ int32_t s_x[4][2][64];  // per wave: a window's bands' column ranges
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t g = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (g >= J.n_egroups) return;
   const uint2 it = J.egroups[g];  // draw, first edge slot
@@ -1654,91 +1745,108 @@ __global__ void k_edge_bins(JobView J) {
   if (rows.x >= rows.y) return;  // no entries
   const uint32_t ne = D.edge_cnt;
   if (it.y >= ne) return;
-  const uint32_t kend = min(it.y + EDGE_GROUP, ne);
-  const int SC = D.mode == MODE_DIRECT ? 1 : 4;
   const int32_t bh = (int32_t)J.band_h;
-  const int32_t rb_lo = rows.x / bh, rb_hi = (rows.y - 1) / bh;  // entry bands
-  const uint32_t blo = D.band_lo, bhi = D.band_hi, ebase = D.entry_base;
-  const double band_rows = (double)(bh * SC);
-  const z2d_edge *edges = J.edges + D.node_off;
-  const uint64_t below = (1ull << lane) - 1ull;
-  for (uint32_t k0 = it.y; k0 < kend; k0 += 64) {
-    const bool valid = k0 + lane < kend;
-    z2d_edge ed{0.0, 0.0, 0.0, 0.0};
-    double top = 0.0, bot = 0.0;
-    int32_t lo = INT32_MAX, hi = INT32_MIN;  // candidate bands, widened by one
-    int32_t xlo = INT32_MAX, xhi = INT32_MIN;  // the edge's sample columns (fill pass)
-    if (valid) {
-      ed = edges[k0 + lane];
-      top = ed.y0 < ed.y1 ? ed.y0 : ed.y1;
-      bot = ed.y0 < ed.y1 ? ed.y1 : ed.y0;
-      if (FILL) {
-        const double xb = ed.x_start + ed.x_inc * (bot - top);
-        const double a = fmin(ed.x_start, xb), c = fmax(ed.x_start, xb);
-        if (a >= -2.0e9 && c <= 2.0e9) {
-          xlo = (int32_t)floor(a);
-          xhi = (int32_t)floor(c);
-        } else {  // huge or non-finite: the whole row
-          xlo = INT32_MIN;
-          xhi = INT32_MAX;
-        }
-      }
-      const double flo = fmax(floor(top / band_rows) - 1.0, (double)rb_lo);
-      const double fhi = fmin(floor(bot / band_rows) + 1.0, (double)rb_hi);
-      if (flo <= fhi) {  // (a NaN edge fails the exact test below)
-        lo = (int32_t)flo;
-        hi = (int32_t)fhi;
-      }
+  const int32_t band_rows = bh * (D.mode == MODE_DIRECT ? 1 : 4);
+  const int32_t blo = (int32_t)D.band_lo, bhi = (int32_t)D.band_hi;
+  const uint32_t ebase = D.entry_base;
+  const uint32_t k = it.y + lane;
+  z2d_edge ed{0.0, 0.0, 0.0, 0.0};
+  double top = 0.0, bot = 0.0;
+  int32_t lo = INT32_MAX, hi = INT32_MIN;  // candidate bands among the entries'
+  int32_t xlo = INT32_MAX, xhi = INT32_MIN;  // the edge's sample columns
+  if (k < min(it.y + EDGE_GROUP, ne)) {
+    ed = draw_edges(J, D)[k];
+    top = ed.y0 < ed.y1 ? ed.y0 : ed.y1;
+    bot = ed.y0 < ed.y1 ? ed.y1 : ed.y0;
+    const double xb = ed.x_start + ed.x_inc * (bot - top);
+    const double a = fmin(ed.x_start, xb), c = fmax(ed.x_start, xb);
+    if (a >= -2.0e9 && c <= 2.0e9) {
+      xlo = (int32_t)floor(a);
+      xhi = (int32_t)floor(c);
+    } else {  // huge or non-finite: the whole row
+      xlo = INT32_MIN;
+      xhi = INT32_MAX;
     }
-    const REdge red = make_redge(ed);  // the copy every band of the edge receives
-    const int32_t ulo = wave_min_i32(lo), uhi = wave_max_i32(hi);
-    // bands in windows of 64: lane j holds the count (then the list
-    // position) of band w + j, so each window takes one vector atomic
-    for (int32_t w = ulo; w <= uhi; w += 64) {
-      const int32_t wend = min(uhi, w + 63);
-      uint32_t cnt = 0;
-      for (int32_t bnd = w; bnd <= wend; bnd++) {
-        const int32_t y0 = bnd * bh;
-        const double ys_lo = (double)(y0 * SC) + 0.5;
-        const double ys_hi = (double)((y0 + bh) * SC - 1) + 0.5;
-        const bool hit = lo <= bnd && bnd <= hi && top < ys_hi && bot >= ys_lo;
-        const uint32_t n = (uint32_t)__popcll(__ballot(hit));
-        if ((int32_t)lane == bnd - w) cnt = n;
-      }
-      const int32_t bj = w + (int32_t)lane;  // this lane's band
-      const bool has = cnt != 0 && bj <= wend && (uint32_t)bj >= blo && (uint32_t)bj <= bhi;
-      const uint32_t idx = has ? ebase + ((uint32_t)bj - blo) : 0u;
-      if (!FILL) {
-        if (has) atomicAdd(&J.entry_ecnt[idx], cnt);
-        continue;
-      }
-      const uint32_t at = has ? J.entry_ecnt[idx] + atomicAdd(&J.entry_cur[idx], cnt) : 0u;
-      for (int32_t bnd = w; bnd <= wend; bnd++) {
-        if ((uint32_t)bnd < blo || (uint32_t)bnd > bhi) continue;
-        const int32_t y0 = bnd * bh;
-        const double ys_lo = (double)(y0 * SC) + 0.5;
-        const double ys_hi = (double)((y0 + bh) * SC - 1) + 0.5;
-        const bool hit = lo <= bnd && bnd <= hi && top < ys_hi && bot >= ys_lo;
-        const uint64_t m = __ballot(hit);
-        if (m == 0) continue;
-        const uint32_t base = __builtin_amdgcn_readlane(at, bnd - w);
-        // the entry's column range, widened by this wave's edges in the band
-        const int32_t rlo = wave_min_i32(hit ? xlo : INT32_MAX);
-        const int32_t rhi = wave_max_i32(hit ? xhi : INT32_MIN);
-        if (lane == 0) {
-          const uint32_t eidx = ebase + ((uint32_t)bnd - blo);
-          atomicMin(&J.entry_xlo[eidx], rlo);
-          atomicMax(&J.entry_xhi[eidx], rhi);
+    if (ed.y0 != ed.y1)  // (a slot without an edge)
+      edge_bands(top, bot, band_rows, max(rows.x / bh, blo), min((rows.y - 1) / bh, bhi), lo, hi);
+  }
+  const REdge red = make_redge(ed);  // the copy every band of the edge receives
+  const int32_t ulo = wave_min_i32(lo), uhi = wave_max_i32(hi);
+  const uint64_t em = __ballot(lo <= hi);
+  const uint64_t below = (1ull << lane) - 1ull;
+  const bool transposed = by_edge(em, ulo, uhi);
+  // bands in windows of 64: lane j holds the count (then the list position)
+  // of band w + j, so each window takes one vector atomic
+  for (int32_t w = ulo; w <= uhi; w += 64) {
+    const int32_t wend = min(uhi, w + 63);
+    const int32_t bj = w + (int32_t)lane;  // this lane's band
+    uint32_t cnt = 0;
+    if (transposed) {
+      int32_t rlo = INT32_MAX, rhi = INT32_MIN;
+      for (uint64_t r = em; r; r &= r - 1) {
+        const uint32_t e = (uint32_t)__builtin_ctzll(r);
+        const int32_t l = (int32_t)lane_u32((uint32_t)lo, e), h = (int32_t)lane_u32((uint32_t)hi, e);
+        if (l <= bj && bj <= h) {
+          cnt++;
+          rlo = min(rlo, (int32_t)lane_u32((uint32_t)xlo, e));
+          rhi = max(rhi, (int32_t)lane_u32((uint32_t)xhi, e));
         }
-        if (hit) {
-          const uint32_t pos = base + (uint32_t)__popcll(m & below);
+      }
+      const uint32_t idx = ebase + (uint32_t)(bj - blo);
+      uint32_t pos = 0;
+      if (cnt) {
+        pos = J.entry_ecnt[idx] + atomicAdd(&J.entry_cur[idx], cnt);
+        atomicMin(&J.entry_xlo[idx], rlo);
+        atomicMax(&J.entry_xhi[idx], rhi);
+      }
+      for (uint64_t r = em; r; r &= r - 1) {
+        const uint32_t e = (uint32_t)__builtin_ctzll(r);
+        const int32_t l = (int32_t)lane_u32((uint32_t)lo, e), h = (int32_t)lane_u32((uint32_t)hi, e);
+        const REdge re{lane_f64(red.top, e), lane_f64(red.x_start, e), lane_f64(red.x_inc, e),
+                       (int32_t)lane_u32((uint32_t)red.ylo, e),
+                       (int32_t)lane_u32((uint32_t)red.yhi2, e)};
+        if (l <= bj && bj <= h) {
           if (pos < J.max_entry_edges)
-            J.entry_edges[pos] = red;
+            J.entry_edges[pos] = re;
           else
             atomicOr(&J.counters[2], 1u);
+          pos++;
         }
       }
+      continue;
     }
+    for (int32_t bnd = w; bnd <= wend; bnd++) {
+      const uint32_t c = (uint32_t)__popcll(__ballot(lo <= bnd && bnd <= hi));
+      if (bj == bnd) cnt = c;
+    }
+    const uint32_t at = cnt ? J.entry_ecnt[ebase + (uint32_t)(bj - blo)] +
+                                  atomicAdd(&J.entry_cur[ebase + (uint32_t)(bj - blo)], cnt)
+                            : 0u;
+    s_x[wv][0][lane] = INT32_MAX;
+    s_x[wv][1][lane] = INT32_MIN;
+    wave_lds_sync();
+    for (int32_t bnd = w; bnd <= wend; bnd++) {
+      const bool hit = lo <= bnd && bnd <= hi;
+      const uint64_t m = __ballot(hit);
+      if (m == 0) continue;
+      const uint32_t base = __builtin_amdgcn_readlane(at, bnd - w);
+      if (hit) {
+        // the entry's column range, widened by this wave's edges in the band
+        atomicMin(&s_x[wv][0][bnd - w], xlo);
+        atomicMax(&s_x[wv][1][bnd - w], xhi);
+        const uint32_t pos = base + (uint32_t)__popcll(m & below);
+        if (pos < J.max_entry_edges)
+          J.entry_edges[pos] = red;
+        else
+          atomicOr(&J.counters[2], 1u);
+      }
+    }
+    wave_lds_sync();
+    if (cnt) {
+      atomicMin(&J.entry_xlo[ebase + (uint32_t)(bj - blo)], s_x[wv][0][lane]);
+      atomicMax(&J.entry_xhi[ebase + (uint32_t)(bj - blo)], s_x[wv][1][lane]);
+    }
+    wave_lds_sync();
   }
 }
 
@@ -1785,8 +1893,6 @@ __device__ __forceinline__ T load_uniform(const T *p) {
 #endif
 }
 
-// Orders this wave's LDS accesses before and after the call (lanes of one
-// wave exchanging data through LDS).
 // Lane `src`'s value of v (every lane of the wave active).
 __device__ __forceinline__ uint32_t lane_read_u32(uint32_t v, uint32_t src) {
   return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)v);
@@ -1795,12 +1901,6 @@ __device__ __forceinline__ double lane_read_f64(double v, uint32_t src) {
   const uint64_t u = (uint64_t)__double_as_longlong(v);
   const uint32_t lo = lane_read_u32((uint32_t)u, src), hi = lane_read_u32((uint32_t)(u >> 32), src);
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Splits a word of two int16 deltas accumulated with 32-bit adds (the low
@@ -3422,7 +3522,7 @@ hipError_t z2d_launch_fill_u32(uint32_t *p, uint64_t n, uint32_t v, hipStream_t 
 
 hipError_t z2d_launch_edge_build(const JobView &J, hipStream_t st) {
   if (J.n_draws == 0) return hipSuccess;
-  dim3 grid((J.n_draws + 3) / 4);  // one wave per draw
+  const dim3 grid((J.n_egroups + 3) / 4);
   hipLaunchKernelGGL(k_edge_build, grid, dim3(256), 0, st, J);
   return hipGetLastError();
 }
@@ -3438,13 +3538,12 @@ hipError_t z2d_launch_rowprog(const JobView &J, const uint32_t *list, uint32_t n
 
 hipError_t z2d_launch_binning(const JobView &J, hipStream_t st) {
   if (J.n_bands == 0) return hipSuccess;
-  // entry edge lists: counts, offsets, then the copies (entry_ecnt,
-  // entry_cur and the entry column ranges were reset by the pipeline's
-  // first fill, z2d_launch_fill_set)
+  // entry edge lists: offsets from k_edge_build's counts, then the copies
+  // (entry_ecnt, entry_cur and the entry column ranges were reset by the
+  // pipeline's first fill, z2d_launch_fill_set)
   dim3 ggrid((J.n_egroups + 3) / 4);
-  if (J.n_egroups) hipLaunchKernelGGL(k_edge_bins<false>, ggrid, dim3(256), 0, st, J);
   scan_u32(J.entry_ecnt, J.max_entries, J.scan_tmp, J.counters + 2, st);
-  if (J.n_egroups) hipLaunchKernelGGL(k_edge_bins<true>, ggrid, dim3(256), 0, st, J);
+  if (J.n_egroups) hipLaunchKernelGGL(k_edge_bins, ggrid, dim3(256), 0, st, J);
   // band lists and entry records
   dim3 grid((J.n_slots + 3) / 4);
   hipLaunchKernelGGL(k_band_pass<false>, grid, dim3(256), 0, st, J);
