@@ -1298,12 +1298,10 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   const size_t o_nodes = L.take(total_nodes * sizeof(FNode));  // written by k_flatten
   const size_t o_edges = L.take(total_nodes * sizeof(z2d_edge));
   const size_t o_bandcnt = L.take(((size_t)n_bands + 1) * sizeof(uint32_t));
-  const size_t o_slotcnt = L.take(((size_t)n_slots + 1) * sizeof(uint32_t));
-  const uint64_t scan_n = std::max<uint64_t>(
-      std::max<uint64_t>(n_slots, max_entries), (uint64_t)n_tiles * spt);
-  // per scan: a ticket and a status word per workgroup (at most
-  // scan_n / SCAN_BLOCK + 1 workgroups)
-  const uint32_t scan_words = (uint32_t)(scan_n / SCAN_BLOCK + 2);
+  // per look-back: a ticket and a status word per workgroup (4,096 values of
+  // the entry scan, 16 slots of the band pass, 16 tiles of the strip pass)
+  const uint32_t scan_words = (uint32_t)(
+      std::max<uint64_t>(std::max<uint64_t>(n_slots, n_tiles) / 16, max_entries / SCAN_BLOCK) + 2);
   const size_t o_scantmp = L.take((size_t)3 * scan_words * sizeof(uint64_t));
   const size_t o_drows = L.take((size_t)nd * sizeof(int2));
   const size_t o_dacc = L.take((size_t)nd * sizeof(DrawAcc));
@@ -1433,7 +1431,6 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   J.slot_info = reinterpret_cast<const uint2 *>(D + o_slotinfo);
   J.band_slot_off = reinterpret_cast<const uint32_t *>(D + o_bso);
   J.n_slots = (uint32_t)n_slots;
-  J.slot_cnt = reinterpret_cast<uint32_t *>(D + o_slotcnt);
   J.scan_tmp = reinterpret_cast<uint64_t *>(D + o_scantmp);
   J.scan_words = scan_words;
   J.entries = reinterpret_cast<BandEntry *>(D + o_entries);

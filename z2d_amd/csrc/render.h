@@ -244,9 +244,9 @@ struct JobView {
   const uint2 *slot_info;         // per slot: band, surface
   const uint32_t *band_slot_off;  // n_bands: the band's first slot
   uint32_t n_slots;
-  uint32_t *slot_cnt;             // n_slots + 1 (scanned in place)
-  // the scans' look-back words: three regions of scan_words u64 (a ticket,
-  // then one status word per workgroup), zero at the start of each render
+  // look-back words (of the entry scan, the band and the strip pass): three
+  // regions of scan_words u64 (a ticket, then one status word per
+  // workgroup), zero at the start of each render
   uint64_t *scan_tmp;
   uint32_t scan_words;
   BandEntry *entries;    // per draw and estimated band, capacity max_entries
@@ -269,7 +269,7 @@ struct JobView {
   uint32_t *order_hist;      // ORDER_BUCKETS + 1
   // per strip (tile * strips_per_tile + strip): the band entries whose
   // composite region meets the strip, in draw order
-  uint32_t *strip_cnt;       // n_tiles * strips_per_tile + 1 (scanned in place)
+  uint32_t *strip_cnt;       // n_tiles * strips_per_tile + 1: offsets in strip_entries
   uint32_t *strip_entries;   // band entry indices, capacity max_strip_entries
   uint32_t max_strip_entries;
   // per strip: nonzero when an entry of its list is not a DRAW_FAST draw

@@ -1104,104 +1104,189 @@ __global__ void __launch_bounds__(256) k_curve_combine(const z2d_path_node *__re
 }
 
 // ---------------------------------------------------------------------------
+// Running sums over the workgroups of a launch, in one pass (decoupled
+// look-back): the workgroups are numbered by a ticket taken when they start,
+// so each waits only on workgroups already running.  A workgroup publishes
+// its aggregate, then its inclusive prefix, in its status word
+// (flag << 32 | value); its first wave sums its predecessors' words, 64 at a
+// time, back to the nearest inclusive prefix.  stat[0] is the ticket and
+// stat[1 + b] the status of workgroup b, all zero at launch.  A wait that
+// outlasts SCAN_SPIN_LIMIT polls (never expected) sets bit 1 of *err and goes
+// on, so every workgroup ends.
+// ---------------------------------------------------------------------------
+constexpr uint64_t SCAN_AGG = 1ull << 32, SCAN_INCL = 2ull << 32;
+constexpr uint32_t SCAN_SPIN_LIMIT = 1u << 20;
+
+__device__ __forceinline__ uint32_t scan_ticket(uint64_t *stat) {
+  return (uint32_t)atomicAdd(reinterpret_cast<unsigned long long *>(stat), 1ull);
+}
+// The sum of the workgroups before `bid` (by one whole wave of it).
+__device__ __forceinline__ uint32_t scan_lookback(uint64_t *stat, uint32_t bid, uint32_t total,
+                                                  uint32_t lane, uint32_t *err) {
+  uint64_t *const st = stat + 1;
+  uint32_t off = 0;
+  if (lane == 0)
+    __hip_atomic_store(&st[bid], (bid == 0 ? SCAN_INCL : SCAN_AGG) | total, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  if (bid == 0) return 0;
+  uint32_t spins = 0;
+  for (int32_t base = (int32_t)bid - 1;; base -= 64) {
+    const int32_t j = base - (int32_t)lane;  // lane 0 the nearest predecessor
+    uint64_t s = SCAN_INCL;                  // before workgroup 0: an inclusive zero
+    for (;;) {
+      if (j >= 0) s = __hip_atomic_load(&st[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__ballot((s >> 32) == 0) == 0) break;
+      if (++spins > SCAN_SPIN_LIMIT) {
+        if (lane == 0) atomicOr(err, 2u);
+        s = SCAN_INCL | (s & 0xFFFFFFFFull);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    const uint64_t pm = __ballot((s >> 32) == 2);
+    const uint32_t first = pm ? (uint32_t)__builtin_ctzll(pm) : 63u;
+    const uint32_t part = (uint32_t)wave_incl_scan(lane <= first ? (int32_t)(uint32_t)s : 0);
+    off += (uint32_t)__builtin_amdgcn_readlane((int32_t)part, 63);
+    if (pm) break;
+  }
+  if (lane == 0)
+    __hip_atomic_store(&st[bid], SCAN_INCL | (off + total), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  return off;
+}
+
+// ---------------------------------------------------------------------------
 // Binning: ordered draw lists per band (band_h rows of one surface).
 // ---------------------------------------------------------------------------
 // One wave per slot: a band and 64 consecutive draws of its surface (every
-// band has at least one slot).  FILL=false counts the draws whose composite
-// rows meet the band; FILL=true writes, after the scan of the slot counts,
-// the band list (the draws' entry indices, in draw order), the band offsets
-// band_cnt and each listed entry's record (its edge list from k_edge_bins).
-template <bool FILL>
-__global__ void k_band_pass(JobView J) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t slot = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (slot >= J.n_slots) return;
-  const uint2 si = J.slot_info[slot];  // band, surface
-  const uint32_t b = si.x, s = si.y;
-  const uint32_t c = slot - J.band_slot_off[b];
-  const int32_t y0 = (int32_t)(b - J.surf_band_off[s]) * (int32_t)J.band_h,
-                y1 = y0 + (int32_t)J.band_h;
-  const uint32_t d = J.surf_draw_off[s] + c * 64 + lane, d1 = J.surf_draw_off[s + 1];
-  const uint32_t lb = b - J.surf_band_off[s];  // band within the surface
-  bool hit = false;
-  uint32_t idx = 0;
-  if (d < d1) {
-    const int2 r = J.draw_rows[d];
-    hit = r.x < y1 && r.y > y0;
-    if (hit) {
-      // the draw's entry for this band (entries are owned by draws)
-      const DevDraw &D = J.draws[d];
-      const uint32_t blo = D.band_lo, bhi = D.band_hi;
-      if (lb < blo || lb > bhi) {
-        atomicOr(&J.counters[2], 1u);  // outside the host's band estimate
-        hit = false;
-      } else {
-        idx = D.entry_base + (lb - blo);
-      }
-    }
-  }
-  const uint64_t m = __ballot(hit);
-  if (!FILL) {
-    if (lane == 0) J.slot_cnt[slot] = (uint32_t)__popcll(m);
-    return;
-  }
-  const uint32_t base = J.slot_cnt[slot];
-  if (hit) {
-    const uint32_t pos = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    if (pos < J.max_entries) {
-      // only indices below the edge capacity were stored
-      const uint32_t off = J.entry_ecnt[idx], cnt = J.entry_ecnt[idx + 1] - off;
-      BandEntry e;
-      e.draw = d;
-      e.edge_off = off;
-      e.edge_cnt = off >= J.max_entry_edges ? 0u : min(cnt, J.max_entry_edges - off);
-      e.band = b;
-      // A tile wholly right of every crossing of the entry's edges, or wholly
-      // left of them, sees winding 0 (contours return to their start), so no
-      // coverage; with a bounded operator outside SSAA (which composites its
-      // whole mask box) nothing changes there.  Sample columns to pixels,
-      // rounded outward.
-      e.px_lo = INT32_MIN;
-      e.px_hi = INT32_MAX;
-      const DevDraw &Dd = J.draws[d];
-      if (Dd.mode != MODE_SSAA &&
-          !(Dd.flags & (DRAW_UNBOUNDED | DRAW_UNBALANCED | DRAW_ROWPROG | DRAW_SERIAL_PLOT))) {
-        const int32_t sc = Dd.mode == MODE_DIRECT ? 1 : 4;
-        const int32_t xl = J.entry_xlo[idx], xh = J.entry_xhi[idx];
-        if (xl > xh) {  // no edges in the band
-          e.px_lo = INT32_MAX;
-          e.px_hi = INT32_MIN;
-        } else if (xl != INT32_MIN && xh != INT32_MAX) {
-          e.px_lo = (int32_t)floor((double)xl / sc);
-          e.px_hi = (int32_t)floor((double)xh / sc);
+// band has at least one slot).  The draws whose composite rows meet the band
+// are counted, a workgroup's slots (PER for each of its 16 waves) take their
+// places by a look-back over the workgroups before, and the wave writes its
+// part of the band list (the draws' entry indices, in draw order), the band's
+// offset in band_cnt and each listed entry's record (its edge list from
+// k_edge_bins).  Bound by latency; as a counting launch, a scan and a writing
+// launch it took a small frame 5 us more.  A workgroup's ticket is an add on
+// one address (12 ns): past 512 workgroups (PASS_GROUPS) each wave takes
+// several slots.
+constexpr uint32_t PASS_WAVES = 16, PASS_GROUPS = 512, BAND_PASS_PER = 4, STRIP_PASS_PER = 8;
+
+template <uint32_t PER>
+__global__ void __launch_bounds__(64 * PASS_WAVES) k_band_pass(JobView J, uint64_t *stat) {
+  __shared__ uint32_t s_cnt[PASS_WAVES * PER], s_bid, s_off;
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (threadIdx.x == 0) s_bid = scan_ticket(stat);
+  __syncthreads();
+  const uint32_t bid = s_bid;
+  if (bid >= gridDim.x) return;  // (uniform) the ticket starts at zero
+  bool hit[PER];
+  uint32_t idx[PER], dr[PER];
+  uint64_t m[PER];
+#pragma unroll
+  for (uint32_t j = 0; j < PER; j++) {
+    const uint32_t slot = (bid * PASS_WAVES + wv) * PER + j;
+    hit[j] = false;
+    idx[j] = dr[j] = 0;
+    if (slot < J.n_slots) {
+      const uint2 si = J.slot_info[slot];  // band, surface
+      const uint32_t b = si.x, s = si.y;
+      const uint32_t lb = b - J.surf_band_off[s];  // band within the surface
+      const int32_t y0 = (int32_t)lb * (int32_t)J.band_h, y1 = y0 + (int32_t)J.band_h;
+      const uint32_t d = J.surf_draw_off[s] + (slot - J.band_slot_off[b]) * 64 + lane;
+      dr[j] = d;
+      if (d < J.surf_draw_off[s + 1]) {
+        const int2 r = J.draw_rows[d];
+        if (r.x < y1 && r.y > y0) {
+          // the draw's entry for this band (entries are owned by draws)
+          const DevDraw &D = J.draws[d];
+          const uint32_t blo = D.band_lo, bhi = D.band_hi;
+          if (lb < blo || lb > bhi) {
+            atomicOr(&J.counters[2], 1u);  // outside the host's band estimate
+          } else {
+            hit[j] = true;
+            idx[j] = D.entry_base + (lb - blo);
+          }
         }
       }
-      J.entries[idx] = e;
-      // the strip pass's tests for this entry: a tile at column tx0 (>= 0)
-      // takes it when it is not wholly beside the entry's crossings (px_lo
-      // >= tx0 + TILE_W + 1 or px_hi <= tx0 - 2) and meets the composite
-      // region (rx0 < tx0 + TILE_W, tx0 < rx1); a strip when its rows meet
-      // [ry0, ry1)
-      const int64_t lo_x = max(max((int64_t)Dd.rx0 - TILE_W, (int64_t)e.px_lo - TILE_W - 1),
-                               (int64_t)-1);
-      const int64_t hi_x = min(min((int64_t)Dd.rx1, (int64_t)e.px_hi + 2), (int64_t)INT32_MAX);
-      uint32_t smask = 0;
-      for (uint32_t st = 0; st < J.strips_per_tile; st++) {
-        const int32_t sy0 = y0 + (int32_t)st * ROWS_PER_THREAD;
-        if (Dd.ry1 > sy0 && Dd.ry0 < sy0 + ROWS_PER_THREAD) smask |= 1u << st;
-      }
-      const bool slow = !(Dd.flags & DRAW_FAST) || e.edge_cnt > PACKED_EDGE_LIMIT;
-      J.band_list[pos] = make_uint4(idx, (uint32_t)(int32_t)lo_x,
-                                    (uint32_t)(int32_t)max(hi_x, lo_x), smask | (slow ? 256u : 0u));
-    } else {
-      atomicOr(&J.counters[2], 1u);
+    }
+    m[j] = __ballot(hit[j]);
+    if (lane == 0) s_cnt[wv * PER + j] = (uint32_t)__popcll(m[j]);
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const uint32_t v = lane < PASS_WAVES * PER ? s_cnt[lane] : 0u;
+    const uint32_t incl = (uint32_t)wave_incl_scan((int32_t)v);
+    const uint32_t total = lane_u32(incl, 63);
+    const uint32_t off = scan_lookback(stat, bid, total, lane, J.counters + 2);
+    if (lane < PASS_WAVES * PER) s_cnt[lane] = incl - v;
+    if (lane == 0) {
+      s_off = off;
+      if (bid == gridDim.x - 1) J.band_cnt[J.n_bands] = off + total;
     }
   }
-  if (lane == 0) {
-    if (c == 0) J.band_cnt[b] = base;
-    if (slot == 0) J.band_cnt[J.n_bands] = J.slot_cnt[J.n_slots];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < PER; j++) {
+    const uint32_t slot = (bid * PASS_WAVES + wv) * PER + j;
+    if (slot >= J.n_slots) break;  // uniform
+    const uint2 si = J.slot_info[slot];
+    const uint32_t b = si.x;
+    const int32_t y0 = (int32_t)(b - J.surf_band_off[si.y]) * (int32_t)J.band_h;
+    const uint32_t base = s_off + s_cnt[wv * PER + j];
+    if (hit[j]) {
+      const uint32_t pos = base + (uint32_t)__popcll(m[j] & ((1ull << lane) - 1ull));
+      if (pos < J.max_entries) {
+        // only indices below the edge capacity were stored
+        const uint32_t off = J.entry_ecnt[idx[j]], cnt = J.entry_ecnt[idx[j] + 1] - off;
+        BandEntry e;
+        e.draw = dr[j];
+        e.edge_off = off;
+        e.edge_cnt = off >= J.max_entry_edges ? 0u : min(cnt, J.max_entry_edges - off);
+        e.band = b;
+        // A tile wholly right of every crossing of the entry's edges, or wholly
+        // left of them, sees winding 0 (contours return to their start), so no
+        // coverage; with a bounded operator outside SSAA (which composites its
+        // whole mask box) nothing changes there.  Sample columns to pixels,
+        // rounded outward.
+        e.px_lo = INT32_MIN;
+        e.px_hi = INT32_MAX;
+        const DevDraw &Dd = J.draws[dr[j]];
+        if (Dd.mode != MODE_SSAA &&
+            !(Dd.flags & (DRAW_UNBOUNDED | DRAW_UNBALANCED | DRAW_ROWPROG | DRAW_SERIAL_PLOT))) {
+          const int32_t sc = Dd.mode == MODE_DIRECT ? 1 : 4;
+          const int32_t xl = J.entry_xlo[idx[j]], xh = J.entry_xhi[idx[j]];
+          if (xl > xh) {  // no edges in the band
+            e.px_lo = INT32_MAX;
+            e.px_hi = INT32_MIN;
+          } else if (xl != INT32_MIN && xh != INT32_MAX) {
+            e.px_lo = (int32_t)floor((double)xl / sc);
+            e.px_hi = (int32_t)floor((double)xh / sc);
+          }
+        }
+        J.entries[idx[j]] = e;
+        // the strip pass's tests for this entry: a tile at column tx0 (>= 0)
+        // takes it when it is not wholly beside the entry's crossings (px_lo
+        // >= tx0 + TILE_W + 1 or px_hi <= tx0 - 2) and meets the composite
+        // region (rx0 < tx0 + TILE_W, tx0 < rx1); a strip when its rows meet
+        // [ry0, ry1)
+        const int64_t lo_x = max(max((int64_t)Dd.rx0 - TILE_W, (int64_t)e.px_lo - TILE_W - 1),
+                                 (int64_t)-1);
+        const int64_t hi_x = min(min((int64_t)Dd.rx1, (int64_t)e.px_hi + 2), (int64_t)INT32_MAX);
+        uint32_t smask = 0;
+        for (uint32_t st = 0; st < J.strips_per_tile; st++) {
+          const int32_t sy0 = y0 + (int32_t)st * ROWS_PER_THREAD;
+          if (Dd.ry1 > sy0 && Dd.ry0 < sy0 + ROWS_PER_THREAD) smask |= 1u << st;
+        }
+        const bool slow = !(Dd.flags & DRAW_FAST) || e.edge_cnt > PACKED_EDGE_LIMIT;
+        J.band_list[pos] = make_uint4(idx[j], (uint32_t)(int32_t)lo_x,
+                                      (uint32_t)(int32_t)max(hi_x, lo_x), smask | (slow ? 256u : 0u));
+      } else {
+        atomicOr(&J.counters[2], 1u);
+      }
+    }
+    if (lane == 0 && slot == J.band_slot_off[b]) J.band_cnt[b] = base;
   }
 }
+static_assert(PASS_WAVES * BAND_PASS_PER <= 64, "one lane per slot in the workgroup's scan");
 
 // Exclusive scan of n u32 values in place; a[n] receives the total.  One
 // workgroup of 1024 lanes walks the array in chunks of 16 values per lane.
@@ -1247,24 +1332,14 @@ __global__ void __launch_bounds__(1024) k_scan(uint32_t *a, uint32_t n) {
   if (t == 0) a[n] = carry;
 }
 
-// Exclusive scan of a[0..n) in place with a[n] = total, in one pass
-// (decoupled look-back): SCAN_BLOCK values per workgroup, the workgroups
-// numbered by a ticket taken when they start, so each waits only on
-// workgroups already running.  A workgroup publishes its aggregate, then its
-// inclusive prefix, in its status word (flag << 32 | value); its first wave
-// sums its predecessors' words, 64 at a time, back to the nearest inclusive
-// prefix.  stat[0] is the ticket and stat[1 + b] the status of workgroup b,
-// all zero at launch.  A wait that outlasts SCAN_SPIN_LIMIT polls (never
-// expected) sets bit 1 of *err and goes on, so every workgroup ends.
-constexpr uint64_t SCAN_AGG = 1ull << 32, SCAN_INCL = 2ull << 32;
-constexpr uint32_t SCAN_SPIN_LIMIT = 1u << 20;
-
+// Exclusive scan of a[0..n) in place with a[n] = total: SCAN_BLOCK values per
+// workgroup, running sums by look-back.
 __global__ void __launch_bounds__(256) k_scan_lb(uint32_t *a, uint32_t n, uint64_t *stat,
                                                  uint32_t *err) {
   __shared__ uint32_t ws[4];
   __shared__ uint32_t s_bid, s_off;
   const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
-  if (t == 0) s_bid = (uint32_t)atomicAdd(reinterpret_cast<unsigned long long *>(stat), 1ull);
+  if (t == 0) s_bid = scan_ticket(stat);
   __syncthreads();
   const uint32_t bid = s_bid;
   if (bid >= gridDim.x) return;  // (uniform) the ticket starts at zero
@@ -1293,37 +1368,7 @@ __global__ void __launch_bounds__(256) k_scan_lb(uint32_t *a, uint32_t n, uint64
   if (lane == 63) ws[w] = x;
   __syncthreads();
   if (w == 0) {
-    const uint32_t total = ws[0] + ws[1] + ws[2] + ws[3];
-    uint64_t *const st = stat + 1;
-    uint32_t off = 0;
-    if (lane == 0)
-      __hip_atomic_store(&st[bid], (bid == 0 ? SCAN_INCL : SCAN_AGG) | total, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    if (bid != 0) {
-      uint32_t spins = 0;
-      for (int32_t base = (int32_t)bid - 1;; base -= 64) {
-        const int32_t j = base - (int32_t)lane;  // lane 0 the nearest predecessor
-        uint64_t s = SCAN_INCL;                  // before workgroup 0: an inclusive zero
-        for (;;) {
-          if (j >= 0) s = __hip_atomic_load(&st[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (__ballot((s >> 32) == 0) == 0) break;
-          if (++spins > SCAN_SPIN_LIMIT) {
-            if (lane == 0) atomicOr(err, 2u);
-            s = SCAN_INCL | (s & 0xFFFFFFFFull);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-        const uint64_t pm = __ballot((s >> 32) == 2);
-        const uint32_t first = pm ? (uint32_t)__builtin_ctzll(pm) : 63u;
-        const uint32_t part = (uint32_t)wave_incl_scan(lane <= first ? (int32_t)(uint32_t)s : 0);
-        off += (uint32_t)__builtin_amdgcn_readlane((int32_t)part, 63);
-        if (pm) break;
-      }
-      if (lane == 0)
-        __hip_atomic_store(&st[bid], SCAN_INCL | (off + total), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
+    const uint32_t off = scan_lookback(stat, bid, ws[0] + ws[1] + ws[2] + ws[3], lane, err);
     if (lane == 0) s_off = off;
   }
   __syncthreads();
@@ -1358,87 +1403,151 @@ static void scan_u32(uint32_t *a, uint32_t n, uint64_t *stat, uint32_t *err, hip
 // ---------------------------------------------------------------------------
 // k_strip_pass: per strip (ROWS_PER_THREAD rows of one tile), the entries of
 // its band list whose composite region meets the strip, in draw order.  One
-// wave per tile walks the band's entries; FILL=false counts per strip,
-// FILL=true writes after the scan, and appends the strips that hold a
-// general-renderer entry to slow_list.  The list's length is one address and
-// adds to it are served one by one, so a workgroup of 16 tiles takes its
-// places with one add (one add per tile took 304 us for 134,000 tiles, a
-// fifth of them with such strips; this form 52 us).
+// wave per tile walks the band's entries twice: counting per strip, and, once
+// the workgroup's tiles (PER for each of its 16 waves) have their places by
+// look-back, writing; the strips that hold a general-renderer entry are
+// appended to slow_list.  That list's length is one address and adds to it
+// are served one by one, so a workgroup takes its places with one add (one
+// add per tile took 304 us for 134,000 tiles, a fifth of them with such
+// strips), and as with its ticket, past PASS_GROUPS workgroups each wave takes
+// several tiles: 14 us for a 4K page, 6 us for a small frame, whose three launches
+// took 14 and 10 and the gaps between them.
 // ---------------------------------------------------------------------------
-constexpr uint32_t STRIP_PASS_TILES = 16;
-
-template <bool FILL>
-__device__ void strip_pass_tile(const JobView &J, uint32_t t, uint32_t lane,
-                                uint32_t &slow_out) {
-  const TileRef T = J.tiles[t];
-  const uint32_t b = J.surf_band_off[T.surface] + T.ty;
-  const uint32_t e0 = min(J.band_cnt[b], J.max_entries);
-  const uint32_t e1 = min(J.band_cnt[b + 1], J.max_entries);
+template <uint32_t PER>
+__global__ void __launch_bounds__(64 * PASS_WAVES) k_strip_pass(JobView J, uint64_t *stat) {
+  constexpr uint32_t TILES = PASS_WAVES * PER;
+  constexpr uint32_t LANE_STRIPS = TILES * MAX_STRIPS_PER_TILE / 64;
+  // per strip of the workgroup, in strip order: its count, then its offset
+  __shared__ uint32_t s_cnt[TILES * MAX_STRIPS_PER_TILE];
+  // per tile: its strips with a general-renderer entry, then their place in
+  // the slow list (above bit 8)
+  __shared__ uint32_t s_slow[TILES];
+  __shared__ uint32_t s_slow_base, s_bid, s_off;
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (threadIdx.x == 0) s_bid = scan_ticket(stat);
+  __syncthreads();
+  const uint32_t bid = s_bid;
+  if (bid >= gridDim.x) return;  // (uniform) the ticket starts at zero
   const uint32_t spt = J.strips_per_tile;
-  const int32_t tx0 = (int32_t)T.tx * TILE_W;
-  uint32_t cnt[MAX_STRIPS_PER_TILE], base[MAX_STRIPS_PER_TILE];
-  uint32_t slow_strips = 0;  // strips whose list holds a general-renderer entry
-#pragma unroll
-  for (int s = 0; s < MAX_STRIPS_PER_TILE; s++) {
-    cnt[s] = 0;
-    base[s] = (FILL && (uint32_t)s < spt) ? J.strip_cnt[t * spt + s] : 0u;
-  }
   const uint64_t below = (1ull << lane) - 1ull;
-  for (uint32_t e = e0; e < e1; e += 64) {
-    uint32_t mask = 0, idx = 0;
-    bool slow = false;  // the entry needs the general renderer
+  // the band list of tile t, and the strips that its entry e + lane meets
+  // (see k_band_pass)
+  uint32_t e0 = 0, e1 = 0;
+  int32_t tx0 = 0;
+  auto tile = [&](uint32_t t) {
+    const TileRef T = J.tiles[t];
+    const uint32_t b = J.surf_band_off[T.surface] + T.ty;
+    e0 = min(J.band_cnt[b], J.max_entries);
+    e1 = min(J.band_cnt[b + 1], J.max_entries);
+    tx0 = (int32_t)T.tx * TILE_W;
+  };
+  auto entry = [&](uint32_t e, uint32_t &idx, bool &slow) {
+    uint32_t mask = 0;
+    idx = 0;
+    slow = false;
     if (e + lane < e1) {
-      const uint4 it = J.band_list[e + lane];  // see k_band_pass
+      const uint4 it = J.band_list[e + lane];
       idx = it.x;
       slow = (it.w & 256u) != 0;
       if (tx0 > (int32_t)it.y && tx0 < (int32_t)it.z) mask = it.w & 255u;
     }
+    return mask;
+  };
+  for (uint32_t j = 0; j < PER; j++) {
+    const uint32_t lt = wv * PER + j, t = bid * TILES + lt;
+    uint32_t cnt[MAX_STRIPS_PER_TILE];
 #pragma unroll
-    for (int s = 0; s < MAX_STRIPS_PER_TILE; s++) {
-      if ((uint32_t)s >= spt) break;  // uniform
-      const bool hit = (mask >> s) & 1u;
-      const uint64_t m = __ballot(hit);
-      if (FILL && __ballot(hit && slow)) slow_strips |= 1u << s;
-      if (FILL && hit) {
-        const uint32_t pos = base[s] + cnt[s] + (uint32_t)__popcll(m & below);
-        if (pos < J.max_strip_entries)
-          J.strip_entries[pos] = idx;
-        else
-          atomicOr(&J.counters[2], 1u);
+    for (int s = 0; s < MAX_STRIPS_PER_TILE; s++) cnt[s] = 0;
+    uint32_t slow_strips = 0;
+    if (t < J.n_tiles) {
+      tile(t);
+      for (uint32_t e = e0; e < e1; e += 64) {
+        uint32_t idx;
+        bool slow;
+        const uint32_t mask = entry(e, idx, slow);
+#pragma unroll
+        for (int s = 0; s < MAX_STRIPS_PER_TILE; s++) {
+          if ((uint32_t)s >= spt) break;  // uniform
+          const bool hit = (mask >> s) & 1u;
+          cnt[s] += (uint32_t)__popcll(__ballot(hit));
+          if (__ballot(hit && slow)) slow_strips |= 1u << s;
+        }
       }
-      cnt[s] += (uint32_t)__popcll(m);
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int s = 0; s < MAX_STRIPS_PER_TILE; s++)
+        if ((uint32_t)s < spt) s_cnt[lt * spt + s] = cnt[s];
+      s_slow[lt] = slow_strips;
     }
   }
-  if (!FILL && lane == 0) {
+  __syncthreads();
+  if (wv == 0) {
+    const uint32_t n = TILES * spt, i0 = LANE_STRIPS * lane;
+    uint32_t sum = 0;
+    for (uint32_t i = i0; i < min(i0 + LANE_STRIPS, n); i++) sum += s_cnt[i];
+    const uint32_t incl = (uint32_t)wave_incl_scan((int32_t)sum);
+    const uint32_t total = lane_u32(incl, 63);
+    const uint32_t off = scan_lookback(stat, bid, total, lane, J.counters + 2);
+    uint32_t run = incl - sum;
+    for (uint32_t i = i0; i < min(i0 + LANE_STRIPS, n); i++) {
+      const uint32_t v = s_cnt[i];
+      s_cnt[i] = run;
+      run += v;
+    }
+    uint32_t srun = 0;  // general-renderer strips of the tiles before
+    for (uint32_t i = 0; i < TILES; i += 64) {
+      const uint32_t sl = i + lane < TILES ? s_slow[i + lane] : 0u;
+      const uint32_t ns = (uint32_t)__popc(sl);
+      const uint32_t sincl = (uint32_t)wave_incl_scan((int32_t)ns);
+      if (i + lane < TILES) s_slow[i + lane] = sl | ((srun + sincl - ns) << 8);
+      srun += lane_u32(sincl, 63);
+    }
+    if (lane == 0) {
+      s_off = off;
+      if (bid == gridDim.x - 1) J.strip_cnt[J.n_tiles * spt] = off + total;
+      if (srun) s_slow_base = atomicAdd(&J.counters[9], srun);
+    }
+  }
+  __syncthreads();
+  const uint32_t off = s_off;
+  for (uint32_t j = 0; j < PER; j++) {
+    const uint32_t lt = wv * PER + j, t = bid * TILES + lt;
+    if (t >= J.n_tiles) break;  // uniform
+    if (lane < spt) {
+      const uint32_t sl = s_slow[lt];
+      const bool slow = (sl >> lane) & 1u;
+      J.strip_cnt[t * spt + lane] = off + s_cnt[lt * spt + lane];
+      J.strip_slow[t * spt + lane] = slow ? 1u : 0u;
+      if (slow)
+        J.slow_list[s_slow_base + (sl >> 8) + (uint32_t)__popc(sl & ((1u << lane) - 1u))] =
+            t * spt + lane;
+    }
+    uint32_t next[MAX_STRIPS_PER_TILE];
 #pragma unroll
     for (int s = 0; s < MAX_STRIPS_PER_TILE; s++)
-      if ((uint32_t)s < spt) J.strip_cnt[t * spt + s] = cnt[s];
+      next[s] = (uint32_t)s < spt ? off + s_cnt[lt * spt + s] : 0u;
+    tile(t);
+    for (uint32_t e = e0; e < e1; e += 64) {
+      uint32_t idx;
+      bool slow;
+      const uint32_t mask = entry(e, idx, slow);
+#pragma unroll
+      for (int s = 0; s < MAX_STRIPS_PER_TILE; s++) {
+        if ((uint32_t)s >= spt) break;  // uniform
+        const bool hit = (mask >> s) & 1u;
+        const uint64_t m = __ballot(hit);
+        if (hit) {
+          const uint32_t pos = next[s] + (uint32_t)__popcll(m & below);
+          if (pos < J.max_strip_entries)
+            J.strip_entries[pos] = idx;
+          else
+            atomicOr(&J.counters[2], 1u);
+        }
+        next[s] += (uint32_t)__popcll(m);
+      }
+    }
   }
-  if (FILL && lane < spt) J.strip_slow[t * spt + lane] = (slow_strips >> lane) & 1u;
-  slow_out = slow_strips;
-}
-
-template <bool FILL>
-__global__ void __launch_bounds__(64 * STRIP_PASS_TILES) k_strip_pass(JobView J) {
-  __shared__ uint32_t s_slow[STRIP_PASS_TILES], s_base;
-  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint32_t t = blockIdx.x * STRIP_PASS_TILES + w;
-  uint32_t slow = 0;
-  if (t < J.n_tiles) strip_pass_tile<FILL>(J, t, lane, slow);
-  if (!FILL) return;
-  if (lane == 0) s_slow[w] = slow;
-  __syncthreads();
-  uint32_t before = 0, total = 0;
-  for (uint32_t i = 0; i < STRIP_PASS_TILES; i++) {
-    if (i == w) before = total;
-    total += (uint32_t)__popc(s_slow[i]);
-  }
-  if (total == 0) return;  // uniform over the workgroup
-  if (threadIdx.x == 0) s_base = atomicAdd(&J.counters[9], total);
-  __syncthreads();
-  if (lane < J.strips_per_tile && ((slow >> lane) & 1u))
-    J.slow_list[s_base + before + (uint32_t)__popc(slow & ((1u << lane) - 1u))] =
-        t * J.strips_per_tile + lane;
 }
 
 // ---------------------------------------------------------------------------
@@ -3545,17 +3654,22 @@ hipError_t z2d_launch_binning(const JobView &J, hipStream_t st) {
   scan_u32(J.entry_ecnt, J.max_entries, J.scan_tmp, J.counters + 2, st);
   if (J.n_egroups) hipLaunchKernelGGL(k_edge_bins, ggrid, dim3(256), 0, st, J);
   // band lists and entry records
-  dim3 grid((J.n_slots + 3) / 4);
-  hipLaunchKernelGGL(k_band_pass<false>, grid, dim3(256), 0, st, J);
-  scan_u32(J.slot_cnt, J.n_slots, J.scan_tmp + J.scan_words, J.counters + 2, st);
-  hipLaunchKernelGGL(k_band_pass<true>, grid, dim3(256), 0, st, J);
+  const dim3 pblock(64 * PASS_WAVES);
+  uint64_t *const bstat = J.scan_tmp + J.scan_words, *const sstat = bstat + J.scan_words;
+  auto groups = [](uint32_t n, uint32_t per) {
+    return dim3((n + PASS_WAVES * per - 1) / (PASS_WAVES * per));
+  };
+  if (groups(J.n_slots, 1).x <= PASS_GROUPS)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_band_pass<1>), groups(J.n_slots, 1), pblock, 0, st, J, bstat);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_band_pass<BAND_PASS_PER>),
+                       groups(J.n_slots, BAND_PASS_PER), pblock, 0, st, J, bstat);
   if (J.n_tiles) {
-    const dim3 tgrid((J.n_tiles + STRIP_PASS_TILES - 1) / STRIP_PASS_TILES);
-    const dim3 tblock(64 * STRIP_PASS_TILES);
-    hipLaunchKernelGGL(k_strip_pass<false>, tgrid, tblock, 0, st, J);
-    scan_u32(J.strip_cnt, J.n_tiles * J.strips_per_tile, J.scan_tmp + 2 * J.scan_words,
-             J.counters + 2, st);
-    hipLaunchKernelGGL(k_strip_pass<true>, tgrid, tblock, 0, st, J);
+    if (groups(J.n_tiles, 1).x <= PASS_GROUPS)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_strip_pass<1>), groups(J.n_tiles, 1), pblock, 0, st, J, sstat);
+    else
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_strip_pass<STRIP_PASS_PER>),
+                         groups(J.n_tiles, STRIP_PASS_PER), pblock, 0, st, J, sstat);
     if (J.strip_order) {
       const uint32_t ns = J.n_tiles * J.strips_per_tile;
       const dim3 og((ns + 255) / 256);
