@@ -46,7 +46,8 @@ hipError_t z2d_launch_composite_paint(const z2d::PaintJob &job, uint32_t kind, b
 hipError_t z2d_launch_flatten(const z2d_path_node *raw, const z2d::FlatJob *jobs, uint32_t n_jobs,
                               z2d::FNode *out, z2d::FlatResult *res, uint32_t *rel,
                               const uint2 *curves, uint32_t n_curves, z2d::FlatTask *tasks,
-                              uint32_t *toff, z2d::FlatCurve *cv, bool emit, hipStream_t st,
+                              uint32_t *toff, z2d::FlatCurve *cv, const uint2 *groups,
+                              uint32_t n_groups, uint32_t *mvi, bool emit, hipStream_t st,
                               const z2d::FillSet *fill, bool any_serial);
 hipError_t z2d_launch_composite(const z2d::CompJob *dev_job, const z2d::CompJob &host_job,
                                 bool stream, hipStream_t st);
@@ -785,6 +786,9 @@ struct z2d_gpu_batch {
   const FlatJob *d_flat_jobs = nullptr;
   FNode *d_flat_out = nullptr;
   uint32_t *d_flat_rel = nullptr;
+  uint32_t *d_flat_mvi = nullptr;
+  const uint2 *d_flat_groups = nullptr;
+  uint32_t n_flat_groups = 0;
   const uint2 *d_flat_curves = nullptr;
   uint32_t n_flat_curves = 0;
   FlatTask *d_flat_tasks = nullptr;
@@ -1094,6 +1098,7 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
   std::vector<FlatJob> jobs;
   std::vector<uint32_t> job_draw;
   std::vector<uint2> curve_list;  // (job, raw node) of every curve, in draw and node order
+  std::vector<uint2> node_groups;  // (job, first node) of every 64 nodes of a draw
   for (uint32_t i = 0; i < (uint32_t)b->draws.size(); i++) {
     const HostDraw &h = b->draws[i];
     if (h.d.input_edges) continue;
@@ -1109,19 +1114,23 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
     for (uint32_t k = 0; k < h.raw_cnt; k++)
       if (b->raw_nodes[h.raw_off + k].tag == Z2D_NODE_CURVE_TO)
         curve_list.push_back(make_uint2((uint32_t)jobs.size(), h.raw_off + k));
+    for (uint32_t k = 0; k < h.raw_cnt; k += 64)
+      node_groups.push_back(make_uint2((uint32_t)jobs.size(), k));
     jobs.push_back(fj);
     job_draw.push_back(i);
   }
-  size_t fo_jobs = 0, fo_res = 0, fo_rel = 0, fo_curves = 0, fo_tasks = 0, fo_toff = 0,
-         fo_cv = 0;
+  size_t fo_jobs = 0, fo_res = 0, fo_rel = 0, fo_mvi = 0, fo_curves = 0, fo_groups = 0,
+         fo_tasks = 0, fo_toff = 0, fo_cv = 0;
   const uint32_t n_curves = (uint32_t)curve_list.size();
   if (!jobs.empty()) {
     Layout FL;
     FL.take(b->raw_nodes.size() * sizeof(z2d_path_node));
     fo_curves = FL.take(curve_list.size() * sizeof(uint2));
+    fo_groups = FL.take(node_groups.size() * sizeof(uint2));
     fo_jobs = FL.take(jobs.size() * sizeof(FlatJob));
     fo_res = FL.take(jobs.size() * sizeof(FlatResult));
     fo_rel = FL.take(b->raw_nodes.size() * sizeof(uint32_t));  // per raw node output offsets
+    fo_mvi = FL.take(b->raw_nodes.size() * sizeof(uint32_t));  // per close its contour's move
     fo_tasks = FL.take((size_t)n_curves * FLAT_TASKS * sizeof(FlatTask));
     fo_toff = FL.take((size_t)n_curves * FLAT_TASKS * sizeof(uint32_t));
     fo_cv = FL.take((size_t)n_curves * sizeof(FlatCurve));
@@ -1132,6 +1141,7 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
     std::memcpy(FH, b->raw_nodes.data(), b->raw_nodes.size() * sizeof(z2d_path_node));
     std::memcpy(FH + fo_jobs, jobs.data(), jobs.size() * sizeof(FlatJob));
     if (n_curves) std::memcpy(FH + fo_curves, curve_list.data(), curve_list.size() * sizeof(uint2));
+    std::memcpy(FH + fo_groups, node_groups.data(), node_groups.size() * sizeof(uint2));
     HIP_OK(ctx, hipMemcpyAsync(FD, FH, fo_res, hipMemcpyHostToDevice, st));
     HIP_OK(ctx, z2d_launch_flatten(reinterpret_cast<const z2d_path_node *>(FD),
                                    reinterpret_cast<const FlatJob *>(FD + fo_jobs),
@@ -1141,8 +1151,11 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
                                    reinterpret_cast<const uint2 *>(FD + fo_curves), n_curves,
                                    reinterpret_cast<FlatTask *>(FD + fo_tasks),
                                    reinterpret_cast<uint32_t *>(FD + fo_toff),
-                                   reinterpret_cast<FlatCurve *>(FD + fo_cv), false, st,
-                                   nullptr, true));
+                                   reinterpret_cast<FlatCurve *>(FD + fo_cv),
+                                   reinterpret_cast<const uint2 *>(FD + fo_groups),
+                                   (uint32_t)node_groups.size(),
+                                   reinterpret_cast<uint32_t *>(FD + fo_mvi), false, st, nullptr,
+                                   true));
     HIP_OK(ctx, hipMemcpyAsync(FH + fo_res, FD + fo_res, jobs.size() * sizeof(FlatResult),
                                hipMemcpyDeviceToHost, st));
     const auto cw0 = std::chrono::steady_clock::now();
@@ -1409,6 +1422,9 @@ static int32_t batch_prepare(z2d_gpu_batch *b) {
     b->d_flat_jobs = reinterpret_cast<const FlatJob *>(b->flat_buf.p + fo_jobs);
     b->d_flat_out = reinterpret_cast<FNode *>(D + o_nodes);
     b->d_flat_rel = reinterpret_cast<uint32_t *>(b->flat_buf.p + fo_rel);
+    b->d_flat_mvi = reinterpret_cast<uint32_t *>(b->flat_buf.p + fo_mvi);
+    b->d_flat_groups = reinterpret_cast<const uint2 *>(b->flat_buf.p + fo_groups);
+    b->n_flat_groups = (uint32_t)node_groups.size();
     b->d_flat_curves = reinterpret_cast<const uint2 *>(b->flat_buf.p + fo_curves);
     b->n_flat_curves = n_curves;
     b->d_flat_tasks = reinterpret_cast<FlatTask *>(b->flat_buf.p + fo_tasks);
@@ -1503,7 +1519,8 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
     e = z2d_launch_flatten(reinterpret_cast<const z2d_path_node *>(b->flat_buf.p),
                            b->d_flat_jobs, b->n_flat_jobs, b->d_flat_out, nullptr,
                            b->d_flat_rel, b->d_flat_curves, b->n_flat_curves, b->d_flat_tasks,
-                           b->d_flat_toff, nullptr, true, st, &F, b->n_flat_serial != 0);
+                           b->d_flat_toff, nullptr, b->d_flat_groups, b->n_flat_groups,
+                           b->d_flat_mvi, true, st, &F, b->n_flat_serial != 0);
   else
     e = z2d_launch_fill_set(F, st);
   if (e == hipSuccess) e = z2d_launch_edge_build(J, st);

@@ -553,15 +553,15 @@ __global__ void k_rowprog(JobView J, const uint32_t *draw_list, uint32_t n_list,
 // device.  A curve starts at its predecessor's end point, so its subdivision
 // is independent of the rest of the draw: k_curve_tasks splits each curve's
 // recursion into FLAT_TASKS subtrees (one thread each) and k_curve_combine
-// turns their counts into offsets and the curve's bounds.  k_flatten_wave
-// takes one wave per fill draw and one lane per raw node: wave scans give the
-// output offsets and the contour state.  Draws whose point-buffer state needs
-// the whole walk (FLAT_NONSIMPLE) go through k_flatten_serial, one thread per
-// draw.  The count pass (EMIT=false, once per prepared batch) returns the
-// number of flattened nodes, the contour-balance and line-after-close flags,
-// the (edge, band) bound and the bounding box of the tracked points, and
-// stores each raw node's output offset; the emit pass (every render) writes
-// the nodes.  The recursion is walked depth-first with the knots of a piece
+// turns their counts into offsets and the curve's bounds.  The count pass
+// (once per prepared batch, k_flatten_wave, one wave per fill draw and one lane
+// per raw node: wave scans give the output offsets and the contour state)
+// returns the number of flattened nodes, the contour-balance and
+// line-after-close flags, the (edge, band) bound and the bounding box of the
+// tracked points, and stores each raw node's output offset; the emit pass
+// (every render, k_flatten_nodes and k_curve_tasks) writes the nodes.  Draws
+// whose point-buffer state needs the whole walk (FLAT_NONSIMPLE) go through
+// k_flatten_serial in both, one thread per draw.  The recursion is walked depth-first with the knots of a piece
 // halved from its parent when descending and recomputed from the curve by its
 // path of halvings when moving to a sibling, which reproduces the recursion's
 // values exactly.
@@ -793,34 +793,22 @@ __device__ __forceinline__ void box_track(double *box, FPt p) {
 // balanced exactly when it ends at its move point.  The distinct-point count
 // is taken over the end points (a curve counted by its end point only), a
 // lower bound of the buffer's length, so a draw kept here has at least 3.
-template <bool EMIT>
 __global__ void __launch_bounds__(256) k_flatten_wave(const z2d_path_node *__restrict__ raw,
                                                       const FlatJob *__restrict__ jobs,
-                                                      uint32_t n_jobs, FNode *out,
-                                                      FlatResult *res, uint32_t *rel,
-                                                      const FlatCurve *__restrict__ cv,
-                                                      FillSet fill) {
+                                                      uint32_t n_jobs, FlatResult *res,
+                                                      uint32_t *rel, uint32_t *mvi,
+                                                      const FlatCurve *__restrict__ cv) {
   constexpr uint32_t NONE = 0xFFFFFFFFu;
-  if (EMIT) {
-    // the render's per-step resets (none of them is read by the flattening),
-    // here instead of a launch of their own
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint32_t f = 0; f < fill.count; f++)
-      for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < fill.n[f]; i += stride)
-        fill.p[f][i] = fill.v[f];
-  }
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t j = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (j >= n_jobs) return;
   const FlatJob J = jobs[j];
-  if (EMIT && J.serial) return;
   const z2d_path_node *nodes = raw + J.raw_off;
   uint32_t *rl = rel + J.raw_off;
-  FNode *o = out + J.node_off;
   const uint32_t n = J.raw_cnt;
   const uint64_t below = (1ull << lane) - 1ull;
   // carried from the previous 64 nodes (wave-uniform)
-  uint32_t c_tag = NONE, c_S = 0, c_out = 0, c_mvS = 0, c_cur = J.curve_base;
+  uint32_t c_tag = NONE, c_S = 0, c_out = 0, c_mvS = 0, c_mvi = 0, c_cur = J.curve_base;
   FPt c_pt{0.0, 0.0}, c_mv{0.0, 0.0};
   bool c_mv_ok = false;
   // per lane, reduced at the end
@@ -877,15 +865,15 @@ __global__ void __launch_bounds__(256) k_flatten_wave(const z2d_path_node *__res
     } else if (tag == Z2D_NODE_CLOSE_PATH) {
       cnt = 1;
       pairs += (uint64_t)flat_band_span(pp.y, mv.y, J.nbands, J.band_h);
+      mvi[J.raw_off + i] = J.raw_off + (at ? base + (uint32_t)src_at : c_mvi);
       if (!mv_ok || (ntag != NONE && ntag != Z2D_NODE_MOVE_TO) || 1u + S - mvS < 3u)
         flags |= FLAT_NONSIMPLE;
     }
     if ((tag == Z2D_NODE_LINE_TO || tag == Z2D_NODE_CURVE_TO) && i == n - 1 && !fpeq(p, mv))
       flags |= FLAT_UNBALANCED;
-    // output offsets from the node counts (a curve's from k_curve_combine),
-    // stored; the emit pass leaves curves to k_curve_tasks
+    // output offsets from the node counts (a curve's from k_curve_combine)
     const uint64_t cm = __ballot(tag == Z2D_NODE_CURVE_TO);
-    if (!EMIT && tag == Z2D_NODE_CURVE_TO) {
+    if (tag == Z2D_NODE_CURVE_TO) {
       const FlatCurve &r = cv[c_cur + (uint32_t)__popcll(cm & below)];
       cnt = r.cnt;
       flags |= r.flags;
@@ -894,17 +882,11 @@ __global__ void __launch_bounds__(256) k_flatten_wave(const z2d_path_node *__res
       box[1] = fmax(box[1], r.box[1]);
       box[2] = fmin(box[2], r.box[2]);
       box[3] = fmax(box[3], r.box[3]);
-    } else if (EMIT && act && tag != Z2D_NODE_CURVE_TO) {
-      // (a close of a draw kept here comes after two lines that move)
-      const bool close = tag == Z2D_NODE_CLOSE_PATH;
-      o[rl[i]] = FNode{close ? mv.x : p.x, close ? mv.y : p.y, tag, close ? 1u : 0u};
     }
     c_cur += (uint32_t)__popcll(cm);
-    if (!EMIT) {
-      const uint32_t x = (uint32_t)wave_incl_scan((int32_t)cnt);
-      if (act) rl[i] = c_out + x - cnt;
-      c_out += lane_u32(x, 63);
-    }
+    const uint32_t x = (uint32_t)wave_incl_scan((int32_t)cnt);
+    if (act) rl[i] = c_out + x - cnt;
+    c_out += lane_u32(x, 63);
     c_tag = lane_u32(tag, 63);
     c_pt = FPt{lane_f64(p.x, 63), lane_f64(p.y, 63)};
     c_S = lane_u32(S, 63);
@@ -912,27 +894,58 @@ __global__ void __launch_bounds__(256) k_flatten_wave(const z2d_path_node *__res
       const uint32_t last = 63u - (uint32_t)__builtin_clzll(mv_mask);
       c_mv = FPt{lane_f64(p.x, last), lane_f64(p.y, last)};
       c_mvS = lane_u32(S, last);
+      c_mvi = base + last;
       c_mv_ok = true;
     }
   }
-  if (!EMIT) {
-    for (int off = 32; off > 0; off >>= 1) {
-      pairs += __shfl_xor(pairs, off, 64);
-      flags |= __shfl_xor(flags, off, 64);
-      box[0] = fmin(box[0], __shfl_xor(box[0], off, 64));
-      box[1] = fmax(box[1], __shfl_xor(box[1], off, 64));
-      box[2] = fmin(box[2], __shfl_xor(box[2], off, 64));
-      box[3] = fmax(box[3], __shfl_xor(box[3], off, 64));
-    }
-    if (lane == 0) {
-      FlatResult r;
-      r.n_nodes = c_out;
-      r.flags = flags;
-      r.edge_pairs = pairs;
-      for (int q = 0; q < 4; q++) r.box[q] = box[q];
-      res[j] = r;
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    pairs += __shfl_xor(pairs, off, 64);
+    flags |= __shfl_xor(flags, off, 64);
+    box[0] = fmin(box[0], __shfl_xor(box[0], off, 64));
+    box[1] = fmax(box[1], __shfl_xor(box[1], off, 64));
+    box[2] = fmin(box[2], __shfl_xor(box[2], off, 64));
+    box[3] = fmax(box[3], __shfl_xor(box[3], off, 64));
   }
+  if (lane == 0) {
+    FlatResult r;
+    r.n_nodes = c_out;
+    r.flags = flags;
+    r.edge_pairs = pairs;
+    for (int q = 0; q < 4; q++) r.box[q] = box[q];
+    res[j] = r;
+  }
+}
+
+// Emit pass, one lane per raw node, 64 of a draw per wave: the nodes other
+// than curves (k_curve_tasks writes those) at the offsets of the count pass.
+// A close gets its contour's move point (mvi), and leads there: a draw kept by
+// k_flatten_wave closes only contours of at least two lines that move.  The
+// wave per draw of the count pass took 40 us for the 2,300 nodes of a page's
+// lines here, a chunk of 64 after the other; this form 7.
+__global__ void __launch_bounds__(256) k_flatten_nodes(const z2d_path_node *__restrict__ raw,
+                                                       const FlatJob *__restrict__ jobs,
+                                                       const uint2 *__restrict__ groups,
+                                                       uint32_t n_groups, FNode *out,
+                                                       const uint32_t *__restrict__ rel,
+                                                       const uint32_t *__restrict__ mvi,
+                                                       FillSet fill) {
+  // the render's per-step resets (none of them is read by the flattening),
+  // here instead of a launch of their own
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint32_t f = 0; f < fill.count; f++)
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < fill.n[f]; i += stride)
+      fill.p[f][i] = fill.v[f];
+  const uint32_t g = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (g >= n_groups) return;
+  const uint2 e = groups[g];  // job, first node
+  const FlatJob &J = jobs[e.x];
+  const uint32_t i = e.y + (threadIdx.x & 63);
+  if (J.serial || i >= J.raw_cnt) return;
+  const uint32_t r = J.raw_off + i, tag = raw[r].tag;
+  if (tag == Z2D_NODE_CURVE_TO) return;
+  const bool close = tag == Z2D_NODE_CLOSE_PATH;
+  const z2d_path_node &p = raw[close ? mvi[r] : r];
+  out[J.node_off + rel[r]] = FNode{p.v[0], p.v[1], tag, close ? 1u : 0u};
 }
 
 // One piece of a curve's Spline walk (task t of FLAT_TASKS): the subtree at
@@ -3692,16 +3705,16 @@ hipError_t z2d_launch_binning(const JobView &J, hipStream_t st) {
 hipError_t z2d_launch_flatten(const z2d_path_node *raw, const FlatJob *jobs, uint32_t n_jobs,
                               FNode *out, FlatResult *res, uint32_t *rel, const uint2 *curves,
                               uint32_t n_curves, FlatTask *tasks, uint32_t *toff, FlatCurve *cv,
-                              bool emit, hipStream_t st, const FillSet *fill,
-                              bool any_serial) {
+                              const uint2 *groups, uint32_t n_groups, uint32_t *mvi, bool emit,
+                              hipStream_t st, const FillSet *fill, bool any_serial) {
   if (n_jobs == 0) return hipSuccess;
   const FillSet no_fill{};
   const dim3 wgrid((n_jobs + 3) / 4), sgrid((n_jobs + 63) / 64);
   const dim3 tgrid((uint32_t)(((uint64_t)n_curves * FLAT_TASKS + 255) / 256)),
       cgrid((n_curves + 255) / 256);
   if (emit) {
-    hipLaunchKernelGGL(k_flatten_wave<true>, wgrid, dim3(256), 0, st, raw, jobs, n_jobs, out, res,
-                       rel, cv, fill ? *fill : no_fill);
+    hipLaunchKernelGGL(k_flatten_nodes, dim3((n_groups + 3) / 4), dim3(256), 0, st, raw, jobs,
+                       groups, n_groups, out, rel, mvi, fill ? *fill : no_fill);
     if (n_curves)
       hipLaunchKernelGGL(k_curve_tasks<true>, tgrid, dim3(256), 0, st, raw, jobs, curves, n_curves,
                          tasks, toff, rel, out);
@@ -3715,8 +3728,8 @@ hipError_t z2d_launch_flatten(const z2d_path_node *raw, const FlatJob *jobs, uin
       hipLaunchKernelGGL(k_curve_combine, cgrid, dim3(256), 0, st, raw, jobs, curves, n_curves,
                          tasks, toff, cv);
     }
-    hipLaunchKernelGGL(k_flatten_wave<false>, wgrid, dim3(256), 0, st, raw, jobs, n_jobs, out, res,
-                       rel, cv, no_fill);
+    hipLaunchKernelGGL(k_flatten_wave, wgrid, dim3(256), 0, st, raw, jobs, n_jobs, res, rel, mvi,
+                       cv);
     hipLaunchKernelGGL(k_flatten_serial<false>, sgrid, dim3(64), 0, st, raw, jobs, n_jobs, out,
                        res);
   }
