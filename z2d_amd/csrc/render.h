@@ -179,11 +179,11 @@ struct BandEntry {
   int32_t px_lo, px_hi;
 };
 
-// Per-draw constants of k_render_fast, the renderer of the common draw
-// (multisample, src_over in integer precision, a solid paint or a linear /
+// Per-draw constants of k_render_fast, the renderer of the common draws
+// (multisample: src_over in integer precision of a solid paint or a linear /
 // radial / conic gradient interpolated in linear RGB with at most FAST_STOPS
-// stops): one fixed-size block per draw, written by k_edge_build, fetched
-// by the strip worker one entry ahead of its use.
+// stops; src of a solid paint; clear): one fixed-size block per draw, written
+// by k_edge_build, fetched by the strip worker one entry ahead of its use.
 constexpr uint32_t FAST_STOPS = 8;
 enum : uint32_t {
   FAST_PAINT_NONE = 0,
@@ -191,6 +191,9 @@ enum : uint32_t {
   FAST_PAINT_LINEAR = 2,  // + gradient type
   FAST_PAINT_RADIAL = 3,
   FAST_PAINT_CONIC = 4,
+  // src of a solid paint, clear: the covered pixel becomes the masked paint
+  // (transparent) whatever it was
+  FAST_PAINT_REPLACE = 5,
 };
 struct alignas(16) FastDraw {
   int32_t rx0, rx1, ry0, ry1;  // composite region
@@ -206,7 +209,7 @@ struct alignas(16) FastDraw {
   float offs[FAST_STOPS];   // stop offsets
   float4 pre[FAST_STOPS];   // stop colors in the interpolation space
   // solid paint: the RGBA8 source masked by each coverage count 0..16
-  // (mask_coverage; entry 16 is the paint itself)
+  // (mask_coverage; entry 16 is the paint itself); clear: zeros
   uint32_t srctab[20];
 };
 constexpr uint32_t FAST_DRAW_CHUNKS = sizeof(FastDraw) / 16;  // 16-byte lanes

@@ -338,7 +338,7 @@ __device__ void write_fast_draw(FastDraw &F, const DevDraw &D, const DevPaint &P
   F.px = P.px.r | (P.px.g << 8) | (P.px.b << 16) | (P.px.a << 24);
   F.n_stops = 0;
   F.identity = 1;
-  if (pf >= FAST_PAINT_LINEAR) write_fast_gradient(F, *P.gradient, pf);
+  if (pf >= FAST_PAINT_LINEAR && pf <= FAST_PAINT_CONIC) write_fast_gradient(F, *P.gradient, pf);
 }
 
 // The copy of the work counters that workgroup (or draw) i adds to.
@@ -429,9 +429,13 @@ __device__ void draw_setup(const JobView &J, uint32_t d, uint32_t flags, const E
   D.flags = flags | DRAW_VISIBLE;
   J.draw_rows[d] = make_int2(D.ry0, D.ry1);
   if (J.fast) {
-    const uint32_t pf = fast_paint(P);
-    if (pf != FAST_PAINT_NONE && D.mode == MODE_MSAA && D.op == Z2D_OP_SRC_OVER &&
-        D.precision == Z2D_PRECISION_INTEGER &&
+    // (a solid src and a clear do not depend on the precision)
+    uint32_t pf = FAST_PAINT_NONE;
+    if (D.op == Z2D_OP_SRC_OVER && D.precision == Z2D_PRECISION_INTEGER)
+      pf = fast_paint(P);
+    else if (D.op == Z2D_OP_CLEAR || (D.op == Z2D_OP_SRC && P.kind == Z2D_PATTERN_OPAQUE))
+      pf = FAST_PAINT_REPLACE;
+    if (pf != FAST_PAINT_NONE && D.mode == MODE_MSAA &&
         !(D.flags & (DRAW_ROWPROG | DRAW_UNBALANCED | DRAW_UNBOUNDED))) {
       D.flags |= DRAW_FAST;
       write_fast_draw(J.fast[d], D, P, pf);
@@ -1696,8 +1700,11 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
   DrawAcc &A = J.draw_acc[d];
   // a solid paint's coverage table, for the fast renderer should the draw be
   // one (lane k: entry k)
-  if (it.y == 0 && J.fast && lane <= 16 && J.paints[D.paint].kind == Z2D_PATTERN_OPAQUE)
-    J.fast[d].srctab[lane] = fast_srctab_entry(J.paints[D.paint], lane);
+  if (it.y == 0 && J.fast && lane <= 16) {
+    const bool clear = D.op == Z2D_OP_CLEAR;
+    if (clear || J.paints[D.paint].kind == Z2D_PATTERN_OPAQUE)
+      J.fast[d].srctab[lane] = clear ? 0u : fast_srctab_entry(J.paints[D.paint], lane);
+  }
 
   ExtAcc acc{0, 0.0, 0.0, 0.0, 0.0};
   uint32_t first = it.y, end = min(it.y + EDGE_GROUP, n);  // the slots counted below
@@ -2674,9 +2681,9 @@ k_render(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t take) {
 }
 
 // ---------------------------------------------------------------------------
-// k_render_fast: the strip worker for the common draw (DRAW_FAST: multisample,
-// src_over in integer precision, a solid paint or a linear-RGB gradient of
-// at most FAST_STOPS stops, an edge list the packed deltas hold), over the
+// k_render_fast: the strip worker for the common draws (DRAW_FAST: multisample,
+// src_over in integer precision of a solid paint or a linear-RGB gradient of
+// at most FAST_STOPS stops, src of a solid paint, clear), over the
 // strips whose every entry is such a draw (k_render skips them).  The
 // coverage and composite arithmetic is k_render's; the difference is how the
 // work reaches the wave: one wave per workgroup, the entries of a strip
@@ -2702,6 +2709,7 @@ struct FastShared {
   // non-zero rule: winding of the edges wholly left of the strip, as a
   // difference array over its sample rows (zero between entries)
   int32_t ldiff[STRIP_SUBROWS + 1];
+  uint32_t stat_pix;  // pixel-draws of the strip (count_stats)
 };
 
 // Phase A: the crossings of a draw's band edges with SR sample rows from ys0
@@ -2939,10 +2947,15 @@ __device__ __forceinline__ int32_t rfl(int32_t v) {
   return (int32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
-// Bound by VALU issue and, at few waves, by latency: six waves per SIMD (80
-// VGPRs, 9 of them spilled, and 5.9 KB of LDS) take 0.79 ms for the 4K scene
-// of 10,000 paths, five (96, none spilled) 0.81, four 0.89.  Strips are
-// handed out as in k_render (take is never STRIPS_SLOW here).
+// Bound by VALU issue and, at few waves, by latency: six waves per SIMD (79
+// VGPRs and 5.9 KB of LDS) take 0.78 ms for the 4K scene of 10,000 paths, five
+// 0.81, four 0.89.  No register is spilled: what lives from entry to entry
+// leaves the registers while a gradient is evaluated, and the formats other
+// than RGBA8 are read and written in a loop over LDS (9 spilled before, a
+// third more code; a page of text 0.087 -> 0.082 ms).  A src or a clear takes
+// one more branch here; its strips were k_render's before (1,024 surfaces of
+// every format, one op in ten of them: 2.97 -> 1.94 ms for both kernels).
+// Strips are handed out as in k_render (take is never STRIPS_SLOW here).
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
 k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first,
               uint32_t take) {
@@ -2955,7 +2968,7 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
       take == STRIPS_ORDERED ? load_uniform(&J.strip_order[item]) : tile_base * spt + item;
   if (load_uniform(&J.strip_slow[sidx])) return;  // k_render's strip
 
-  uint32_t stat_pix = 0, stat_entries = 0;  // work counters (count_stats)
+  uint32_t stat_entries = 0;  // work counter (count_stats; the pixels' in LDS)
   {
     const TileRef T = load_uniform(&J.tiles[sidx / spt]);
     const uint32_t strip = sidx % spt;
@@ -2971,6 +2984,7 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
     for (uint32_t i = lane; i < (uint32_t)(FAST_ACC_ROWS * FAST_ACC_COLS / 4); i += 64)
       reinterpret_cast<uint4 *>(&sh.acc[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
     if (lane <= (uint32_t)STRIP_SUBROWS) sh.ldiff[lane] = 0;
+    if (lane == 0) sh.stat_pix = 0u;
     wave_lds_sync();
     const int32_t px = tx0 + (int32_t)lane;
     const bool col_ok = px < W;
@@ -2987,11 +3001,15 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
                                : 0u);
       }
     } else {
-#pragma unroll
+      // (a loop through LDS: the format switches once in the code, not per row)
+#pragma unroll 1
       for (int i = 0; i < ROWS_PER_THREAD; i++) {
         const int32_t py = ty0 + i;
-        pix[i] = px2_unpack((col_ok && py < H) ? load_raw(S, (int64_t)py * W + px) : 0u, S.fmt);
+        sh.u.c.ppaint[i][lane] = px2_to_rgba8(
+            px2_unpack((col_ok && py < H) ? load_raw(S, (int64_t)py * W + px) : 0u, S.fmt));
       }
+#pragma unroll
+      for (int i = 0; i < ROWS_PER_THREAD; i++) pix[i] = px2_rgba8(sh.u.c.ppaint[i][lane]);
     }
     // packed alpha surfaces hold fewer bits than a lane between draws
     const int a_bits = S.fmt >= Z2D_FORMAT_ALPHA4 ? fmt_bits(S.fmt) : 8;
@@ -3096,12 +3114,12 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
         }
         if (__ballot(cov != 0) == 0) continue;  // nothing covered in this strip (uniform)
         dirty |= cov;
-        const bool solid = pf == FAST_PAINT_SOLID;
+        const bool solid = pf == FAST_PAINT_SOLID || pf == FAST_PAINT_REPLACE;
         if (!solid || J.count_stats) {
           uint32_t need = 0;
 #pragma unroll
           for (int i = 0; i < ROWS_PER_THREAD; i++) need |= (kk[i] > 0 ? 1u : 0u) << i;
-          stat_pix += (uint32_t)__popc(need);
+          if (J.count_stats) atomicAdd(&sh.stat_pix, (uint32_t)__popc(need));
           if (!solid) {
             const int32_t np = __popc(need);
             const int32_t incl_p = wave_incl_scan(np);
@@ -3111,6 +3129,11 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
             for (int i = 0; i < ROWS_PER_THREAD; i++)
               if ((need >> i) & 1u) sh.u.c.plist[o++] = (uint8_t)((i << 6) | lane);
             wave_lds_sync();
+            // the gradients' 64-bit arithmetic needs the registers of the
+            // strip's pixels: they wait in a row of acc, zero again after
+            uint4 &kept = *reinterpret_cast<uint4 *>(&sh.acc[0][lane * 4]);
+            kept = make_uint4(px2_to_rgba8(pix[0]), px2_to_rgba8(pix[1]), px2_to_rgba8(pix[2]),
+                              px2_to_rgba8(pix[3]));
             if (pf == FAST_PAINT_LINEAR)
               fast_gradient<FAST_PAINT_LINEAR>(B, sh, tot_p, lane, tx0, ty0);
             else if (pf == FAST_PAINT_RADIAL)
@@ -3118,6 +3141,25 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
             else
               fast_gradient<FAST_PAINT_CONIC>(B, sh, tot_p, lane, tx0, ty0);
             wave_lds_sync();
+            const uint4 back = kept;
+            pix[0] = px2_rgba8(back.x);
+            pix[1] = px2_rgba8(back.y);
+            pix[2] = px2_rgba8(back.z);
+            pix[3] = px2_rgba8(back.w);
+            kept = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++) kk[i] = (int)((cov >> (8 * i)) & 0xFFu);
+          }
+        }
+        if (pf == FAST_PAINT_REPLACE) {
+          // over a transparent pixel src_over gives the source, whatever it
+          // is; a format without alpha reads back as opaque
+          const uint32_t under =
+              S.fmt == Z2D_FORMAT_RGB || S.fmt == Z2D_FORMAT_XRGB ? 0x00FF0000u : 0u;
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++) {
+            pix[i].rb = kk[i] > 0 ? 0u : pix[i].rb;
+            pix[i].ga = kk[i] > 0 ? under : pix[i].ga;
           }
         }
         if (solid) {
@@ -3147,10 +3189,12 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
       }
     } else {
 #pragma unroll
+      for (int i = 0; i < ROWS_PER_THREAD; i++) sh.u.c.ppaint[i][lane] = px2_to_rgba8(pix[i]);
+#pragma unroll 1
       for (int i = 0; i < ROWS_PER_THREAD; i++) {
         const int32_t py = ty0 + i;
         if (!col_ok || py >= H) continue;
-        uint32_t raw = px2_pack(pix[i], S.fmt);
+        uint32_t raw = px2_pack(px2_rgba8(sh.u.c.ppaint[i][lane]), S.fmt);
         bool changed = ((dirty >> (8 * i)) & 0xFFu) != 0;
         if (S.clip) {
           // Clip stage: Surface.composite(dst, mask, .dst_in) after the draws.
@@ -3163,7 +3207,10 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
       }
     }
   }
-  if (J.count_stats) strip_stats(J, stat_pix, stat_entries, 0u, lane);
+  if (J.count_stats) {
+    wave_lds_sync();
+    strip_stats(J, lane == 0 ? sh.stat_pix : 0u, stat_entries, 0u, lane);
+  }
 }
 
 // ---------------------------------------------------------------------------
