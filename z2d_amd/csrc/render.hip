@@ -2293,11 +2293,14 @@ __device__ __forceinline__ void strip_stats(const JobView &J, uint32_t stat_pix,
 // which renders every draw of a strip's list over its ROWS_PER_THREAD x
 // TILE_W pixels; they stay in registers from the first draw to the last.
 // The hardware's dispatcher hands out the strips (a workgroup for each, or
-// for every fourth where there are many, see z2d_launch_render).  (Persistent waves took
-// them from a counter before; adds to one address are served one after
-// another, about 12 ns each, so the 537,000 strips of a batch of 1,024 uneven
-// surfaces took 6.5 ms in each renderer whatever was on them: 6.39 + 6.58 ms,
-// now 2.06 + 1.16; a page of text, 32,400 strips, 428 us, now 110.)
+// for every fourth where there are many, see z2d_launch_render).  (Persistent
+// waves took them from a counter before; adds to one address are served one
+// after another, about 12 ns each, so the 537,000 strips of a batch of 1,024
+// uneven surfaces took 6.5 ms in each renderer whatever was on them: 6.39 +
+// 6.58 ms, with the dispatcher 2.06 + 1.16; a page of text, 32,400 strips, 428
+// us, then 110.)  Three waves per SIMD (168 VGPRs, 12 spilled): two and four
+// take 1.1 times as long on a scene of every operator.  Half of the time the
+// chip waits for the strips with the most draws.
 //   STRIPS_SLOW     a launch over all tiles: item i is slow_list[i]
 //   STRIPS_ORDERED  a launch over all tiles in J.strip_order
 //   STRIPS_TILES    tiles [tile_base, tile_base + tile_count)
@@ -2348,317 +2351,340 @@ k_render(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t take) {
 #pragma unroll
     for (int i = 0; i < ROWS_PER_THREAD; i++) orig[i] = pix[i];
 
-    for (uint32_t e = e0; e < e1; e++) {
-      const BandEntry E = load_uniform(&J.entries[load_uniform(&J.strip_entries[e])]);
-      const DevDraw D = load_uniform(&J.draws[E.draw]);
-      // uniform: the draw's composite region misses this strip
-      if (D.rx1 <= tx0 || D.rx0 >= tx0 + TILE_W) continue;
-      if (D.ry1 <= ty0 || D.ry0 >= ty0 + ROWS_PER_THREAD) continue;
-
-      const DevPaint &P = J.paints[D.paint];
-      const uint32_t p_kind = load_uniform(&P.kind);
-      const I4 p_px = load_uniform(&P.px);
-      const DevGradient *const p_grad = load_uniform(&P.gradient);
-      // a linear or radial gradient pattern interpolated in linear RGB with
-      // its stops staged: sampled by dense_gradient, without the paint in LDS
-      // (conic gradients go through paint_int: atan2 inlined here would
-      // spill)
-      uint32_t g_type = Z2D_GRADIENT_CONIC, g_method = 0, g_nstops = 0;
-      if (p_grad) {
-        g_type = load_uniform(&p_grad->type);
-        g_method = load_uniform(&p_grad->method);
-        g_nstops = load_uniform(&p_grad->n_stops);
+    for (uint32_t c = e0; c < e1; c += 64) {
+      // this chunk's entries, one per lane, and which of their draws' regions
+      // meet the strip (a load chain of five for each entry becomes one for 64
+      // of them and two each: 1917x1080 with every operator, precision and
+      // mode, 600 paths, 0.541 -> 0.527 ms)
+      uint32_t g_draw = 0, g_off = 0, g_cnt = 0, g_paint = 0;
+      const DevGradient *g_grad = nullptr;
+      bool meets = false;
+      if (c + lane < e1) {
+        const BandEntry E = J.entries[J.strip_entries[c + lane]];
+        const DevDraw &Dl = J.draws[E.draw];
+        g_draw = E.draw;
+        g_off = E.edge_off;
+        g_cnt = E.edge_cnt;
+        g_paint = Dl.paint;
+        g_grad = J.paints[g_paint].gradient;
+        meets = Dl.rx1 > tx0 && Dl.rx0 < tx0 + TILE_W && Dl.ry1 > ty0 &&
+                Dl.ry0 < ty0 + ROWS_PER_THREAD;
       }
-      const bool grad_dense = p_kind == Z2D_PATTERN_GRADIENT && g_type != Z2D_GRADIENT_CONIC &&
-                              g_method == Z2D_INTERP_LINEAR_RGB && g_nstops <= STAGED_STOPS;
-      StopView sv{nullptr, nullptr};
-      if (p_kind != Z2D_PATTERN_OPAQUE && !grad_dense) {
-        // the paint and its gradient in LDS for the samplers
-        wave_lds_sync();
-        constexpr uint32_t PW = sizeof(DevPaint) / 4, GW = sizeof(DevGradient) / 4;
-        static_assert(PW <= 64 && GW <= 128, "staging sizes");
-        if (lane < PW) reinterpret_cast<uint32_t *>(&sh.paint)[lane] =
-            reinterpret_cast<const uint32_t *>(&J.paints[D.paint])[lane];
+      for (uint64_t todo = __ballot(meets); todo != 0; todo &= todo - 1) {
+        const uint32_t j = (uint32_t)__ffsll((unsigned long long)todo) - 1;
+        const uint32_t e_off = __builtin_amdgcn_readlane(g_off, j);
+        const uint32_t e_cnt = __builtin_amdgcn_readlane(g_cnt, j);
+        const DevDraw D = load_uniform(&J.draws[__builtin_amdgcn_readlane(g_draw, j)]);
+        const DevPaint &P = J.paints[__builtin_amdgcn_readlane(g_paint, j)];
+        const DevGradient *const p_grad = reinterpret_cast<const DevGradient *>(
+            (uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(uint64_t)g_grad, j) |
+            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((uint32_t)((uint64_t)g_grad >> 32), j)
+             << 32));
+        const uint32_t p_kind = load_uniform(&P.kind);
+        const I4 p_px = load_uniform(&P.px);
+        // a linear or radial gradient pattern interpolated in linear RGB with
+        // its stops staged: sampled by dense_gradient, without the paint in LDS
+        // (conic gradients go through paint_int: atan2 inlined here would
+        // spill)
+        uint32_t g_type = Z2D_GRADIENT_CONIC, g_method = 0, g_nstops = 0;
         if (p_grad) {
-          const uint32_t *gs = reinterpret_cast<const uint32_t *>(p_grad);
-          uint32_t *gd = reinterpret_cast<uint32_t *>(&sh.grad);
-          if (lane < GW) gd[lane] = gs[lane];
-          if (lane + 64 < GW) gd[lane + 64] = gs[lane + 64];
-          if (lane == 0) sh.paint.gradient = &sh.grad;
+          g_type = load_uniform(&p_grad->type);
+          g_method = load_uniform(&p_grad->method);
+          g_nstops = load_uniform(&p_grad->n_stops);
         }
-        wave_lds_sync();
-      }
-      if (p_grad) {
-        const DevGradient G = load_uniform(p_grad);
-        if (G.n_stops <= STAGED_STOPS) {
+        const bool grad_dense = p_kind == Z2D_PATTERN_GRADIENT && g_type != Z2D_GRADIENT_CONIC &&
+                                g_method == Z2D_INTERP_LINEAR_RGB && g_nstops <= STAGED_STOPS;
+        StopView sv{nullptr, nullptr};
+        if (p_kind != Z2D_PATTERN_OPAQUE && !grad_dense) {
+          // the paint and its gradient in LDS for the samplers
           wave_lds_sync();
-          if (lane < G.n_stops) {
-            sh.soff[lane] = G.offs[lane];
-            sh.spre[lane] = G.pre[lane];
+          constexpr uint32_t PW = sizeof(DevPaint) / 4, GW = sizeof(DevGradient) / 4;
+          static_assert(PW <= 64 && GW <= 128, "staging sizes");
+          if (lane < PW) reinterpret_cast<uint32_t *>(&sh.paint)[lane] =
+              reinterpret_cast<const uint32_t *>(&J.paints[D.paint])[lane];
+          if (p_grad) {
+            const uint32_t *gs = reinterpret_cast<const uint32_t *>(p_grad);
+            uint32_t *gd = reinterpret_cast<uint32_t *>(&sh.grad);
+            if (lane < GW) gd[lane] = gs[lane];
+            if (lane + 64 < GW) gd[lane + 64] = gs[lane + 64];
+            if (lane == 0) sh.paint.gradient = &sh.grad;
           }
           wave_lds_sync();
-          sv = StopView{sh.soff, sh.spre};
-        } else {
-          sv = StopView{G.offs, G.pre};
         }
-      }
-      const int SC = D.mode == MODE_DIRECT ? 1 : 4;
-      const int SR = ROWS_PER_THREAD * SC;  // sample rows in this strip
-      const int32_t ys_base = ty0 * SC;
-      const int32_t xs_base = tx0 * SC;
-      const int32_t cols = TILE_W * SC;
-      const bool direct_unb = D.mode == MODE_DIRECT && (D.flags & DRAW_UNBOUNDED);
-
-      if (J.count_stats) stat_entries++;
-      int kk[ROWS_PER_THREAD];
-      if (direct_unb) {
-        // Row records give the whole result of the reference's quirky
-        // per-pair clears (src/internal/raster/direct.zig:88-124): cleared
-        // pixels become transparent, the rest composite at full coverage
-        // onto themselves or onto a cleared pixel.
-        const RowRec *R = J.rows + D.row_off;
-#pragma unroll
-        for (int i = 0; i < ROWS_PER_THREAD; i++) {
-          const int32_t py = ty0 + i;
-          kk[i] = 0;
-          if (!col_ok || py >= H) continue;
-          const RowRec rr = load_uniform(&R[py - D.row_y0]);
-          if (rr.kind == 1) continue;
-          if (rr.kind == 0 || px < rr.s || px >= rr.e) {
-            pix[i] = pack(I4{0, 0, 0, 0}, S.fmt);
-            continue;
-          }
-          if (rr.kind != 2) pix[i] = pack(I4{0, 0, 0, 0}, S.fmt);
-          kk[i] = 1;
-        }
-      } else {
-        const REdge *edges = J.entry_edges + E.edge_off;
-        const uint32_t ne = E.edge_off >= J.max_entry_edges
-                                ? 0u
-                                : min(E.edge_cnt, J.max_entry_edges - E.edge_off);
-        const bool eo = D.rule == Z2D_FILL_EVEN_ODD;
-        const bool packed = ne <= PACKED_EDGE_LIMIT;  // uniform
-
-        // ---- phase A: winding deltas of this draw's band edges.  Each
-        // crossing adds its direction at its sample column (crossings left of
-        // the strip at column 0, right of it nowhere); work items are the
-        // (edge, active sample row) pairs, compacted by a wave scan.
-        uint32_t inner = 0;  // a crossing at a column past 0 (per lane)
-        if (packed) {
-          for (uint32_t c0 = 0; c0 < ne; c0 += 64) {
-            const uint32_t k = c0 + lane;
-            int32_t n_sr = 0, lo = 0;
-            REdge ed{0.0, 0.0, 0.0, 0, 0};
-            if (k < ne) {
-              ed = edges[k];
-              const int32_t a = max(ed.ylo, ys_base), b = min(ed.yhi2 >> 1, ys_base + SR - 1);
-              if (a <= b) {
-                n_sr = b - a + 1;
-                lo = a - ys_base;
-                // every crossing right of the strip: no effect here (the
-                // crossings are monotone in the row, so the extremes are at
-                // the first and last active rows)
-                const double xa = redge_x(ed.top, ed.x_start, ed.x_inc, a);
-                const double xb = redge_x(ed.top, ed.x_start, ed.x_inc, b);
-                if (fmin(xa, xb) > (double)(xs_base + cols) + 1.0) n_sr = 0;
-              }
-            }
-            const int32_t incl = wave_incl_scan(n_sr);
-            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
-            if (total == 0) continue;  // uniform
-            sh.u.a.cedge[lane] = ed;
-            sh.clo[lane] = lo;
-            const uint32_t my_off = (uint32_t)(incl - n_sr);
-            sh.coff[lane] = my_off;
-            // each edge marks its own items (at most SR per edge)
-            for (int t = 0; t < n_sr; t++) sh.u.a.own[my_off + (uint32_t)t] = (uint8_t)lane;
+        if (p_grad) {
+          const DevGradient G = load_uniform(p_grad);
+          if (G.n_stops <= STAGED_STOPS) {
             wave_lds_sync();
-            for (uint32_t it = lane; it < total; it += 64) {
-              const uint32_t lj = sh.u.a.own[it];
-              const REdge ce = sh.u.a.cedge[lj];
-              const int sr = sh.clo[lj] + (int)(it - sh.coff[lj]);
-              const int32_t x = round_i32(redge_x(ce.top, ce.x_start, ce.x_inc, ys_base + sr));
-              const int32_t xr = x - xs_base;
-              if (xr >= cols) continue;
-              const int32_t col = xr < 0 ? 0 : xr;
-              inner |= (uint32_t)col;
-              const int32_t dv = eo ? 1 : ((ce.yhi2 & 1) ? -1 : 1);
-              atomicAdd(&sh.acc[sr][col >> 1], (col & 1) ? ((uint32_t)dv << 16) : (uint32_t)dv);
+            if (lane < G.n_stops) {
+              sh.soff[lane] = G.offs[lane];
+              sh.spre[lane] = G.pre[lane];
             }
             wave_lds_sync();
-          }
-        }
-
-        // ---- phase B: coverage per pixel (samples covered of SC x SC), then
-        // the composite in draw order.
-        const RowRec *R = (D.flags & DRAW_ROWPROG) ? J.rows + D.row_off : nullptr;
-        const int c_lo = (int)lane * SC;
-        // every delta at column 0: each sample row's winding is the same
-        // across the strip, so a pixel row's coverage is 4 samples per
-        // sample row inside (no prefix sums)
-        const bool uniform = packed && SC == 4 && !R && __ballot(inner != 0) == 0;
-        if (uniform) {
-          uint32_t w0 = 0;  // lane < 16: sample row `lane`'s column-0 word
-          if (lane < (uint32_t)SR) {
-            w0 = sh.acc[lane][0];
-            sh.acc[lane][0] = 0u;
-          }
-          int32_t lo, hi;
-          unpack_pair(w0, lo, hi);
-          const uint64_t in_rows = __ballot(lane < (uint32_t)SR && wind_in(lo, eo));
-#pragma unroll
-          for (int i = 0; i < ROWS_PER_THREAD; i++)
-            kk[i] = 4 * __popcll((in_rows >> (4 * i)) & 0xFull);
-        } else if (packed && SC == 4) {
-          if (eo) {
-            if (R) coverage_msaa<true, true>(sh.acc, lane, xs_base, ys_base, R, D.row_y0, D.row_n, kk);
-            else coverage_msaa<true, false>(sh.acc, lane, xs_base, ys_base, R, 0, 0, kk);
+            sv = StopView{sh.soff, sh.spre};
           } else {
-            if (R) coverage_msaa<false, true>(sh.acc, lane, xs_base, ys_base, R, D.row_y0, D.row_n, kk);
-            else coverage_msaa<false, false>(sh.acc, lane, xs_base, ys_base, R, 0, 0, kk);
+            sv = StopView{G.offs, G.pre};
           }
-        } else if (packed) {
-          // one sample per pixel: rows paired into one scan
-  #pragma unroll
-          for (int pr = 0; pr < ROWS_PER_THREAD / 2; pr++) {
-            int32_t d[2];
-  #pragma unroll
-            for (int q = 0; q < 2; q++) {
-              uint32_t *slot = &sh.acc[pr * 2 + q][lane >> 1];
-              const uint32_t v = *slot;
-              if ((lane & 1) == 0) *slot = 0u;
-              int32_t lo, hi;
-              unpack_pair(v, lo, hi);
-              d[q] = (lane & 1) ? hi : lo;
-            }
-            const uint32_t pk = (uint32_t)d[0] + ((uint32_t)d[1] << 16);
-            const uint32_t inc = (uint32_t)wave_incl_scan((int32_t)pk);
-            int32_t w[2];
-            unpack_pair(inc, w[0], w[1]);
-  #pragma unroll
-            for (int q = 0; q < 2; q++) {
-              int32_t cutoff = INT32_MAX;
-              if (R) {
-                const int32_t rr = ys_base + pr * 2 + q - D.row_y0;
-                if (rr >= 0 && rr < D.row_n) cutoff = load_uniform(&R[rr]).cutoff;
-              }
-              kk[pr * 2 + q] = (wind_in(w[q], eo) && xs_base + c_lo < cutoff) ? 1 : 0;
-            }
-          }
-        } else {
-          // more band edges than the packed deltas can hold: each lane
-          // evaluates the crossings of its own sample rows
-          if (J.count_stats) stat_unpacked++;
-  #pragma unroll
+        }
+        const int SC = D.mode == MODE_DIRECT ? 1 : 4;
+        const int SR = ROWS_PER_THREAD * SC;  // sample rows in this strip
+        const int32_t ys_base = ty0 * SC;
+        const int32_t xs_base = tx0 * SC;
+        const int32_t cols = TILE_W * SC;
+        const bool direct_unb = D.mode == MODE_DIRECT && (D.flags & DRAW_UNBOUNDED);
+
+        if (J.count_stats) stat_entries++;
+        int kk[ROWS_PER_THREAD];
+        if (direct_unb) {
+          // Row records give the whole result of the reference's quirky
+          // per-pair clears (src/internal/raster/direct.zig:88-124): cleared
+          // pixels become transparent, the rest composite at full coverage
+          // onto themselves or onto a cleared pixel.
+          const RowRec *R = J.rows + D.row_off;
+#pragma unroll
           for (int i = 0; i < ROWS_PER_THREAD; i++) {
-            int k = 0;
-            for (int o = 0; o < SC; o++) {
-              const int32_t ys = ys_base + i * SC + o;
-              const double mid = (double)ys + 0.5;
-              int32_t w[4] = {0, 0, 0, 0};
-              for (uint32_t q = 0; q < ne; q++) {
-                const REdge ed = edges[q];
-                if (ys < ed.ylo || ys > (ed.yhi2 >> 1)) continue;
-                const int32_t x = round_i32(ed.x_start + (ed.x_inc * (mid - ed.top)));
-                const int32_t dv = eo ? 1 : ((ed.yhi2 & 1) ? -1 : 1);
-                const int32_t xr = x - xs_base;
-  #pragma unroll
-                for (int j = 0; j < 4; j++)
-                  if (j < SC && xr <= c_lo + j) w[j] += dv;
-              }
-              int32_t cutoff = INT32_MAX;
-              if (R) {
-                const int32_t rr = ys - D.row_y0;
-                if (rr >= 0 && rr < D.row_n) cutoff = load_uniform(&R[rr]).cutoff;
-              }
-  #pragma unroll
-              for (int j = 0; j < 4; j++)
-                if (j < SC && wind_in(w[j], eo) && xs_base + c_lo + j < cutoff) k++;
+            const int32_t py = ty0 + i;
+            kk[i] = 0;
+            if (!col_ok || py >= H) continue;
+            const RowRec rr = load_uniform(&R[py - D.row_y0]);
+            if (rr.kind == 1) continue;
+            if (rr.kind == 0 || px < rr.s || px >= rr.e) {
+              pix[i] = pack(I4{0, 0, 0, 0}, S.fmt);
+              continue;
             }
-            kk[i] = k;
+            if (rr.kind != 2) pix[i] = pack(I4{0, 0, 0, 0}, S.fmt);
+            kk[i] = 1;
           }
-        }
-        wave_lds_sync();
-      }
-
-      uint32_t n_cov = 0;
-      if (D.op == Z2D_OP_SRC_OVER && D.precision == Z2D_PRECISION_INTEGER &&
-          D.mode != MODE_SSAA) {
-        uint32_t need = 0;  // covered pixels inside the composite region
-#pragma unroll
-        for (int i = 0; i < ROWS_PER_THREAD; i++) {
-          const int32_t py = ty0 + i;
-          if (col_ok && py < H && px >= D.rx0 && px < D.rx1 && py >= D.ry0 && py < D.ry1 &&
-              kk[i] > 0)
-            need |= 1u << i;
-        }
-        const bool solid = p_kind == Z2D_PATTERN_OPAQUE;
-        const int kfull = SC * SC;
-        if (__ballot(need != 0) == 0) continue;  // nothing covered in this strip (uniform)
-        if (solid) {
-          // the 17 possible masked sources of a solid paint
-          if (lane <= 16) {
-            const I4 m = (int)lane >= kfull ? p_px : mask_coverage(p_px, (int)lane);
-            sh.srctab[lane] = m.r | (m.g << 8) | (m.b << 16) | (m.a << 24);
-          }
-          wave_lds_sync();
         } else {
-          // paint samples of the covered pixels, evaluated densely: the
-          // (row, lane) pairs are listed with a wave scan and taken 64 at a
-          // time by one evaluation site; results go to LDS by pixel
-          const int32_t np = __popc(need);
-          const int32_t incl_p = wave_incl_scan(np);
-          const uint32_t tot_p = (uint32_t)__builtin_amdgcn_readlane(incl_p, 63);
-          uint32_t o = (uint32_t)(incl_p - np);
+          const REdge *edges = J.entry_edges + e_off;
+          const uint32_t ne = e_off >= J.max_entry_edges
+                                  ? 0u
+                                  : min(e_cnt, J.max_entry_edges - e_off);
+          const bool eo = D.rule == Z2D_FILL_EVEN_ODD;
+          const bool packed = ne <= PACKED_EDGE_LIMIT;  // uniform
+
+          // ---- phase A: winding deltas of this draw's band edges.  Each
+          // crossing adds its direction at its sample column (crossings left of
+          // the strip at column 0, right of it nowhere); work items are the
+          // (edge, active sample row) pairs, compacted by a wave scan.
+          uint32_t inner = 0;  // a crossing at a column past 0 (per lane)
+          if (packed) {
+            for (uint32_t c0 = 0; c0 < ne; c0 += 64) {
+              const uint32_t k = c0 + lane;
+              int32_t n_sr = 0, lo = 0;
+              REdge ed{0.0, 0.0, 0.0, 0, 0};
+              if (k < ne) {
+                ed = edges[k];
+                const int32_t a = max(ed.ylo, ys_base), b = min(ed.yhi2 >> 1, ys_base + SR - 1);
+                if (a <= b) {
+                  n_sr = b - a + 1;
+                  lo = a - ys_base;
+                  // every crossing right of the strip: no effect here (the
+                  // crossings are monotone in the row, so the extremes are at
+                  // the first and last active rows)
+                  const double xa = redge_x(ed.top, ed.x_start, ed.x_inc, a);
+                  const double xb = redge_x(ed.top, ed.x_start, ed.x_inc, b);
+                  if (fmin(xa, xb) > (double)(xs_base + cols) + 1.0) n_sr = 0;
+                }
+              }
+              const int32_t incl = wave_incl_scan(n_sr);
+              const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
+              if (total == 0) continue;  // uniform
+              sh.u.a.cedge[lane] = ed;
+              sh.clo[lane] = lo;
+              const uint32_t my_off = (uint32_t)(incl - n_sr);
+              sh.coff[lane] = my_off;
+              // each edge marks its own items (at most SR per edge)
+              for (int t = 0; t < n_sr; t++) sh.u.a.own[my_off + (uint32_t)t] = (uint8_t)lane;
+              wave_lds_sync();
+              for (uint32_t it = lane; it < total; it += 64) {
+                const uint32_t lj = sh.u.a.own[it];
+                const REdge ce = sh.u.a.cedge[lj];
+                const int sr = sh.clo[lj] + (int)(it - sh.coff[lj]);
+                const int32_t x = round_i32(redge_x(ce.top, ce.x_start, ce.x_inc, ys_base + sr));
+                const int32_t xr = x - xs_base;
+                if (xr >= cols) continue;
+                const int32_t col = xr < 0 ? 0 : xr;
+                inner |= (uint32_t)col;
+                const int32_t dv = eo ? 1 : ((ce.yhi2 & 1) ? -1 : 1);
+                atomicAdd(&sh.acc[sr][col >> 1], (col & 1) ? ((uint32_t)dv << 16) : (uint32_t)dv);
+              }
+              wave_lds_sync();
+            }
+          }
+
+          // ---- phase B: coverage per pixel (samples covered of SC x SC), then
+          // the composite in draw order.
+          const RowRec *R = (D.flags & DRAW_ROWPROG) ? J.rows + D.row_off : nullptr;
+          const int c_lo = (int)lane * SC;
+          // every delta at column 0: each sample row's winding is the same
+          // across the strip, so a pixel row's coverage is 4 samples per
+          // sample row inside (no prefix sums)
+          const bool uniform = packed && SC == 4 && !R && __ballot(inner != 0) == 0;
+          if (uniform) {
+            uint32_t w0 = 0;  // lane < 16: sample row `lane`'s column-0 word
+            if (lane < (uint32_t)SR) {
+              w0 = sh.acc[lane][0];
+              sh.acc[lane][0] = 0u;
+            }
+            int32_t lo, hi;
+            unpack_pair(w0, lo, hi);
+            const uint64_t in_rows = __ballot(lane < (uint32_t)SR && wind_in(lo, eo));
 #pragma unroll
-          for (int i = 0; i < ROWS_PER_THREAD; i++)
-            if ((need >> i) & 1u) sh.u.c.plist[o++] = (uint8_t)((i << 6) | lane);
-          wave_lds_sync();
-          if (grad_dense) {
-            const DevGradient G = load_uniform(p_grad);
-            if (G.type == Z2D_GRADIENT_LINEAR)
-              dense_gradient<Z2D_GRADIENT_LINEAR>(G, sh, tot_p, lane, tx0, ty0);
-            else
-              dense_gradient<Z2D_GRADIENT_RADIAL>(G, sh, tot_p, lane, tx0, ty0);
+            for (int i = 0; i < ROWS_PER_THREAD; i++)
+              kk[i] = 4 * __popcll((in_rows >> (4 * i)) & 0xFull);
+          } else if (packed && SC == 4) {
+            if (eo) {
+              if (R)
+                coverage_msaa<true, true>(sh.acc, lane, xs_base, ys_base, R, D.row_y0, D.row_n, kk);
+              else coverage_msaa<true, false>(sh.acc, lane, xs_base, ys_base, R, 0, 0, kk);
+            } else {
+              if (R)
+                coverage_msaa<false, true>(sh.acc, lane, xs_base, ys_base, R, D.row_y0, D.row_n, kk);
+              else coverage_msaa<false, false>(sh.acc, lane, xs_base, ys_base, R, 0, 0, kk);
+            }
+          } else if (packed) {
+            // one sample per pixel: rows paired into one scan
+    #pragma unroll
+            for (int pr = 0; pr < ROWS_PER_THREAD / 2; pr++) {
+              int32_t d[2];
+    #pragma unroll
+              for (int q = 0; q < 2; q++) {
+                uint32_t *slot = &sh.acc[pr * 2 + q][lane >> 1];
+                const uint32_t v = *slot;
+                if ((lane & 1) == 0) *slot = 0u;
+                int32_t lo, hi;
+                unpack_pair(v, lo, hi);
+                d[q] = (lane & 1) ? hi : lo;
+              }
+              const uint32_t pk = (uint32_t)d[0] + ((uint32_t)d[1] << 16);
+              const uint32_t inc = (uint32_t)wave_incl_scan((int32_t)pk);
+              int32_t w[2];
+              unpack_pair(inc, w[0], w[1]);
+    #pragma unroll
+              for (int q = 0; q < 2; q++) {
+                int32_t cutoff = INT32_MAX;
+                if (R) {
+                  const int32_t rr = ys_base + pr * 2 + q - D.row_y0;
+                  if (rr >= 0 && rr < D.row_n) cutoff = load_uniform(&R[rr]).cutoff;
+                }
+                kk[pr * 2 + q] = (wind_in(w[q], eo) && xs_base + c_lo < cutoff) ? 1 : 0;
+              }
+            }
           } else {
-#pragma unroll 1
-            for (uint32_t it = lane; it < tot_p; it += 64) {
-              const uint32_t v = sh.u.c.plist[it];
-              const uint32_t pl = v & 63u, pi = v >> 6;
-              const I4 c = paint_int(sh.paint, sv, J.blue_noise, tx0 + (int32_t)pl,
-                                     ty0 + (int32_t)pi);
-              sh.u.c.ppaint[pi][pl] = c.r | (c.g << 8) | (c.b << 16) | (c.a << 24);
+            // more band edges than the packed deltas can hold: each lane
+            // evaluates the crossings of its own sample rows
+            if (J.count_stats) stat_unpacked++;
+    #pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++) {
+              int k = 0;
+              for (int o = 0; o < SC; o++) {
+                const int32_t ys = ys_base + i * SC + o;
+                const double mid = (double)ys + 0.5;
+                int32_t w[4] = {0, 0, 0, 0};
+                for (uint32_t q = 0; q < ne; q++) {
+                  const REdge ed = edges[q];
+                  if (ys < ed.ylo || ys > (ed.yhi2 >> 1)) continue;
+                  const int32_t x = round_i32(ed.x_start + (ed.x_inc * (mid - ed.top)));
+                  const int32_t dv = eo ? 1 : ((ed.yhi2 & 1) ? -1 : 1);
+                  const int32_t xr = x - xs_base;
+    #pragma unroll
+                  for (int j = 0; j < 4; j++)
+                    if (j < SC && xr <= c_lo + j) w[j] += dv;
+                }
+                int32_t cutoff = INT32_MAX;
+                if (R) {
+                  const int32_t rr = ys - D.row_y0;
+                  if (rr >= 0 && rr < D.row_n) cutoff = load_uniform(&R[rr]).cutoff;
+                }
+    #pragma unroll
+                for (int j = 0; j < 4; j++)
+                  if (j < SC && wind_in(w[j], eo) && xs_base + c_lo + j < cutoff) k++;
+              }
+              kk[i] = k;
             }
           }
           wave_lds_sync();
         }
-        const bool fast_full = (D.flags & DRAW_FAST_SRC) != 0;
-        // the solid fast path stores the source where coverage is full
-        const uint32_t full_raw = fast_full ? pack(p_px, S.fmt) : 0u;
-        src_over_rows(pix, kk, need, solid, fast_full, kfull, full_raw, sh, lane, S.fmt, n_cov);
-      } else {
-        // every other operator / precision / mode: one composite instance,
-        // rows in a rolled loop over a copy of the strip's pixels
-        uint32_t tp[ROWS_PER_THREAD];
+
+        uint32_t n_cov = 0;
+        if (D.op == Z2D_OP_SRC_OVER && D.precision == Z2D_PRECISION_INTEGER &&
+            D.mode != MODE_SSAA) {
+          uint32_t need = 0;  // covered pixels inside the composite region
 #pragma unroll
-        for (int i = 0; i < ROWS_PER_THREAD; i++) tp[i] = pix[i];
+          for (int i = 0; i < ROWS_PER_THREAD; i++) {
+            const int32_t py = ty0 + i;
+            if (col_ok && py < H && px >= D.rx0 && px < D.rx1 && py >= D.ry0 && py < D.ry1 &&
+                kk[i] > 0)
+              need |= 1u << i;
+          }
+          const bool solid = p_kind == Z2D_PATTERN_OPAQUE;
+          const int kfull = SC * SC;
+          if (__ballot(need != 0) == 0) continue;  // nothing covered in this strip (uniform)
+          if (solid) {
+            // the 17 possible masked sources of a solid paint
+            if (lane <= 16) {
+              const I4 m = (int)lane >= kfull ? p_px : mask_coverage(p_px, (int)lane);
+              sh.srctab[lane] = m.r | (m.g << 8) | (m.b << 16) | (m.a << 24);
+            }
+            wave_lds_sync();
+          } else {
+            // paint samples of the covered pixels, evaluated densely: the
+            // (row, lane) pairs are listed with a wave scan and taken 64 at a
+            // time by one evaluation site; results go to LDS by pixel
+            const int32_t np = __popc(need);
+            const int32_t incl_p = wave_incl_scan(np);
+            const uint32_t tot_p = (uint32_t)__builtin_amdgcn_readlane(incl_p, 63);
+            uint32_t o = (uint32_t)(incl_p - np);
+#pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++)
+              if ((need >> i) & 1u) sh.u.c.plist[o++] = (uint8_t)((i << 6) | lane);
+            wave_lds_sync();
+            if (grad_dense) {
+              const DevGradient G = load_uniform(p_grad);
+              if (G.type == Z2D_GRADIENT_LINEAR)
+                dense_gradient<Z2D_GRADIENT_LINEAR>(G, sh, tot_p, lane, tx0, ty0);
+              else
+                dense_gradient<Z2D_GRADIENT_RADIAL>(G, sh, tot_p, lane, tx0, ty0);
+            } else {
 #pragma unroll 1
-        for (int i = 0; i < ROWS_PER_THREAD; i++) {
-          const int32_t py = ty0 + i;
-          if (!col_ok || py >= H) continue;
-          const bool in_region = px >= D.rx0 && px < D.rx1 && py >= D.ry0 && py < D.ry1;
-          if (!in_region) continue;
-          uint32_t v = tp[i];
-          if (D.mode == MODE_MSAA && (D.flags & DRAW_UNBOUNDED) && msaa_preclear(D, W, px, py))
-            v = pack(I4{0, 0, 0, 0}, S.fmt);
-          const int k = kk[i];
-          n_cov += k > 0;
-          tp[i] = composite_cov(v, S.fmt, k, SC * SC, D, P, sv, J.blue_noise, px, py);
-        }
+              for (uint32_t it = lane; it < tot_p; it += 64) {
+                const uint32_t v = sh.u.c.plist[it];
+                const uint32_t pl = v & 63u, pi = v >> 6;
+                const I4 c = paint_int(sh.paint, sv, J.blue_noise, tx0 + (int32_t)pl,
+                                       ty0 + (int32_t)pi);
+                sh.u.c.ppaint[pi][pl] = c.r | (c.g << 8) | (c.b << 16) | (c.a << 24);
+              }
+            }
+            wave_lds_sync();
+          }
+          const bool fast_full = (D.flags & DRAW_FAST_SRC) != 0;
+          // the solid fast path stores the source where coverage is full
+          const uint32_t full_raw = fast_full ? pack(p_px, S.fmt) : 0u;
+          src_over_rows(pix, kk, need, solid, fast_full, kfull, full_raw, sh, lane, S.fmt, n_cov);
+        } else {
+          // every other operator / precision / mode: one composite instance,
+          // rows in a rolled loop over a copy of the strip's pixels
+          uint32_t tp[ROWS_PER_THREAD];
 #pragma unroll
-        for (int i = 0; i < ROWS_PER_THREAD; i++) pix[i] = tp[i];
+          for (int i = 0; i < ROWS_PER_THREAD; i++) tp[i] = pix[i];
+#pragma unroll 1
+          for (int i = 0; i < ROWS_PER_THREAD; i++) {
+            const int32_t py = ty0 + i;
+            if (!col_ok || py >= H) continue;
+            const bool in_region = px >= D.rx0 && px < D.rx1 && py >= D.ry0 && py < D.ry1;
+            if (!in_region) continue;
+            uint32_t v = tp[i];
+            if (D.mode == MODE_MSAA && (D.flags & DRAW_UNBOUNDED) && msaa_preclear(D, W, px, py))
+              v = pack(I4{0, 0, 0, 0}, S.fmt);
+            const int k = kk[i];
+            n_cov += k > 0;
+            tp[i] = composite_cov(v, S.fmt, k, SC * SC, D, P, sv, J.blue_noise, px, py);
+          }
+#pragma unroll
+          for (int i = 0; i < ROWS_PER_THREAD; i++) pix[i] = tp[i];
+        }
+        if (J.count_stats) stat_pix += n_cov;  // per lane
       }
-      if (J.count_stats) stat_pix += n_cov;  // per lane
     }
 
     if (S.clip) {
