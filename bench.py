@@ -257,8 +257,8 @@ def bench_uneven_batch(gpu, ctx, n_surfaces=4096, seed=0xC4):
     20% alpha8, cleared to 0, 1-50 paths each of the 4K scene's
     distribution; 30% of the paths stroked: width U(0.5, 8), joins and caps
     uniform, 25% dashed).  Strokes are tessellated on the host when the batch
-    is built.  One persistent launch vs one launch per surface over the same
-    prepared batch; the persistent launch also as a replayed hipGraph of the
+    is built.  One launch for all vs one launch per surface over the same
+    prepared batch; the one launch also as a replayed hipGraph of the
     whole pipeline.  The band height is picked by the autotuner first.  The
     host build is timed both as one call per draw and through draw_n
     (strokes tessellated on host threads)."""

@@ -170,7 +170,7 @@ void z2d_gpu_surface_destroy(z2d_gpu_surface *s);
 
 /* ---- batches ----------------------------------------------------------------
  * Many fills on many resident surfaces rendered by one pipeline launch
- * (edge build, binning, one persistent tile-render launch).  Draws on one
+ * (edge build, binning, one tile-render launch).  Draws on one
  * surface are applied in the order they were added, exactly like
  * successive painter.fill calls.  No reference counterpart: it batches the
  * reference's per-call painter.fill. */
@@ -188,7 +188,7 @@ int32_t z2d_gpu_batch_fill_polygon(z2d_gpu_batch *b, z2d_gpu_surface *surface,
                                    uint32_t op, uint32_t precision);
 /* Uploads the batch's inputs to HBM (no rendering). */
 int32_t z2d_gpu_batch_prepare(z2d_gpu_batch *b);
-/* Renders the prepared batch.  mode 0: one persistent launch for all
+/* Renders the prepared batch.  mode 0: one launch for all
  * surfaces; mode 1: one launch per surface.  Asynchronous. */
 int32_t z2d_gpu_batch_render(z2d_gpu_batch *b, uint32_t mode);
 int32_t z2d_gpu_batch_wait(z2d_gpu_batch *b);
