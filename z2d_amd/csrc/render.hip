@@ -1654,13 +1654,17 @@ __device__ __forceinline__ double redge_x(double top, double x_start, double x_i
 // meets: top < b's last sample row + 0.5 and bot >= its first + 0.5 (the
 // active-edge test over the band; lo > hi: none).  Both hold over a range of
 // bands; floor estimates, wider by one, are corrected with the exact
-// comparisons.
+// comparisons.  No sample row meets an edge without height (a slot without an
+// edge, a caller's horizontal edge) or with a NaN end: no band has it,
+// whatever [rb_lo, rb_hi] is, so that k_edge_build, which counts, and
+// k_edge_bins, which places, agree on every edge.
 __device__ __forceinline__ void edge_bands(double top, double bot, int32_t rows, int32_t rb_lo,
                                            int32_t rb_hi, int32_t &lo, int32_t &hi) {
-  const double flo = fmax(floor(top / (double)rows) - 1.0, (double)rb_lo);
-  const double fhi = fmin(floor(bot / (double)rows) + 1.0, (double)rb_hi);
   lo = INT32_MAX;
   hi = INT32_MIN;
+  if (!(top < bot)) return;
+  const double flo = fmax(floor(top / (double)rows) - 1.0, (double)rb_lo);
+  const double fhi = fmin(floor(bot / (double)rows) + 1.0, (double)rb_hi);
   if (!(flo <= fhi)) return;
   int32_t l = (int32_t)flo, h = (int32_t)fhi;
 #pragma unroll
@@ -1746,13 +1750,10 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
     const uint32_t k = k0 + lane;
     const bool slot = k < end;
     z2d_edge ed{0.0, 0.0, 0.0, 0.0};
-    bool emit = false;
     if (serial) {
       if (slot) ed = out[k];
-      emit = slot;
     } else if (input) {
       if (slot) ed = J.in_edges[D.in_edge_off + k];
-      emit = slot;
     } else {
       const FNode *nodes = J.nodes + D.node_off;
       FNode nd{0.0, 0.0, 0xFFFFFFFFu, 0u}, pv{0.0, 0.0, 0xFFFFFFFFu, 0u};
@@ -1763,9 +1764,10 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
       // (a line or close before the first move is rejected on the host)
       const bool moves = !pt_eq(px, py, nd.x, nd.y);
       const double ax = px * scale, ay = py * scale, bx = nd.x * scale, by = nd.y * scale;
-      emit = slot && k > 0 && moves && (ay < by || ay > by) &&
-             (nd.tag == Z2D_NODE_LINE_TO ||
-              (nd.tag == Z2D_NODE_CLOSE_PATH && nd.closes && ptag != Z2D_NODE_CLOSE_PATH));
+      const bool emit =
+          slot && k > 0 && moves && (ay < by || ay > by) &&
+          (nd.tag == Z2D_NODE_LINE_TO ||
+           (nd.tag == Z2D_NODE_CLOSE_PATH && nd.closes && ptag != Z2D_NODE_CLOSE_PATH));
       double top = 0.0, bot = 0.0, left = 0.0, right = 0.0;
       if (emit) {  // Polygon.addEdge (src/internal/tess/Polygon.zig:61-109)
         ed.y0 = ay;
@@ -1800,7 +1802,7 @@ __global__ void __launch_bounds__(256) k_edge_build(JobView J) {
     // the edges counted per band of the draw's entries
     const double top = ed.y0 < ed.y1 ? ed.y0 : ed.y1, bot = ed.y0 < ed.y1 ? ed.y1 : ed.y0;
     int32_t lo = INT32_MAX, hi = INT32_MIN;
-    if (emit) edge_bands(top, bot, band_rows, (int32_t)D.band_lo, (int32_t)D.band_hi, lo, hi);
+    edge_bands(top, bot, band_rows, (int32_t)D.band_lo, (int32_t)D.band_hi, lo, hi);
     const int32_t ulo = wave_min_i32(lo), uhi = wave_max_i32(hi);
     const uint64_t em = __ballot(lo <= hi);
     const bool transposed = by_edge(em, ulo, uhi);
@@ -1896,8 +1898,7 @@ __global__ void __launch_bounds__(256) k_edge_bins(JobView J) {
       xlo = INT32_MIN;
       xhi = INT32_MAX;
     }
-    if (ed.y0 != ed.y1)  // (a slot without an edge)
-      edge_bands(top, bot, band_rows, max(rows.x / bh, blo), min((rows.y - 1) / bh, bhi), lo, hi);
+    edge_bands(top, bot, band_rows, max(rows.x / bh, blo), min((rows.y - 1) / bh, bhi), lo, hi);
   }
   const REdge red = make_redge(ed);  // the copy every band of the edge receives
   const int32_t ulo = wave_min_i32(lo), uhi = wave_max_i32(hi);
