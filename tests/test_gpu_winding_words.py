@@ -2,7 +2,10 @@
 changes: closed paths that go round 1 to 300 times in either direction (a
 byte holds windings to 127, 254 edges are the most that cannot exceed it),
 slanted so that the loops cross several strips and lie left of others, both
-fill rules, equal to the oracle."""
+fill rules, and the same between hundreds of short edges, where a strip's
+edges are many but a sample row's crossings few; equal to the oracle."""
+import math
+
 import numpy as np
 import pytest
 
@@ -37,5 +40,27 @@ def test_loops(n, rule):
                       abi.fill_opts(abi.AA_DEFAULT, rule, "src_over")))
     want = run_draws(OracleBackend(), abi.RGBA, w, h, init.reshape(-1), draws)
     got = run_draws(gpu_backend(), abi.RGBA, w, h, init.reshape(-1), draws)
+    msg = diff_report(got.data(), want.data())
+    assert not msg, msg
+
+
+@pytest.mark.parametrize("n", [0, 1, 30, 62, 63, 64, 65, 100])
+def test_loops_among_short_edges(n):
+    """2n crossings of a sample row by the loops, and those of two wavy
+    columns of 500 short edges each (a stroke's outline looks like that)."""
+    w, h = 230, 21
+    init = np.full(w * h * 4, 255, np.uint8)
+    draws = []
+    for sign, twist, x0 in ((1, 0.0, 20.0), (-1, 0.03, 100.0), (1, -0.02, 215.0)):
+        loops = _loops(max(1, n), sign, w, h, twist)[:-1] if n else np.zeros(0, abi.NODE_DTYPE)
+        m = 500
+        side = [(x0 + 3.0 * math.sin(0.7 * i), 1.0 + (h - 2.0) * i / m) for i in range(m + 1)]
+        pts = side + [(x + 6.0, y) for x, y in side[::-1]]
+        wavy = abi.nodes_array([(abi.MOVE_TO, *pts[0])] + [(abi.LINE_TO, *p) for p in pts[1:]] +
+                               [(abi.CLOSE_PATH,), (abi.MOVE_TO, *pts[0])])
+        draws.append((abi.solid_pattern(abi.rgba(40, 90, 20, 120)), np.concatenate([loops, wavy]),
+                      abi.fill_opts(abi.AA_DEFAULT, abi.NON_ZERO, "src_over")))
+    want = run_draws(OracleBackend(), abi.RGBA, w, h, init, draws)
+    got = run_draws(gpu_backend(), abi.RGBA, w, h, init, draws)
     msg = diff_report(got.data(), want.data())
     assert not msg, msg

@@ -2745,16 +2745,15 @@ struct FastShared {
 // `left` for even-odd, per lane, to be combined over the wave; two entries of
 // a row difference array for non-zero); the other edges' (edge, sample row)
 // items are compacted by a wave scan and spread over the lanes.
-// inner: nonzero in some lane if a crossing lies past column 0; n_cross: the
-// edges with items.
+// inner: nonzero in some lane if a crossing lies past column 0.  count
+// (WIND_NZ): the difference array's high halves get the rows' items.
 template <int MODE, int SR>
 __device__ __forceinline__ void fast_edges(const REdge *edges, uint32_t ne, FastShared &sh,
                                            uint32_t lane, int32_t ys0, int32_t xs_base,
-                                           uint32_t &inner, uint32_t &left, uint32_t &n_cross) {
+                                           bool count, uint32_t &inner, uint32_t &left) {
   constexpr int32_t COLS = TILE_W * 4;
   inner = 0;
   left = 0;
-  n_cross = 0;
   for (uint32_t c0 = 0; c0 < ne; c0 += 64) {
     const uint32_t k = c0 + lane;
     int32_t n_sr = 0, lo = 0;
@@ -2788,7 +2787,10 @@ __device__ __forceinline__ void fast_edges(const REdge *edges, uint32_t ne, Fast
     const int32_t incl = wave_incl_scan(n_sr);
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
     if (total == 0) continue;  // uniform
-    if (MODE == WIND_NZ) n_cross += (uint32_t)__popcll(__ballot(n_sr > 0));
+    if (MODE == WIND_NZ && count && n_sr > 0) {
+      atomicAdd(&sh.ldiff[lo], 1 << 16);
+      atomicAdd(&sh.ldiff[lo + n_sr], -(1 << 16));
+    }
     const uint32_t my_off = (uint32_t)(incl - n_sr);
     // an owner's first item, first row and direction
     const uint32_t info = ((ed.yhi2 & 1) ? 0x80000000u : 0u) | ((uint32_t)lo << 16) | my_off;
@@ -2830,8 +2832,9 @@ __device__ __forceinline__ void fast_edges(const REdge *edges, uint32_t ne, Fast
   }
 }
 
-// The non-zero rule's left edges: each sample row's winding from the
-// difference array (cleared), in lane `row`, 0 in the others.
+// The non-zero rule's left edges: each sample row's winding (and the row's
+// items, where they were counted, in the high half) from the difference array
+// (cleared), in lane `row`, 0 in the others.
 __device__ __forceinline__ int32_t left_windings(FastShared &sh, uint32_t lane) {
   wave_lds_sync();
   int32_t dl = 0;
@@ -2850,10 +2853,10 @@ __device__ __forceinline__ void coverage_halves(const REdge *edges, uint32_t ne,
                                              int *kk) {
 #pragma unroll 1
   for (int h = 0; h < 2; h++) {
-    uint32_t inner, left, n_cross;
+    uint32_t inner, left;
     fast_edges<WIND_NZ16, STRIP_SUBROWS / 2>(edges, ne, sh, lane,
-                                             ys_base + h * (STRIP_SUBROWS / 2), xs_base, inner,
-                                             left, n_cross);
+                                             ys_base + h * (STRIP_SUBROWS / 2), xs_base, false,
+                                             inner, left);
     const int32_t wl = left_windings(sh, lane);
     if (wl != 0 && lane < (uint32_t)STRIP_SUBROWS / 2)
       atomicAdd(&sh.acc[lane >> 1][0], (uint32_t)wl << (16u * (lane & 1u)));
@@ -3084,25 +3087,32 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
 
         // ---- phases A and B: covered samples per pixel
         int kk[ROWS_PER_THREAD];
-        uint32_t inner, left, n_cross;
+        uint32_t inner, left;
         if (eo) {
-          fast_edges<WIND_EO, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, inner, left,
-                                             n_cross);
+          fast_edges<WIND_EO, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, false, inner,
+                                             left);
           if (__ballot(left != 0))  // parity of the left edges over the wave
             left = (uint32_t)__builtin_amdgcn_readlane((int32_t)wave_xor_scan(left), 63);
           coverage_eo(sh.acc, lane, left, kk);
         } else {
-          fast_edges<WIND_NZ, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, inner, left,
-                                             n_cross);
-          int32_t wl = 0;
-          if (__ballot(left != 0)) {
-            wl = left_windings(sh, lane);
+          // |winding| <= half the edges (contours return to their start), and
+          // in a sample row <= that left of the strip plus the row's
+          // crossings in it.  (By the strip's edges instead of its rows'
+          // crossings the strips of a stroke's many short edges were taken
+          // three times: 47 served requests of 91 px, 223 us of this kernel,
+          // 186 now; 64 surfaces of 128 px one by one, 158 us each and 133.)
+          const bool many = ne > 254u;
+          fast_edges<WIND_NZ, STRIP_SUBROWS>(edges, ne, sh, lane, ys_base, xs_base, many, inner,
+                                             left);
+          int32_t most = 0;
+          if (many || __ballot(left != 0)) {
+            int32_t wl, cross;
+            unpack_pair((uint32_t)left_windings(sh, lane), wl, cross);
+            most = abs(wl) + cross;
             if (wl != 0) atomicAdd(&sh.acc[lane >> 2][0], (uint32_t)wl << (8u * (lane & 3u)));
           }
           wave_lds_sync();
-          // |winding| <= half the edges (contours return to their start), and
-          // <= that at the strip's left plus the edges crossing it
-          if (ne > 254u && n_cross + (uint32_t)wave_max_i32(abs(wl)) > 127u) {
+          if (many && wave_max_i32(most) > 127) {
 #pragma unroll
             for (int i = 0; i < FAST_ACC_ROWS; i++)
               *reinterpret_cast<uint4 *>(&sh.acc[i][lane * 4]) = make_uint4(0u, 0u, 0u, 0u);
