@@ -54,6 +54,15 @@ def test_gradient(gtype, n, w, h, dither):
         assert not msg, f"{fmt} {op}: {msg}"
 
 
+@pytest.mark.parametrize("gtype", [0, 1, 2])
+@pytest.mark.parametrize("w,h", [(1024, 320), (1025, 320), (5003, 67)])
+@pytest.mark.parametrize("dither", [None, 2])
+def test_lane_of_one_and_of_four_pixels(gtype, w, h, dither):
+    """327,680 pixels are the most that are painted by a lane each; beyond,
+    a lane's four, and a row of more than 16 workgroups' in several steps."""
+    test_gradient(gtype, 6, w, h, dither)
+
+
 @pytest.mark.parametrize("dither", [0, 1, 2])
 def test_color_dither(dither):
     rng = SplitMix64(0xC01 + dither)

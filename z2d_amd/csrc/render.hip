@@ -3529,8 +3529,8 @@ __global__ void __launch_bounds__(256) k_composite_quad(QuadJob J) {
 }
 
 // ---------------------------------------------------------------------------
-// k_composite_paint: a whole surface painted with a gradient or a dither, four
-// pixels of a row per lane, per pixel what comp_pixel computes for the same
+// k_composite_paint: a whole surface painted with a gradient or a dither, PX
+// (four or one) pixels of a row per lane, per pixel what comp_pixel computes for the same
 // batch.  Bound by VALU work (the f64 offset, the stop search, the divisions):
 // the gradient's constants and stops are in LDS once per workgroup, the
 // source kind is a template parameter, and the dither thresholds, which
@@ -3540,7 +3540,7 @@ __global__ void __launch_bounds__(256) k_composite_quad(QuadJob J) {
 // ---------------------------------------------------------------------------
 constexpr uint32_t PAINT_COLOR = 3;  // KIND: a gradient type, or a color's dither
 
-template <uint32_t KIND, bool DITHER>
+template <uint32_t KIND, bool DITHER, uint32_t PX>
 __global__ void __launch_bounds__(256) k_composite_paint(PaintJob J) {
   __shared__ FastDraw B;
   const DevPaint &P = *J.paint;
@@ -3555,14 +3555,14 @@ __global__ void __launch_bounds__(256) k_composite_paint(PaintJob J) {
   const uint32_t d_type = DITHER ? load_uniform(&P.dither_type) : 0u;
   const F4 color = load_uniform(&P.dither_color);
   const float sc = DITHER ? 1.0f / (float)((1 << load_uniform(&P.dither_scale)) - 1) : 0.0f;
-  const int32_t x0 = (int32_t)((blockIdx.x * 64u + threadIdx.x) * 4u);
-  const int32_t step = (int32_t)(gridDim.x * 256u);  // a multiple of 64
+  const int32_t x0 = (int32_t)((blockIdx.x * 64u + threadIdx.x) * PX);
+  const int32_t step = (int32_t)(gridDim.x * 64u * PX);  // a multiple of 64
   for (int32_t y = (int32_t)(blockIdx.y * blockDim.y + threadIdx.y); y < J.h;
        y += (int32_t)(gridDim.y * blockDim.y)) {
     float th[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // the columns' thresholds, scaled
     if (DITHER && d_type != Z2D_DITHER_NONE) {
 #pragma unroll
-      for (int l = 0; l < 4; l++) {
+      for (int l = 0; l < (int)PX; l++) {
         const int x = x0 + l;
         const float m = d_type == Z2D_DITHER_BAYER
                             ? bayer8(x, y)
@@ -3572,13 +3572,13 @@ __global__ void __launch_bounds__(256) k_composite_paint(PaintJob J) {
       }
     }
     for (int32_t x = x0; x < J.w; x += step) {
-      const uint32_t n = (uint32_t)min(4, J.w - x);
+      const uint32_t n = (uint32_t)min((int32_t)PX, J.w - x);
       const uint64_t at = (uint64_t)y * (uint32_t)J.w + (uint32_t)x;
       Quad32 dst{};
       if (J.op != Z2D_OP_SRC) dst = quad_words<false>(J.dst + at, n);
       Quad32 res;
 #pragma unroll 1
-      for (uint32_t l = 0; l < 4; l++) {
+      for (uint32_t l = 0; l < PX; l++) {
         I4 s;
         F4 c = color;
         if constexpr (KIND != PAINT_COLOR) {
@@ -3889,21 +3889,40 @@ hipError_t z2d_launch_composite_quad(const QuadJob &job, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Up to this many pixels a lane paints one: such a surface leaves most of the
+// chip idle, and a lane's four pixels are one chain after the other.  A call
+// on 640x480 (linear to conic, dithered or not) takes 25.3 to 28.3 us with one
+// and 26.2 to 34.3 with four, on 150x150 24.7 to 26.5 and 25.9 to 33.5 (the
+// general kernel, which gives every pixel a lane where the width is no
+// multiple of four: 26.8 to 28.8); on 701x601 linear takes 27.2 and 26.4,
+// conic 29.8 and 31.6, on 1024x768 radial 31.0 and 27.8.
+constexpr uint64_t PAINT_SINGLE = 5u << 16;
+
+template <uint32_t KIND, bool DITHER>
+static void launch_paint(const PaintJob &J, hipStream_t st) {
+  const bool single = (uint64_t)J.w * (uint32_t)J.h <= PAINT_SINGLE;
+  const uint32_t cols = single ? 64u : 256u;  // of a workgroup
+  const dim3 block(64, 4);
+  const uint32_t bx = ((uint32_t)J.w + cols - 1) / cols, by = (uint32_t)((J.h + 3) / 4);
+  // some 4,096 workgroups: enough for eight waves a SIMD twice over
+  const dim3 grid(min(bx, 16u), min(by, 4096u / min(bx, 16u)));
+  if (single)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<KIND, DITHER, 1>), grid, block, 0, st, J);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<KIND, DITHER, 4>), grid, block, 0, st, J);
+}
+
 // kind: a gradient type or PAINT_COLOR.
 hipError_t z2d_launch_composite_paint(const PaintJob &J, uint32_t kind, bool dither,
                                       hipStream_t st) {
-  const dim3 block(64, 4);
-  const uint32_t bx = (uint32_t)((J.w + 255) / 256), by = (uint32_t)((J.h + 3) / 4);
-  // some 4,096 workgroups: enough for eight waves a SIMD twice over
-  const dim3 grid(min(bx, 16u), min(by, 4096u / min(bx, 16u)));
   switch (kind * 2 + (dither ? 1 : 0)) {
-    case 0: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<0, false>), grid, block, 0, st, J); break;
-    case 1: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<0, true>), grid, block, 0, st, J); break;
-    case 2: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<1, false>), grid, block, 0, st, J); break;
-    case 3: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<1, true>), grid, block, 0, st, J); break;
-    case 4: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<2, false>), grid, block, 0, st, J); break;
-    case 5: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<2, true>), grid, block, 0, st, J); break;
-    default: hipLaunchKernelGGL(HIP_KERNEL_NAME(k_composite_paint<PAINT_COLOR, true>), grid, block, 0, st, J);
+    case 0: launch_paint<0, false>(J, st); break;
+    case 1: launch_paint<0, true>(J, st); break;
+    case 2: launch_paint<1, false>(J, st); break;
+    case 3: launch_paint<1, true>(J, st); break;
+    case 4: launch_paint<2, false>(J, st); break;
+    case 5: launch_paint<2, true>(J, st); break;
+    default: launch_paint<PAINT_COLOR, true>(J, st);
   }
   return hipGetLastError();
 }
