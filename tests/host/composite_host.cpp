@@ -107,7 +107,8 @@ static uint64_t check_rewrites(uint64_t &cases) {
     const I4 m = mask_coverage(unpack8(sw), k);
     if (mask_coverage_rgba8(sw, k) != (m.r | (m.g << 8) | (m.b << 16) | (m.a << 24))) bad++;
   }
-  // f2u8 (truncf of v + (0.5 - 2^-25), clamped) against roundf
+  // f2u8 (the device's form, its conversion instruction stated in C by
+  // cvt_u32_sat: truncation of v + (0.5 - 2^-25), clamped) against roundf
   // with the branches it replaces: every 61st float bit pattern and the
   // neighbourhoods of the halves 0.5 .. 65535.5
   auto f2u8_ref = [](float v) -> uint32_t {
@@ -133,6 +134,44 @@ static uint64_t check_rewrites(uint64_t &cases) {
       }
       v = std::nextafterf(v, t == 0 ? 0.0f : 1e9f);
       if (t == 1) v = std::nextafterf(v, 1e9f);
+    }
+  }
+  // div255f against the division, every value below 65536
+  auto same = [](float a, float b) { return a == b || (a != a && b != b); };  // (zeros: any sign)
+  for (uint32_t v = 0; v < 65536; v++) {
+    cases++;
+    if (!same(div255f(v), (float)v / 255.0f)) bad++;
+  }
+  // div_by against the division: every pair of 8-bit lanes (a zero divisor
+  // among them), then operands as the float operators form them (products and
+  // differences of lanes and of floats in [0, 1], down to neighbouring
+  // floats), then any two normal floats whose quotient is normal too
+  for (uint32_t i = 0; i < 256; i++)
+    for (uint32_t j = 0; j < 256; j++) {
+      const float a = (float)i / 255.0f, b = (float)j / 255.0f;
+      cases++;
+      if (!same(div_by(a, divisor(b)), a / b)) bad++;
+    }
+  for (int i = 0; i < (1 << 21); i++) {
+    float v[4];
+    for (float &f : v)
+      f = rnd(2) ? (float)rnd(256) / 255.0f : (float)(next_u64() >> 40) * 0x1p-24f;
+    if (rnd(4) == 0) v[1] = std::nextafterf(v[0], 2.0f);
+    const float as[3] = {v[2], v[2] * v[3], (v[2] - v[3]) * v[0]}, bs[2] = {v[0] - v[1], v[0]};
+    for (float a : as)
+      for (float b : bs) {
+        cases++;
+        if (!same(div_by(a, divisor(b)), a / b)) bad++;
+      }
+    const uint64_t r = next_u64();
+    const uint32_t wa = (uint32_t)r, wb = (uint32_t)(r >> 32);
+    float a, b;
+    std::memcpy(&a, &wa, 4);
+    std::memcpy(&b, &wb, 4);
+    if (std::fabs(a) >= 0x1p-60f && std::fabs(a) <= 0x1p60f && std::fabs(b) >= 0x1p-65f &&
+        std::fabs(b) <= 0x1p65f) {
+      cases++;
+      if (!same(div_by(a, divisor(b)), a / b)) bad++;
     }
   }
   // round_i32 (truncation of v + copysign(0.5 - 2^-54, v)) against

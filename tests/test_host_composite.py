@@ -8,8 +8,11 @@ coverage 0..16 (multisample) and 0..1 (direct).  The same harness checks the
 device code's arithmetic rewrites against the forms they replace: src_over
 and the coverage mask on RGBA8 words two channels at a time (every channel
 triple, then random words), the branchless float-to-lane conversion
-(every 61st float and the neighbourhoods of the halves), overlay and hard
-light on 8-bit lanes (random lanes against the signed per-channel forms).
+(every 61st float and the neighbourhoods of the halves; the conversion
+instruction itself is stated in C here), the divisions by a shared reciprocal
+(every pair of 8-bit lanes, random operands) and by 255 (every value), overlay
+and hard light on 8-bit lanes (random lanes against the signed per-channel
+forms).
 Runs on the CPU."""
 import os
 import shutil

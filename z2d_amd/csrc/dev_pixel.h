@@ -102,6 +102,19 @@ Z2D_PX __forceinline__ double zmodd(double x, double y) {
   double a = fmod(x, y);
   return x < 0.0 ? fmod(a + y, y) : a;
 }
+// v_cvt_u32_f32: truncates, takes NaN and everything below zero to 0 and
+// saturates above (written out because a C conversion of such values is
+// undefined); the host states the same.
+Z2D_PX __forceinline__ uint32_t cvt_u32_sat(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+#else
+  return !(v >= 1.0f) ? 0u : v >= 0x1p32f ? 0xFFFFFFFFu : (uint32_t)v;
+#endif
+}
+
 // round(255*v) to an 8-bit channel; saturates outside the range the
 // reference defines (its @intFromFloat is undefined there).
 // roundf(v) (half away from zero), then 0 below zero or for NaN and 65535
@@ -109,17 +122,11 @@ Z2D_PX __forceinline__ double zmodd(double x, double y) {
 // v >= 0 (checked over all 2^32 floats with the sign copied onto the
 // addend), and for v < 0 it is at most 0 as roundf(v) is, so the clamp
 // gives 0 either way; the clamp takes NaN to 0.
-// The device's conversion truncates, takes NaN and everything below zero to 0
-// and saturates above, so there one integer minimum is left of the clamp.
+// The conversion takes NaN and everything below zero to 0 and saturates above,
+// so one integer minimum is left of the clamp.
 Z2D_PX __forceinline__ uint32_t f2u8(float v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t r;
-  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v + 0x1.fffffep-2f));
-  return min(r, 65535u);
-#else
-  const float r = truncf(v + 0x1.fffffep-2f);
-  return (uint32_t)fminf(fmaxf(r, 0.0f), 65535.0f);
-#endif
+  const uint32_t r = cvt_u32_sat(v + 0x1.fffffep-2f);
+  return r < 65535u ? r : 65535u;
 }
 
 // (int32_t)round(v) (half away from zero) as one add and the truncating

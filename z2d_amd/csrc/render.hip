@@ -2928,13 +2928,8 @@ __device__ __forceinline__ float fast_conic_offset(const FastDraw &g, int x, int
   return (float)(ang / two_pi);
 }
 
-// f2u8 of a value below 65536 as one add and the hardware's conversion, which
-// truncates and takes everything below zero, and NaN, to 0.
-__device__ __forceinline__ uint32_t f2u8_sat(float v) {
-  uint32_t r;
-  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v + 0x1.fffffep-2f));
-  return r;
-}
+// f2u8 of a value below 65536.
+__device__ __forceinline__ uint32_t f2u8_sat(float v) { return cvt_u32_sat(v + 0x1.fffffep-2f); }
 
 // Paint samples of the covered pixels listed in plist (as dense_gradient).
 template <uint32_t PF>
