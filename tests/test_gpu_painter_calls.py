@@ -3,14 +3,15 @@ the call before: small after large and large after small, strokes and
 polygons between fills, calls that fail between calls that succeed, a call
 whose buffers are too large to keep, and calls from two threads at once; each
 equal to the oracle's."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
-from z2d_amd import abi, scenes
+from z2d_amd import abi, gpu, scenes
 from gpu_util import diff_report, gpu_backend
-from oracle_backend import OracleBackend
+from oracle_backend import OracleBackend, lib as oracle_lib
 from stroke_check import StrokeCheckBackend
 from zscene import Surface
 
@@ -35,6 +36,14 @@ def _run(calls, backend, check):
         for kind, pat, nodes, opts in jobs:
             assert getattr(backend, kind)(got, pat, nodes, opts) == 0
             assert getattr(check, kind)(want, pat, nodes, opts) == 0
+            if kind == "stroke":  # and its outline as a polygon
+                rc, edges, ext, aa = gpu.stroke_polygon(nodes, opts, abi.RGBA)
+                args = (C.byref(pat), edges.ctypes.data, len(edges), (C.c_double * 4)(*ext), aa,
+                        abi.EVEN_ODD, opts.op, opts.precision)
+                dg, dw = got.desc(), want.desc()
+                assert rc == 0
+                assert gpu.lib().z2d_gpu_fill_polygon(backend.ctx.h, C.byref(dg), *args) == 0
+                assert oracle_lib().zo_fill_polygon(C.byref(dw), *args) == 0
             bad = nodes.copy()
             bad["tag"][0] = abi.LINE_TO  # a line before any move
             assert backend.fill(got, pat, bad, abi.fill_opts()) != 0
@@ -49,9 +58,9 @@ def test_sequence():
 def test_large_call_between_small_ones():
     be, ob = gpu_backend(), OracleBackend()
     rng = scenes.SplitMix64(0x1A6)
-    # a polyline of 60,000 lines down a tall surface: (edge, band) copies
-    # beyond what a context keeps
-    n, w, h = 60000, 64, 8192
+    # a polyline of 20,000 lines down a tall surface: some 3.4 million (edge,
+    # band) copies of 32 bytes, beyond the 64 MiB that a context keeps
+    n, w, h = 20000, 64, 8192
     pts = [(rng.uniform(0, w), rng.uniform(0, h)) for _ in range(n)]
     big = abi.nodes_array([(abi.MOVE_TO, *pts[0])] + [(abi.LINE_TO, *p) for p in pts[1:]] +
                           [(abi.CLOSE_PATH,), (abi.MOVE_TO, *pts[0])])
@@ -62,10 +71,9 @@ def test_large_call_between_small_ones():
         got, want = Surface(abi.RGBA, sw, sh), Surface(abi.RGBA, sw, sh)
         opts = abi.fill_opts(abi.AA_DEFAULT, abi.EVEN_ODD, "src_over")
         assert be.fill(got, pat, nodes, opts) == 0
-        if sh < 4096:  # (the oracle's serial loop over 60,000 edges a row)
-            if nodes is not big:
-                assert ob.fill(want, pat, nodes, opts) == 0
-                assert not diff_report(got.data(), want.data())
+        assert ob.fill(want, pat, nodes, opts) == 0
+        msg = diff_report(got.data(), want.data())
+        assert not msg, f"{sw}x{sh}: {msg}"
 
 
 def test_two_threads():
