@@ -200,7 +200,6 @@ struct z2d_gpu_ctx {
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   DevBuf comp_arena;
   HostBuf comp_stage;
-  int n_cus = 256;
   float last_comp_ms = 0.0f;  // device time of the last composite kernel
   DevBuf png_work;            // scanline stream, segment staging, offsets
   DevBuf png_out;             // the encoded file
@@ -2105,9 +2104,6 @@ int32_t z2d_gpu_create(int32_t device, z2d_gpu_ctx **out) {
     delete ctx;
     return Z2D_ERR_DEVICE;
   }
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-    ctx->n_cus = prop.multiProcessorCount;
   ctx->comp_scratch = comp_scratch_for(device);  // device is current
   *out = ctx;
   return Z2D_OK;

@@ -197,9 +197,8 @@ enum : uint32_t {
 };
 struct alignas(16) FastDraw {
   int32_t rx0, rx1, ry0, ry1;  // composite region
-  uint32_t flags, rule, paint, px;  // DRAW_* flags, fill rule, FAST_PAINT_*, solid RGBA8
-  uint32_t n_stops, identity, pad0, pad1;
-  uint32_t pad2[4];
+  uint32_t rule, paint;        // fill rule, FAST_PAINT_*
+  uint32_t n_stops, identity;  // gradient: stops, whether the inverse matrix is the identity
   // gradient: geom[0..1], the inverse matrix, the type's constants
   // (linear: dx, dy, 1/|d|^2, degenerate; radial: r1, r2, cdx, cdy, dr,
   // min_dr, a, 1/a; conic: the start angle mod 2 pi)

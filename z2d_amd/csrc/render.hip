@@ -325,17 +325,15 @@ __device__ void write_fast_gradient(FastDraw &F, const DevGradient &G, uint32_t 
   }
 }
 
-// A fast draw's block: its region and flags, and the paint's constants
+// A fast draw's block: its region and rule, and the paint's constants
 // (the solid paint's table is written by the draw's lanes 0..16 before).
 __device__ void write_fast_draw(FastDraw &F, const DevDraw &D, const DevPaint &P, uint32_t pf) {
   F.rx0 = D.rx0;
   F.rx1 = D.rx1;
   F.ry0 = D.ry0;
   F.ry1 = D.ry1;
-  F.flags = D.flags;
   F.rule = D.rule;
   F.paint = pf;
-  F.px = P.px.r | (P.px.g << 8) | (P.px.b << 16) | (P.px.a << 24);
   F.n_stops = 0;
   F.identity = 1;
   if (pf >= FAST_PAINT_LINEAR && pf <= FAST_PAINT_CONIC) write_fast_gradient(F, *P.gradient, pf);
@@ -2967,11 +2965,6 @@ __device__ __forceinline__ void fast_gradient(const FastDraw &B, FastShared &sh,
   }
 }
 
-__device__ __forceinline__ uint32_t rfl(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int32_t rfl(int32_t v) {
-  return (int32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-}
-
 // Bound by VALU issue and, at few waves, by latency: six waves per SIMD (79
 // VGPRs and 5.9 KB of LDS) take 0.78 ms for the 4K scene of 10,000 paths, five
 // 0.81, four 0.89.  No register is spilled: what lives from entry to entry
@@ -3066,8 +3059,8 @@ k_render_fast(JobView J, uint32_t tile_base, uint32_t tile_count, uint32_t first
                       rx1 = __builtin_amdgcn_readlane(nb.y, 0),
                       ry0 = __builtin_amdgcn_readlane(nb.z, 0),
                       ry1 = __builtin_amdgcn_readlane(nb.w, 0);
-        const bool eo = __builtin_amdgcn_readlane(nb.y, 1) == Z2D_FILL_EVEN_ODD;
-        const uint32_t pf = __builtin_amdgcn_readlane(nb.z, 1);
+        const bool eo = __builtin_amdgcn_readlane(nb.x, 1) == Z2D_FILL_EVEN_ODD;
+        const uint32_t pf = __builtin_amdgcn_readlane(nb.y, 1);
         if (j + 1 < nc) {
           const uint32_t dn = __builtin_amdgcn_readlane(g_draw, j + 1);
           if (lane < FAST_DRAW_CHUNKS) nb = reinterpret_cast<const uint4 *>(J.fast + dn)[lane];
