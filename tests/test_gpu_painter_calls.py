@@ -4,6 +4,7 @@ polygons between fills, calls that fail between calls that succeed, a call
 whose buffers are too large to keep, and calls from two threads at once; each
 equal to the oracle's."""
 import ctypes as C
+import mmap
 import threading
 
 import numpy as np
@@ -74,6 +75,28 @@ def test_large_call_between_small_ones():
         assert ob.fill(want, pat, nodes, opts) == 0
         msg = diff_report(got.data(), want.data())
         assert not msg, f"{sw}x{sh}: {msg}"
+
+
+def _resident():
+    with open("/proc/self/statm") as f:
+        return int(f.read().split()[1]) * mmap.PAGESIZE
+
+
+def test_inputs_of_a_failed_call_are_not_kept():
+    """8.6 million edges down 512 bands are more (edge, band) pairs than a
+    batch can index, which is found before any buffer is made: the context
+    keeps none of the 275 MB either."""
+    be, s = gpu_backend(), Surface(abi.RGBA, 64, 8192)
+    edges = np.zeros(8600000, abi.EDGE_DTYPE)
+    edges["y1"] = 4.0 * 8192
+    d, pat = s.desc(), abi.solid_pattern(abi.rgba(1, 2, 3, 4))
+    ext = (C.c_double * 4)(0.0, 4.0 * 8192, 0.0, 256.0)
+    before = _resident()
+    assert gpu.lib().z2d_gpu_fill_polygon(be.ctx.h, C.byref(d), C.byref(pat), edges.ctypes.data,
+                                          len(edges), ext, abi.AA_DEFAULT, 0, abi.OP["src_over"],
+                                          0) == abi.ERR_OUT_OF_MEMORY
+    assert _resident() - before < 128 << 20
+    _run(_calls(0xF41, 2), be, StrokeCheckBackend())
 
 
 def test_two_threads():

@@ -2370,7 +2370,8 @@ void z2d_gpu_batch_destroy(z2d_gpu_batch *b) {
 // One painter call on a descriptor through a single-draw batch.  The context
 // keeps one: every call ends with the stream drained, so its buffers are free
 // again when it returns (a call that finds it in use by another thread makes
-// its own).  Buffers beyond kPainterKeep bytes are given back.
+// its own).  One that holds more than kPainterKeep bytes of buffers, or of its
+// call's inputs, is given back.
 constexpr size_t kPainterKeep = (size_t)64 << 20;
 
 static int32_t single_draw(z2d_gpu_ctx *ctx, z2d_surface_desc *surface,
@@ -2398,13 +2399,14 @@ static int32_t single_draw(z2d_gpu_ctx *ctx, z2d_surface_desc *surface,
       (void)hipStreamSynchronize(ctx->stream);  // uploads of a failed prepare
   }
   batch_clear(&b);
-  if (b.arena.cap + b.stage.cap + b.flat_buf.cap + b.flat_stage.cap > kPainterKeep) {
-    b.arena.release();
-    b.stage.release();
-    b.flat_buf.release();
-    b.flat_stage.release();
-    b.raw_nodes.shrink_to_fit();
-    b.in_edges.shrink_to_fit();
+  // (a call that fails before its buffers are made leaves its inputs alone)
+  const size_t inputs = b.raw_nodes.capacity() * sizeof(z2d_path_node) +
+                        b.in_edges.capacity() * sizeof(z2d_edge) +
+                        b.paints.stops.capacity() * sizeof(DevStop);
+  if (&b == ctx->painter && (inputs > kPainterKeep || b.arena.cap + b.stage.cap + b.flat_buf.cap +
+                                                              b.flat_stage.cap > kPainterKeep)) {
+    z2d_gpu_batch_destroy(ctx->painter);
+    ctx->painter = nullptr;
   }
   int32_t rc2 = surface_release(ctx, ref, rc == Z2D_OK);
   return rc ? rc : rc2;
