@@ -808,7 +808,7 @@ struct z2d_gpu_batch {
   float last_pipeline_ms = 0.0f, last_render_ms = 0.0f;
   uint32_t count_stats = 0;
   uint32_t band_h = TILE_H;  // rows per band (bin height), a multiple of ROWS_PER_THREAD
-  uint32_t longest_first = 0;  // strip queue order of the single-launch render
+  uint32_t longest_first = 0;  // strip order of the single-launch render
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   bool render_timed = false;  // the last render recorded ev[1] before the tile render
   bool timed = true;          // renders record their device time
@@ -1493,9 +1493,10 @@ static hipError_t batch_enqueue(z2d_gpu_batch *b, uint32_t mode, bool mark_rende
   const uint32_t ns = J.n_surfaces;
   const hipStream_t st = bstream(b);
   // every per-render reset: counters, what the draws' edges add up, the
-  // entries' edge counts and cursors, their column ranges (empty until the edge binning widens them) and the
-  // scans' look-back words; done by the flattening's per-node kernel when
-  // there is one, else in a launch of their own
+  // entries' edge counts and cursors, their column ranges (empty until the
+  // edge binning widens them) and the scans' look-back words; done by the
+  // flattening's per-node kernel when there is one, else in a launch of their
+  // own
   FillSet F{};
   auto add = [&](uint32_t *p, uint64_t n, uint32_t v) {
     if (n == 0) return;
@@ -2244,7 +2245,7 @@ int32_t z2d_gpu_batch_set_band_height(z2d_gpu_batch *b, uint32_t rows) {
 }
 
 // The autotuner: renders the batch once per candidate (band height 8, 16, 32
-// with the natural queue order, then each with the longest-first order; a
+// with the natural strip order, then each with the longest-first order; a
 // warm-up and `reps` timed pipelines each), keeps the fastest and prepares
 // the batch for it.  The surfaces are saved before and restored after every
 // candidate, so the batch's targets end as they started.

@@ -264,7 +264,7 @@ struct JobView {
   uint32_t max_entry_edges;
   uint32_t band_h;           // rows per band
   uint32_t strips_per_tile;  // band_h / ROWS_PER_THREAD
-  // longest-first queue order of the single-launch render (null: natural
+  // longest-first strip order of the single-launch render (null: natural
   // order): strips by decreasing list length, from a counting sort over
   // ORDER_BUCKETS lengths
   uint32_t *strip_order;     // n_tiles * strips_per_tile
